@@ -20,6 +20,15 @@
 //     built by scattering the stored values at their tile ids;
 //   * C: lane l holds rows 4*(l/16) + i, i < 4, of its MFMA column, i.e. the
 //     output columns tile + q*VEC + v for the v-th MFMA.
+// What bounds it: the row gathers (a kernel of the same loads and nothing
+// else takes 2.6 ms of the 3.1 on the 2^20-node R-MAT at N = 256, 0.21 of
+// 0.36 on the 2^18-node one at N = 128), then the float32 MFMAs, which do
+// 16-row work on columns of one or two entries (0.07 ms of those 0.36, 0.28
+// of 4.3 on the 232,965-row block model at N = 128).  So the loop is built to
+// leave one exposed latency per group, the gathers' own, few vector
+// instructions around them, and five waves per SIMD to overlap one wave's
+// MFMAs with the others' gathers (a second group in flight per wave at three
+// to four waves per SIMD measured 10-35% slower).
 // For FP32 the same group is fed as 8 steps of v_mfma_f32_16x16x4_f32 where
 // step j pairs A_g[:, j] with B row j of block g.  The k order inside a
 // group is a permutation shared by A and B, so every mapping sums the same
@@ -82,11 +91,12 @@ struct SpmmParams {
   int32_t nnz;         // entries of tile / vals
   int32_t n_ct;        // column tiles
   int32_t num_items;   // windows (unbalanced) or chunks (balanced)
-  int32_t chunk;       // balanced chunk length in TC blocks
+  int32_t chunk;       // balanced: chunk length in TC blocks; unbalanced: windows per unit
   int32_t *queue;      // persistent work counter
   const int2 *runs;    // balanced: run [b, e) of every chunk, cut flags in the sign bits
   float *parts;        // balanced, deterministic merge: partial-tile slots (NULL: atomics)
   int32_t span;        // balanced cut span in TC blocks (a multiple of chunk)
+  int32_t ct_blocks;   // workgroups per column tile when column tiles go one after another, 0: side by side
 };
 
 // Kernels take the arrays as restrict-qualified arguments: the compiler may
@@ -101,7 +111,7 @@ struct SpmmParams {
   SpmmParams {                                                                             \
     a_rwo, a_rowid, a_tile, a_off, a_atox, a_vals, a_B, a_C, a_p.num_windows,              \
         a_p.num_blocks, a_p.M, a_p.b_rows, a_p.N, a_p.nnz, a_p.n_ct, a_p.num_items,        \
-        a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span                                \
+        a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span, a_p.ct_blocks                                \
   }
 
 template <int VEC>
@@ -291,198 +301,275 @@ __device__ __forceinline__ void mfma_group(const float (&a)[8], const breg_t<PRE
   }
 }
 
-// Metadata of one K=32 group (up to 4 TC blocks of one window), loaded one
-// group ahead of its use so that its latency hides behind the previous
-// group's B gathers.  Loading does not need the group's length: the offsets
-// of all 4 candidate blocks are read and `resolve_meta` trims them once the
-// length is known.
-struct GroupMeta {
-  int bb;                  // first block (wave-uniform)
-  int f0, f1, f2, f3, f4;  // TCblock_offset[bb + k], raw
-  int o0, o1, o2, o3, o4;  // element offsets of the group's blocks (resolved)
-  int4 r0, r1;             // SparseAToX of block g (raw; masked where used)
-  int nblk;                // blocks in the group (resolved, wave-uniform)
-  int tile;                // tile id of element f0 + lane (raw)
-  float val;               // its value (raw)
-  int rid;                 // window of block bb + lane, -1 at or past the run's end
-  int fe;                  // without WALK: TCblock_offset[min(bb + 4, b1)], the group's end
+// Columns of this lane in every subtile: VEC consecutive ones from c[s].  The
+// last tile's lanes past N - VEC are moved back so that every vector lies
+// inside a row of B and C: they recompute (and store again, bit for bit) the
+// columns of their neighbours, no load or store needs a mask, and N need not
+// be a multiple of VEC (only N >= VEC).
+template <int NSUB>
+struct Cols {
+  int c[NSUB];
+};
+template <int VEC, int NSUB>
+__device__ __forceinline__ Cols<NSUB> lane_cols(int ct, int N) {
+  Cols<NSUB> o;
+#pragma unroll
+  for (int s = 0; s < NSUB; ++s)
+    o.c[s] = min(ct * (16 * VEC * NSUB) + s * 16 * VEC + (lane_id() & 15) * VEC, N - VEC);
+  return o;
+}
+
+// The arrays a wave reads, as buffer resources (WIDE = false): 32-bit byte
+// offsets, one vector instruction per address, and loads past an array's
+// end return zero, so the loop carries no 64-bit address arithmetic and no
+// masks.  The host takes this form when every array is below 2 GiB and B
+// has fewer than 2^24 rows of fewer than 2^24 bytes (fits_buffers); larger
+// operands take 64-bit pointers (WIDE = true).
+template <bool WIDE>
+struct Bufs {};
+template <>
+struct Bufs<false> {
+  __amdgpu_buffer_rsrc_t tile, vals, atox, b;
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_buf(const void *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
+}
+template <int PREC, bool WIDE, bool DENSE>
+__device__ __forceinline__ Bufs<WIDE> make_bufs(const SpmmParams &p) {
+  Bufs<WIDE> o;
+  if constexpr (!WIDE) {
+    constexpr uint32_t esz = is_bf16b<PREC>() ? 2 : 4;
+    // whole 4-element vectors (kDense; the host checks their alignment, so the
+    // last one lies in the same 16 bytes as an element of the array)
+    const uint32_t n4 = ((uint32_t)p.nnz + 3u) & ~3u;
+    o.tile = make_buf(p.tile, DENSE ? n4 : (uint32_t)p.nnz);
+    o.vals = make_buf(p.vals, p.vals ? (DENSE ? n4 : (uint32_t)p.nnz) * 4u : 0u);
+    o.atox = make_buf(p.atox, (uint32_t)p.num_blocks * (kBlkW * 4u));
+    o.b = make_buf(p.B, (uint32_t)p.b_rows * ((uint32_t)p.N * esz));
+  }
+  return o;
+}
+
+// Block data of 64 consecutive blocks from sb, lane l holding block sb + l.
+// Groups starting in the first kStageBlocks of them find their (up to 4)
+// blocks and the following block's offset inside the stage.
+constexpr int kStageBlocks = 56;
+struct Stage {
+  int sb;
+  int off;  // TCblock_offset, clamped to the stored elements
+  int wid;  // balanced schedule: window id, -1 at or past the run's end
 };
 
-// Loads are unconditional and their results are only consumed one group
-// later, so nothing in the current group waits on them.  With WALK the
-// lane also reads the window id of block bb + lane: the 64-block look-ahead
-// from which the group's length (it stops at the next window start) is
-// found without another round trip.
-template <bool WALK>
-__device__ __forceinline__ void load_meta(const SpmmParams &p, int bb, int b1, bool has_vals,
-                                          GroupMeta &m) {
-  const int lane = lane_id();
-  const int g = lane >> 4;
-  const int T = p.num_blocks;
-  m.bb = bb;
-  m.f0 = p.off[bb];
-  m.f1 = p.off[min(bb + 1, T)];
-  m.f2 = p.off[min(bb + 2, T)];
-  m.f3 = p.off[min(bb + 3, T)];
-  m.f4 = p.off[min(bb + 4, T)];
-  const int blk = min(bb + g, b1 - 1);
-  const int4 *ap = reinterpret_cast<const int4 *>(p.atox + (int64_t)blk * kBlkW);
-  m.r0 = ap[0];
-  m.r1 = ap[1];
-  // The first 64 stored elements of the group, one per lane (a group holds
-  // 36 on average for R-MAT; more than 64 take the slow path in build_a).
-  const int e0 = min(max(m.f0, 0), p.nnz);
-  const int ec = e0 < p.nnz - lane ? e0 + lane : p.nnz - 1;
-  m.tile = p.tile[ec];
-  m.val = has_vals ? p.vals[ec] : 1.0f;
-  if constexpr (WALK) {
-    const int rb = bb + lane;
-    m.rid = rb < b1 ? p.rowid[rb] : -1;
+template <bool BALANCED>
+__device__ __forceinline__ Stage load_stage(const SpmmParams &p, int sb, int e) {
+  Stage s;
+  s.sb = sb;
+  const int i = sb + lane_id();
+  s.off = p.off[min(i, p.num_blocks)];
+  s.wid = BALANCED && i < e ? p.rowid[i] : -1;
+  return s;
+}
+
+// How the blocks are shared out (walk_blocks).
+constexpr int kWindows = 0, kBalanced = 1, kSplit = 2;
+
+// How a kernel reads its operands.
+constexpr int kPtr = 0;    // 64-bit pointers (operands of any size)
+constexpr int kBuf = 1;    // buffers, one element per lane
+constexpr int kDense = 2;  // buffers, four consecutive elements per lane
+
+// One K = 32 group: its wave-uniform position, and the per-lane metadata
+// loaded one group ahead of its use.
+struct Group {
+  int bb;          // first block
+  int nblk;        // blocks (1 .. 4)
+  int w;           // window
+  int o0, o1, o2, o3, o4;  // element offsets of its blocks; o4: its end
+  int4 r0, r1;     // SparseAToX of block bb + lane / 16
+  // Tile ids and values of the group's first elements.  Plain: elements
+  // o0 + lane and o0 + 64 + lane (the second 64 are loaded only for groups
+  // that have them).  Dense: elements (o0 & ~3) + 4 lane + k in byte k of
+  // tile and in v<k>.
+  int tile, tile2;
+  float v0, v1, v2, v3;
+};
+
+// Loads of a group's metadata.  They are issued before the previous group's
+// gathers and used after them, so their latency is never on the wave's path.
+template <int MODE>
+__device__ __forceinline__ void load_rows(const SpmmParams &p, const Bufs<MODE == kPtr> &bufs, Group &m) {
+  const int blk = m.bb + (lane_id() >> 4);
+  if constexpr (MODE == kPtr) {
+    const int4 *ap = reinterpret_cast<const int4 *>(p.atox + (int64_t)min(blk, p.num_blocks - 1) * kBlkW);
+    m.r0 = ap[0];
+    m.r1 = ap[1];
   } else {
-    m.fe = p.off[min(bb + kGroup, b1)];
+    const uint32_t ao = (uint32_t)blk * (kBlkW * 4u);
+    m.r0 = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(bufs.atox, ao, 0, 0));
+    m.r1 = __builtin_bit_cast(int4, __builtin_amdgcn_raw_buffer_load_b128(bufs.atox, ao + 16, 0, 0));
   }
 }
 
-// Group length and element offsets.  WALK: the group ends before the first
-// block of the look-ahead whose window differs from its predecessor's (or
-// at the run's end, where the look-ahead holds -1); else at b1.
-template <bool WALK>
-__device__ __forceinline__ void resolve_meta(const SpmmParams &p, int b1, GroupMeta &m) {
-  if constexpr (!WALK) {
-    // The group's end offset was loaded with the rest (its length is known
-    // up front); offsets past it are clamped to it, which for non-decreasing
-    // offsets is the end itself -- no index into the offsets by a run-time
-    // count, which the compiler would place in scratch memory.
-    m.nblk = min(kGroup, b1 - m.bb);
-    const int o4 = min(m.fe, p.nnz);
-    m.o0 = min(m.f0, o4);
-    m.o1 = min(m.f1, o4);
-    m.o2 = min(m.f2, o4);
-    m.o3 = min(m.f3, o4);
-    m.o4 = o4;
-    return;
+template <int MODE>
+__device__ __forceinline__ void load_elems(const SpmmParams &p, const Bufs<MODE == kPtr> &bufs, bool has_vals,
+                                           Group &m) {
+  const int lane = lane_id();
+  m.v0 = m.v1 = 1.0f;
+  if constexpr (MODE == kDense) {
+    m.v2 = m.v3 = 1.0f;
+    const uint32_t e = (uint32_t)(m.o0 & ~3) + 4u * (uint32_t)lane;
+    m.tile = (int)__builtin_amdgcn_raw_buffer_load_b32(bufs.tile, e, 0, 0);
+    if (has_vals) {
+      const floatx4 v = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(bufs.vals, e * 4, 0, 0));
+      m.v0 = v[0];
+      m.v1 = v[1];
+      m.v2 = v[2];
+      m.v3 = v[3];
+    }
+  } else if constexpr (MODE == kBuf) {
+    const uint32_t e = (uint32_t)(m.o0 + lane);
+    m.tile = __builtin_amdgcn_raw_buffer_load_b8(bufs.tile, e, 0, 0);
+    if (has_vals) m.v0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(bufs.vals, e * 4, 0, 0));
+    if (m.o4 - m.o0 > kWave) {
+      m.tile2 = __builtin_amdgcn_raw_buffer_load_b8(bufs.tile, e + kWave, 0, 0);
+      if (has_vals)
+        m.v1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(bufs.vals, (e + kWave) * 4, 0, 0));
+    }
+  } else {
+    const int last = p.nnz - 1;
+    const int e = m.o0 < p.nnz - lane ? m.o0 + lane : last;
+    m.tile = p.tile[e];
+    if (has_vals) m.v0 = p.vals[e];
+    if (m.o4 - m.o0 > kWave) {
+      const int e2 = e < p.nnz - kWave ? e + kWave : last;
+      m.tile2 = p.tile[e2];
+      if (has_vals) m.v1 = p.vals[e2];
+    }
   }
-  const int prev = __shfl_up(m.rid, 1, 64);
-  const uint64_t starts = __ballot(lane_id() > 0 && m.rid != prev);
-  const int nblk = starts ? min(kGroup, (int)__builtin_ctzll(starts)) : kGroup;
-  // selects, not an indexed array (which would live in scratch memory)
-  auto f = [&m](int k) {
-    return k == 0 ? m.f0 : k == 1 ? m.f1 : k == 2 ? m.f2 : k == 3 ? m.f3 : m.f4;
-  };
-  const int o4 = min(f(nblk), p.nnz);
-  m.o0 = min(m.f0, o4);
-  m.o1 = min(f(min(1, nblk)), o4);
-  m.o2 = min(f(min(2, nblk)), o4);
-  m.o3 = min(f(min(3, nblk)), o4);
-  m.o4 = o4;
-  m.nblk = nblk;
 }
 
-// This lane's 8 B rows (-1 for lanes whose block lies past the run).
-__device__ __forceinline__ void meta_rows(const GroupMeta &m, int (&rows)[8]) {
-  const bool gv = (lane_id() >> 4) < m.nblk;
-  rows[0] = gv ? m.r0.x : -1;
-  rows[1] = gv ? m.r0.y : -1;
-  rows[2] = gv ? m.r0.z : -1;
-  rows[3] = gv ? m.r0.w : -1;
-  rows[4] = gv ? m.r1.x : -1;
-  rows[5] = gv ? m.r1.y : -1;
-  rows[6] = gv ? m.r1.z : -1;
-  rows[7] = gv ? m.r1.w : -1;
-}
+template <int PREC, int VEC>
+struct BElem {
+  typedef typename std::conditional<is_bf16b<PREC>(), __bf16, float>::type type;
+  // a row's vector: aligned to its element only (any N)
+  typedef breg_t<PREC, VEC> type_u __attribute__((aligned(is_bf16b<PREC>() ? 8 : 4)));
+};
 
-// B rows of the group into registers: loads from clamped addresses, then
-// zero for slots without a row or columns past N (no branches around loads).
+// This lane's 8 rows of B through 64-bit pointers: loads from clamped
+// addresses, zero where the row is not one of B's (or ok is false).
 template <int PREC, int VEC, int NSUB>
-__device__ __forceinline__ void gather_b(const SpmmParams &p, const int (&rows)[8], int colbase,
-                                         breg_t<PREC, VEC> (&breg)[NSUB][8]) {
+__device__ __forceinline__ void gather_ptr(const SpmmParams &p, const int (&rows)[8], bool ok,
+                                           const Cols<NSUB> &cols,
+                                           breg_t<PREC, VEC> (&breg)[NSUB][8]) {
   typedef breg_t<PREC, VEC> vt;
-  typedef typename std::conditional<is_bf16b<PREC>(), __bf16, float>::type et;
+  typedef typename BElem<PREC, VEC>::type et;
   const et *B = static_cast<const et *>(p.B);
-  const int64_t N = p.N;
   vt zero;
-  if constexpr (VEC == 1 && !is_bf16b<PREC>()) zero = 0.f;
+  if constexpr (VEC == 1) zero = (et)0.f;
   else
 #pragma unroll
     for (int v = 0; v < VEC; ++v) zero[v] = (et)0.f;
 #pragma unroll
-  for (int s = 0; s < NSUB; ++s) {
-    const int col = colbase + s * 16 * VEC;
-    const bool colok = col < p.N;
-    const int colc = colok ? col : 0;
+  for (int s = 0; s < NSUB; ++s)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int r = rows[j];
-      const bool ok = colok && (unsigned)r < (unsigned)p.b_rows;
-      const int rc = ok ? r : 0;
-      const vt v = *reinterpret_cast<const vt *>(B + (int64_t)rc * N + colc);
-      breg[s][j] = ok ? v : zero;
+      const bool in = ok && (unsigned)rows[j] < (unsigned)p.b_rows;
+      const vt v = *reinterpret_cast<const typename BElem<PREC, VEC>::type_u *>(
+          B + (int64_t)(in ? rows[j] : 0) * p.N + cols.c[s]);
+      breg[s][j] = in ? v : zero;
+    }
+}
+
+// B rows of the group into registers.  Lanes whose block lies past the group,
+// and slots whose row is not one of B's, get zeros: through buffers, from
+// byte offsets past B's end (its size is below 2^31).
+template <int PREC, int VEC, int NSUB, bool WIDE>
+__device__ __forceinline__ void gather_b(const SpmmParams &p, const Bufs<WIDE> &bufs, const Group &m,
+                                         const Cols<NSUB> &cols, breg_t<PREC, VEC> (&breg)[NSUB][8]) {
+  typedef breg_t<PREC, VEC> vt;
+  const int rows[8] = {m.r0.x, m.r0.y, m.r0.z, m.r0.w, m.r1.x, m.r1.y, m.r1.z, m.r1.w};
+  const bool ok = (lane_id() >> 4) < m.nblk;
+  if constexpr (WIDE) {
+    gather_ptr<PREC, VEC, NSUB>(p, rows, ok, cols, breg);
+  } else {
+    constexpr uint32_t esz = is_bf16b<PREC>() ? 2 : 4;
+    const uint32_t stride = (uint32_t)p.N * esz;
+    uint32_t base[NSUB];
+#pragma unroll
+    for (int s = 0; s < NSUB; ++s) base[s] = ok ? (uint32_t)cols.c[s] * esz : 0x80000000u;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t r = __umul24(min((uint32_t)rows[j], (uint32_t)p.b_rows), stride);
+#pragma unroll
+      for (int s = 0; s < NSUB; ++s) {
+        const uint32_t o = r + base[s];
+        constexpr int bytes = VEC * (int)esz;
+        if constexpr (bytes == 16)
+          breg[s][j] = __builtin_bit_cast(vt, __builtin_amdgcn_raw_buffer_load_b128(bufs.b, o, 0, 0));
+        else if constexpr (bytes == 8)
+          breg[s][j] = __builtin_bit_cast(vt, __builtin_amdgcn_raw_buffer_load_b64(bufs.b, o, 0, 0));
+        else
+          breg[s][j] = __builtin_bit_cast(vt, __builtin_amdgcn_raw_buffer_load_b32(bufs.b, o, 0, 0));
+      }
     }
   }
 }
 
 // Dense 16x8 A tiles of the group in this wave's LDS, then this lane's
-// operand A_g[q][0..7].
-__device__ __forceinline__ void build_a(const SpmmParams &p, const GroupMeta &m, bool has_vals,
-                                        float *lds, float (&a)[8]) {
+// operand A_g[q][0..7].  Element (block gg, row, slot) lies at float
+// (slot / 4) * 256 + (16 gg + row) * 4 + slot % 4: lane 16 gg + row reads its
+// two float4 with consecutive lanes on consecutive addresses (no bank
+// conflicts).  Stored elements are added (LDS float atomics): a CSR with a
+// repeated (row, column) pair puts several elements on one tile id, and the
+// product must count each of them, as the CSR product does.
+template <int MODE>
+__device__ __forceinline__ void build_a(const SpmmParams &p, const Bufs<MODE == kPtr> &bufs, const Group &m,
+                                        bool has_vals, float *lds, float (&a)[8]) {
   const int lane = lane_id();
-  const int g = lane >> 4;
-  const int q = lane & 15;
   floatx4 *t4 = reinterpret_cast<floatx4 *>(lds);
   const floatx4 z4 = {0.f, 0.f, 0.f, 0.f};
-  t4[lane * 2] = z4;
-  t4[lane * 2 + 1] = z4;
+  t4[lane] = z4;
+  t4[kWave + lane] = z4;
   wave_lds_sync();
-  // Stored elements are added into the tile (LDS float atomics): a CSR with
-  // a repeated (row, column) pair puts several elements on one tile id, and
-  // the product must count each of them, as the CSR product does.
-  if (m.o0 + lane < m.o4) {
-    const int e = m.o0 + lane;
+  auto add = [&](int e, int t, float v) {
     const int gg = (e >= m.o1) + (e >= m.o2) + (e >= m.o3);
-    atomicAdd(&lds[gg * (kBlkH * kBlkW) + (m.tile & (kBlkH * kBlkW - 1))], m.val);
-  }
-  for (int e = m.o0 + 64 + lane; e < m.o4; e += 64) {
-    const int gg = (e >= m.o1) + (e >= m.o2) + (e >= m.o3);
-    const float v = has_vals ? p.vals[e] : 1.0f;
-    atomicAdd(&lds[gg * (kBlkH * kBlkW) + (p.tile[e] & (kBlkH * kBlkW - 1))], v);
+    atomicAdd(&lds[((t & 4) << 6) | (gg << 6) | (((t >> 3) & 15) << 2) | (t & 3)], v);
+  };
+  if constexpr (MODE == kDense) {
+    int e = (m.o0 & ~3) + 4 * lane;
+    auto add4 = [&](int t, float v0, float v1, float v2, float v3) {
+      if (e >= m.o0 && e < m.o4) add(e, t, v0);
+      if (e + 1 >= m.o0 && e + 1 < m.o4) add(e + 1, t >> 8, v1);
+      if (e + 2 >= m.o0 && e + 2 < m.o4) add(e + 2, t >> 16, v2);
+      if (e + 3 < m.o4) add(e + 3, t >> 24, v3);
+    };
+    add4(m.tile, m.v0, m.v1, m.v2, m.v3);
+    for (int first = (m.o0 & ~3) + 4 * kWave; first < m.o4; first += 4 * kWave) {  // more than 253 elements
+      e += 4 * kWave;
+      const int t = (int)__builtin_amdgcn_raw_buffer_load_b32(bufs.tile, (uint32_t)e, 0, 0);
+      floatx4 v = {1.f, 1.f, 1.f, 1.f};
+      if (has_vals)
+        v = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(bufs.vals, (uint32_t)e * 4u, 0, 0));
+      add4(t, v[0], v[1], v[2], v[3]);
+    }
+  } else {
+    int e = m.o0 + lane;
+    if (e < m.o4) add(e, m.tile, m.v0);
+    if (m.o4 - m.o0 > kWave) {
+      e += kWave;
+      if (e < m.o4) add(e, m.tile2, m.v1);
+      for (e += kWave; e < m.o4; e += kWave) add(e, p.tile[e], has_vals ? p.vals[e] : 1.0f);
+    }
   }
   wave_lds_sync();
-  const floatx4 lo = t4[(g * (kBlkH * kBlkW) + q * kBlkW) / 4];
-  const floatx4 hi = t4[(g * (kBlkH * kBlkW) + q * kBlkW) / 4 + 1];
+  const floatx4 lo = t4[lane];
+  const floatx4 hi = t4[kWave + lane];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     a[j] = lo[j];
     a[j + 4] = hi[j];
   }
   wave_lds_sync();
-}
-
-// Accumulates the TC blocks [b0, b1) of one window into acc.  Software
-// pipelined: group i's B gathers are issued, then group i+1's metadata, then
-// group i's A tile is built and multiplied.
-template <int PREC, int VEC, int NSUB>
-__device__ __forceinline__ void run_blocks(const SpmmParams &p, int b0, int b1, int colbase,
-                                           float *lds, floatx4 (&acc)[NSUB][VEC],
-                                           bool has_vals) {
-  if (b0 >= b1) return;
-  GroupMeta cur;
-  load_meta<false>(p, b0, b1, has_vals, cur);
-  resolve_meta<false>(p, b1, cur);
-  for (int bb = b0; bb < b1; bb += kGroup) {
-    breg_t<PREC, VEC> breg[NSUB][8];
-    int rows[8];
-    meta_rows(cur, rows);
-    gather_b<PREC, VEC, NSUB>(p, rows, colbase, breg);
-    // The last group re-reads its own metadata instead of branching.
-    const int bn = (bb + kGroup < b1) ? bb + kGroup : bb;
-    GroupMeta nxt;
-    load_meta<false>(p, bn, b1, has_vals, nxt);
-    float a[8];
-    build_a(p, cur, has_vals, lds, a);
-    mfma_group<PREC, VEC, NSUB>(a, breg, acc, has_vals);
-    cur = nxt;
-    resolve_meta<false>(p, b1, cur);
-  }
 }
 
 template <int VEC, int NSUB>
@@ -493,54 +580,70 @@ __device__ __forceinline__ void zero_acc(floatx4 (&acc)[NSUB][VEC]) {
     for (int v = 0; v < VEC; ++v) acc[s][v] = floatx4{0.f, 0.f, 0.f, 0.f};
 }
 
-// Writes the 16 rows of window w held in acc.
-template <int VEC, int NSUB>
-__device__ __forceinline__ void store_window(const SpmmParams &p, int w, int colbase,
-                                             const floatx4 (&acc)[NSUB][VEC]) {
-  typedef typename VecType<VEC>::type vfloat;
-  const int lane = lane_id();
+// A row's vector in C: aligned to a float only (any N).
+template <int VEC>
+struct CVec {
+  typedef typename VecType<VEC>::type type __attribute__((aligned(4)));
+};
+
+// lane_id(), recomputed where it is used: what is derived from it cannot be
+// hoisted out of the walk loop, where the rarely run store paths' addresses
+// would be held in registers (or scratch) across every group.
+__device__ __forceinline__ int lane_here() {
+  int lane = lane_id();
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
+// First of this lane's four rows of C in window w, at column col.
+template <bool WIDE>
+__device__ __forceinline__ float *c_rows(const SpmmParams &p, int w, int lane, int col) {
+  float *base = p.C + (int64_t)w * kBlkH * p.N;  // wave-uniform
   const int g = lane >> 4;
-  const int64_t N = p.N;
+  if constexpr (WIDE) return base + (int64_t)(4 * g) * p.N + col;
+  return reinterpret_cast<float *>(reinterpret_cast<char *>(base) + (uint32_t)(4 * g * p.N + col) * 4u);
+}
+
+// Writes the 16 rows of window w held in acc.
+template <int VEC, int NSUB, bool WIDE>
+__device__ __forceinline__ void store_window(const SpmmParams &p, int w, const Cols<NSUB> &cols,
+                                             const floatx4 (&acc)[NSUB][VEC]) {
+  typedef typename CVec<VEC>::type vfloat;
+  if (w < 0) return;
+  const int lane = lane_here();
+  const int64_t left = p.M - (int64_t)w * kBlkH - 4 * (lane >> 4);  // rows from this lane's first on
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t row = (int64_t)w * kBlkH + 4 * g + i;
-    if (row < 0 || row >= p.M) continue;
+  for (int s = 0; s < NSUB; ++s) {
+    float *c = c_rows<WIDE>(p, w, lane, cols.c[s]);
 #pragma unroll
-    for (int s = 0; s < NSUB; ++s) {
-      const int col = colbase + s * 16 * VEC;
-      if (col >= p.N) continue;
+    for (int i = 0; i < 4; ++i) {
       vfloat out;
       if constexpr (VEC == 1) out = acc[s][0][i];
       else
 #pragma unroll
         for (int v = 0; v < VEC; ++v) out[v] = acc[s][v][i];
-      __builtin_nontemporal_store(out, reinterpret_cast<vfloat *>(p.C + row * N + col));
+      if (i < left) __builtin_nontemporal_store(out, reinterpret_cast<vfloat *>(c + (int64_t)i * p.N));
     }
   }
 }
 
 // Zeroes this wave's column tile of windows [w0, w1) (empty windows: no TC
 // block writes them, so any wave may, at any time of the launch).
-template <int VEC, int NSUB>
-__device__ __forceinline__ void zero_windows(const SpmmParams &p, int w0, int w1, int colbase) {
-  typedef typename VecType<VEC>::type vfloat;
+template <int VEC, int NSUB, bool WIDE>
+__device__ __forceinline__ void zero_windows(const SpmmParams &p, int w0, int w1, const Cols<NSUB> &cols) {
+  typedef typename CVec<VEC>::type vfloat;
   const vfloat z = vzero<VEC>();
-  const int g = lane_id() >> 4;
-  const int64_t N = p.N;
-  // Rolled: rare, and unrolled stores would hold their addresses in registers
-  // across the whole SpMM loop.
+  const int lane = lane_here();
 #pragma unroll 1
-  for (int r = max(w0, 0) * kBlkH; r < w1 * kBlkH; r += kBlkH) {
+  for (int w = max(w0, 0); w < w1; ++w) {
+    const int64_t left = p.M - (int64_t)w * kBlkH - 4 * (lane >> 4);
 #pragma unroll 1
-    for (int i = 0; i < 4; ++i) {
-      const int64_t row = (int64_t)r + 4 * g + i;
-      if (row >= p.M) continue;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int s = 0; s < NSUB; ++s) {
-        const int col = colbase + s * 16 * VEC;
-        if (col < p.N) __builtin_nontemporal_store(z, reinterpret_cast<vfloat *>(p.C + row * N + col));
-      }
-    }
+      for (int s = 0; s < NSUB; ++s)
+        if (i < left)
+          __builtin_nontemporal_store(
+              z, reinterpret_cast<vfloat *>(c_rows<WIDE>(p, w, lane, cols.c[s]) + (int64_t)i * p.N));
   }
 }
 
@@ -555,26 +658,27 @@ __device__ __forceinline__ void zero_windows(const SpmmParams &p, int w0, int w1
 // tiles of 16 x TW floats; k_balance_fixup sums them in chunk order.  The
 // chunk index is the one run_unit left in the wave's LDS state word.
 template <int VEC, int NSUB>
-__device__ __forceinline__ void add_window_atomic(const SpmmParams &p, int w, int colbase,
+__device__ __forceinline__ void add_window_atomic(const SpmmParams &p, int w, int ct, const Cols<NSUB> &cols,
                                                   float *lds, const floatx4 (&acc)[NSUB][VEC],
                                                   bool last_role) {
   constexpr int TW = 16 * VEC * NSUB;  // tile width in floats
-  const int lane = lane_id();
+  const int lane = lane_here();
   const int g = lane >> 4;
-  const int q = lane & 15;
+  const int col0 = ct * TW;  // first column of the tile
 #pragma unroll
-  for (int s = 0; s < NSUB; ++s)
+  for (int s = 0; s < NSUB; ++s) {
+    const int lc = cols.c[s] - col0;  // below 0: a moved-back lane's columns of the previous tile
 #pragma unroll
     for (int v = 0; v < VEC; ++v)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) lds[(4 * g + i) * TW + s * 16 * VEC + q * VEC + v] = acc[s][v][i];
+      for (int i = 0; i < 4; ++i)
+        if (lc + v >= 0) lds[(4 * g + i) * TW + lc + v] = acc[s][v][i];
+  }
   wave_lds_sync();
-  const int col0 = colbase - q * VEC;  // first column of the tile
   const int64_t N = p.N;
   if (p.parts) {
     const int item = wave_uniform(reinterpret_cast<const int *>(lds)[wave_lds_floats<VEC, NSUB>()]);
     const int slot = 2 * item + (last_role ? 1 : 0);
-    const int ct = wave_uniform(col0) / TW;
     float *dst = p.parts + ((int64_t)slot * p.n_ct + ct) * (kBlkH * TW);
 #pragma unroll 1
     for (int k = 0; k < kBlkH * TW / 64; ++k) dst[k * 64 + lane] = lds[k * 64 + lane];
@@ -594,68 +698,157 @@ __device__ __forceinline__ void add_window_atomic(const SpmmParams &p, int w, in
   wave_lds_sync();
 }
 
-// Accumulates the TC blocks [b, e) of the balanced schedule, which may span
-// many windows, as ONE software pipeline: groups never cross a window start
-// (they are the groups a per-window loop would form), and when a group opens
-// a new window the accumulators of the previous one are stored and cleared.
-// Window `atomic_w0` (if >= 0) and `atomic_w1` (if >= 0) are merged with
-// atomic adds (windows cut at chunk boundaries), every other window is
-// stored whole.  Empty windows are zeroed by the wave that passes them: the
-// gap before the run's first window (after the previous block's window), the
-// gaps between consecutive windows, and -- for the run that ends at the last
-// block -- the windows after it.  Window starts come from the look-ahead of
-// window ids loaded with each group's metadata, so no window is searched for.
-template <int PREC, int VEC, int NSUB>
-__device__ __forceinline__ void walk_blocks(const SpmmParams &p, int b, int e, int colbase,
-                                            float *lds, floatx4 (&acc)[NSUB][VEC],
-                                            bool has_vals, int atomic_w0, int atomic_w1) {
-  GroupMeta cur;
-  load_meta<true>(p, b, e, has_vals, cur);
-  const int prev_w = b > 0 ? wave_uniform(p.rowid[b - 1]) : -1;
-  resolve_meta<true>(p, e, cur);
-  int cw = wave_uniform(cur.rid);
-  // pending empty windows [gap0, gap1): zeroed at one place in the loop
-  int gap0 = prev_w + 1;
-  int gap1 = min(cw, p.num_windows);
+// The blocks of one work unit as ONE software pipeline over K = 32 groups,
+// windows and all: groups never cross a window start (they are the groups a
+// per-window loop would form), and when a group opens a new window the
+// accumulators of the previous one are stored and cleared.
+//   Balanced schedule: the blocks [b, e) of a chunk's run.  Window starts
+//     come from the stage's window ids (one ballot per stage).  Windows
+//     atomic_w0 / atomic_w1 (if >= 0) are merged with atomic adds (windows
+//     cut at chunk boundaries), every other window is stored whole.
+//   Unbalanced schedule: the windows [w0, w1), at most 63 of them; lane l
+//     holds RowWindowOffset[w0 + l].
+//   Split schedule: the blocks [b, e) of window w0, left in acc.
+// Empty windows are zeroed by the wave that passes them: the gap before the
+// unit's first block, the gaps between its windows, and after its last one.
+//
+// Per group i: the next group's position (scalar, from the stage held in
+// registers: no load to wait for), its metadata loads, group i's gathers,
+// the previous window's stores if the window changed, group i's A tile, the
+// MFMAs.  Loads retire in order, so waiting for the gathers of group i also
+// waits for the metadata of group i + 1, which was issued before them: one
+// exposed memory latency per group, the gathers' own.
+template <int PREC, int VEC, int NSUB, int SCHED, int MODE>
+__device__ __forceinline__ void walk_blocks(const SpmmParams &p, int b, int e, int w0, int w1, int rwo,
+                                            int ct, float *lds, int atomic_w0, int atomic_w1,
+                                            floatx4 (&acc)[NSUB][VEC]) {
+  constexpr bool BALANCED = SCHED == kBalanced;
+  constexpr bool WIDE = MODE == kPtr;
+  const bool has_vals = p.vals != nullptr;
+  const Cols<NSUB> cols = lane_cols<VEC, NSUB>(ct, p.N);
+  const Bufs<WIDE> bufs = make_bufs<PREC, WIDE, MODE == kDense>(p);
   zero_acc<VEC, NSUB>(acc);
+  Group cur;
+  int wi = 0, wend = 0;  // unbalanced: current window (relative to w0) and its end
+  if constexpr (SCHED == kSplit) {
+    wend = e;
+  } else if constexpr (!BALANCED) {
+    const int nw = w1 - w0;
+    while (wi < nw && __builtin_amdgcn_readlane(rwo, wi) >= __builtin_amdgcn_readlane(rwo, wi + 1)) ++wi;
+    if (wi == nw) {
+      zero_windows<VEC, NSUB, WIDE>(p, w0, w1, cols);
+      return;
+    }
+    b = __builtin_amdgcn_readlane(rwo, wi);
+    wend = __builtin_amdgcn_readlane(rwo, wi + 1);
+  }
+  cur.bb = b;
+  load_rows<MODE>(p, bufs, cur);  // needs no block offset: ahead of the stage's latency
+  Stage st = load_stage<BALANCED>(p, b, e);
+  Stage ahead = st;
+  if (b + kStageBlocks < e) ahead = load_stage<BALANCED>(p, b + kStageBlocks, e);
+  uint64_t starts = 0;
+  auto find_starts = [&]() {
+    if constexpr (BALANCED) {
+      const int prev = __shfl_up(st.wid, 1, 64);
+      starts = __ballot(st.wid != prev);  // bit 0 is never looked at
+    }
+  };
+  // Position of the group that starts at block bb (inside the stage).
+  auto place = [&](int bb, Group &m) {
+    const int k = bb - st.sb;
+    m.bb = bb;
+    if constexpr (BALANCED) {
+      m.nblk = 1 + (int)__builtin_ctzll((starts >> (k + 1)) | 8u);
+      m.w = __builtin_amdgcn_readlane(st.wid, k);
+    } else {
+      m.nblk = min(kGroup, wend - bb);
+      m.w = w0 + wi;
+    }
+    // Blocks past the group's end need no offset: an element below o4 lies
+    // below their starts.
+    m.o4 = min(__builtin_amdgcn_readlane(st.off, k + m.nblk), p.nnz);
+    m.o0 = max(__builtin_amdgcn_readlane(st.off, k), 0);
+    m.o1 = __builtin_amdgcn_readlane(st.off, k + 1);
+    m.o2 = __builtin_amdgcn_readlane(st.off, k + 2);
+    m.o3 = __builtin_amdgcn_readlane(st.off, k + 3);
+  };
+  find_starts();
+  place(b, cur);
+  load_elems<MODE>(p, bufs, has_vals, cur);
+  int cw = cur.w;
+  // pending empty windows [gap0, gap1): zeroed at one place in the loop
+  int gap0 = w0;
+  int gap1 = cw;
+  if constexpr (BALANCED) {
+    gap0 = (b > 0 ? wave_uniform(p.rowid[b - 1]) : -1) + 1;
+    gap1 = min(cw, p.num_windows);
+  }
   while (true) {
+    // next group
+    int bn = cur.bb + cur.nblk;
+    bool more;
+    if constexpr (BALANCED || SCHED == kSplit) {
+      more = bn < e;
+    } else {
+      more = true;
+      if (bn >= wend) {
+        const int nw = w1 - w0;
+        do {
+          ++wi;
+        } while (wi < nw && __builtin_amdgcn_readlane(rwo, wi) >= __builtin_amdgcn_readlane(rwo, wi + 1));
+        more = wi < nw;
+        if (more) {
+          bn = __builtin_amdgcn_readlane(rwo, wi);
+          wend = __builtin_amdgcn_readlane(rwo, wi + 1);
+        }
+      }
+    }
+    Group nxt = cur;  // the last group re-reads its own metadata
+    if (more) {
+      if ((unsigned)(bn - st.sb) >= (unsigned)kStageBlocks) {
+        if ((unsigned)(bn - ahead.sb) < (unsigned)kStageBlocks) st = ahead;
+        else st = load_stage<BALANCED>(p, bn, e);
+        if (st.sb + kStageBlocks < e) ahead = load_stage<BALANCED>(p, st.sb + kStageBlocks, e);
+        find_starts();
+      }
+      place(bn, nxt);
+    }
+    load_rows<MODE>(p, bufs, nxt);
+    load_elems<MODE>(p, bufs, has_vals, nxt);
     breg_t<PREC, VEC> breg[NSUB][8];
-    int rows[8];
-    meta_rows(cur, rows);
-    gather_b<PREC, VEC, NSUB>(p, rows, colbase, breg);
+    gather_b<PREC, VEC, NSUB, WIDE>(p, bufs, cur, cols, breg);
     // The previous window's stores go out after this group's gathers: loads
     // and stores retire through one in-order counter, so a store issued first
     // would hold up the wait for the gathers.
-    const int w = wave_uniform(cur.rid);  // window of block cur.bb (lane 0)
-    if (w != cw) {
-      if (cw == atomic_w0 || cw == atomic_w1)
-        add_window_atomic<VEC, NSUB>(p, cw, colbase, lds, acc, cw != atomic_w0);
-      else store_window<VEC, NSUB>(p, cw, colbase, acc);
+    if (SCHED != kSplit && cur.w != cw) {
+      if (BALANCED && (cw == atomic_w0 || cw == atomic_w1))
+        add_window_atomic<VEC, NSUB>(p, cw, ct, cols, lds, acc, cw != atomic_w0);
+      else store_window<VEC, NSUB, WIDE>(p, cw, cols, acc);
       zero_acc<VEC, NSUB>(acc);
       gap0 = cw + 1;
-      gap1 = min(w, p.num_windows);
-      cw = w;
+      gap1 = min(cur.w, p.num_windows);
+      cw = cur.w;
     }
-    if (gap0 < gap1) {
-      zero_windows<VEC, NSUB>(p, gap0, gap1, colbase);
+    if (SCHED != kSplit && gap0 < gap1) {
+      zero_windows<VEC, NSUB, WIDE>(p, gap0, gap1, cols);
       gap0 = gap1;
     }
-    const int bn = cur.bb + cur.nblk;
-    const bool more = bn < e;
-    // The last group re-reads its own metadata instead of branching.
-    GroupMeta nxt;
-    load_meta<true>(p, more ? bn : cur.bb, e, has_vals, nxt);
     float a[8];
-    build_a(p, cur, has_vals, lds, a);
+    build_a<MODE>(p, bufs, cur, has_vals, lds, a);
     mfma_group<PREC, VEC, NSUB>(a, breg, acc, has_vals);
     if (!more) break;
     cur = nxt;
-    resolve_meta<true>(p, e, cur);
   }
-  if (cw == atomic_w0 || cw == atomic_w1)
-    add_window_atomic<VEC, NSUB>(p, cw, colbase, lds, acc, cw != atomic_w0);
-  else store_window<VEC, NSUB>(p, cw, colbase, acc);
-  if (e == p.num_blocks) zero_windows<VEC, NSUB>(p, cw + 1, p.num_windows, colbase);
+  if constexpr (SCHED == kSplit) return;  // the caller merges acc
+  if (BALANCED && (cw == atomic_w0 || cw == atomic_w1))
+    add_window_atomic<VEC, NSUB>(p, cw, ct, cols, lds, acc, cw != atomic_w0);
+  else store_window<VEC, NSUB, WIDE>(p, cw, cols, acc);
+  if constexpr (BALANCED) {
+    if (e == p.num_blocks) zero_windows<VEC, NSUB, WIDE>(p, cw + 1, p.num_windows, cols);
+  } else {
+    zero_windows<VEC, NSUB, WIDE>(p, cw + 1, w1, cols);
+  }
 }
 
 // End of window w whose block b is known: one ballot over the next 64 block
@@ -676,20 +869,16 @@ __device__ __forceinline__ int window_start_from(const int32_t *rowid, int b, in
   return wave_lower_bound<int32_t>(rowid, 0, b - 64, w);
 }
 
-template <int PREC, int VEC, int NSUB, bool BALANCED>
+template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
 __device__ __forceinline__ void run_unit(const SpmmParams &p, int item, int ct, float *lds) {
-  const int lane = lane_id();
-  const int colbase = ct * (16 * VEC * NSUB) + (lane & 15) * VEC;
-  const bool has_vals = p.vals != nullptr;
   floatx4 acc[NSUB][VEC];
   if constexpr (!BALANCED) {
-    const int w = item;
+    const int w0 = item * p.chunk;
+    const int w1 = min(w0 + p.chunk, p.num_windows);
     // Offsets are clamped to the blocks actually passed in.
-    const int b1 = max(0, min(p.rwo[w + 1], p.num_blocks));
-    const int b0 = max(0, min(p.rwo[w], b1));
-    zero_acc<VEC, NSUB>(acc);
-    run_blocks<PREC, VEC, NSUB>(p, b0, b1, colbase, lds, acc, has_vals);
-    store_window<VEC, NSUB>(p, w, colbase, acc);
+    const int rwo = max(0, min(p.rwo[min(w0 + lane_id(), w1)], p.num_blocks));
+    const int end = __builtin_amdgcn_readlane(rwo, w1 - w0);
+    walk_blocks<PREC, VEC, NSUB, kWindows, MODE>(p, 0, end, w0, w1, rwo, ct, lds, -1, -1, acc);
   } else {
     // The chunk's run and the windows it merges atomically were worked out
     // by the preparation kernel (k_balance_prep).
@@ -705,41 +894,89 @@ __device__ __forceinline__ void run_unit(const SpmmParams &p, int item, int ct, 
       reinterpret_cast<int *>(lds)[wave_lds_floats<VEC, NSUB>()] = item;
       wave_lds_sync();
     }
-    walk_blocks<PREC, VEC, NSUB>(p, b, e, colbase, lds, acc, has_vals, w_first, w_last);
+    walk_blocks<PREC, VEC, NSUB, kBalanced, MODE>(p, b, e, 0, 0, 0, ct, lds, w_first, w_last, acc);
   }
 }
 
-// Waves per SIMD the compiler must leave room for (its register budget),
-// per instance.  Left to itself it keeps the balanced kernels' accumulators
-// in AGPRs and stops at 5 waves with 32-column tiles; asked for 7 it fits
-// them in 70 VGPRs without scratch, and the SpMM runs ~5% faster (R-MAT
-// scale 20: 4.23 -> 4.00 ms at N = 256, 0.60 -> 0.56 ms at N = 32).  With
-// 64-column tiles, 5 waves instead of 4 measured no faster; the bf16x3 and
-// bf16x6 splits would spill.  Those keep the default.
+// Waves per SIMD the compiler must leave room for (its register budget), per
+// instance: asked for these it keeps the accumulators out of the AGPRs and
+// spills nothing in the loop; left to itself it stops one or two waves short.
+// The bf16x3 and bf16x6 splits would spill and keep the default.
 template <int PREC, int VEC, int NSUB, bool BALANCED>
 constexpr int spmm_waves_per_eu() {
-  if (!BALANCED || PREC == DTC_PRECISION_BF16X3 || PREC == DTC_PRECISION_BF16X6) return 1;
-  return VEC * NSUB <= 2 ? 7 : 1;
+  if (PREC == DTC_PRECISION_BF16X3 || PREC == DTC_PRECISION_BF16X6) return 1;
+  if (is_bf16b<PREC>()) return VEC == 8 ? 4 : 5;
+  return VEC * NSUB <= 2 ? 6 : VEC * NSUB == 4 ? 5 : 1;
 }
 
-// Workgroup i serves column tile i % n_ct.  Workgroups are dispatched to the
+// Workgroup i serves column tile i % n_ct: workgroups are dispatched to the
 // 8 XCDs round robin, so when n_ct divides 8 every XCD (and its L2) only
-// sees one column tile of B: 1/n_ct of each gathered row.
-template <int PREC, int VEC, int NSUB, bool BALANCED>
+// sees one column tile of B.  With ct_blocks set, the column tiles go one
+// after another instead (workgroup i serves tile i / ct_blocks): all XCDs
+// then gather from the same column slice of B at a time.
+template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
 __global__ __launch_bounds__(256) __attribute__((
     amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED>()))) void spmm_kernel(SPMM_KERNEL_ARGS) {
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
   __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   const int wave = wave_uniform(threadIdx.x >> 6);
-  const int ct = blockIdx.x % p.n_ct;
-  const int item = (blockIdx.x / p.n_ct) * kWavesPerBlock + wave;
+  const int ct = p.ct_blocks ? blockIdx.x / p.ct_blocks : blockIdx.x % p.n_ct;
+  const int group = p.ct_blocks ? blockIdx.x % p.ct_blocks : blockIdx.x / p.n_ct;
+  const int item = group * kWavesPerBlock + wave;
   if (item >= p.num_items) return;
-  run_unit<PREC, VEC, NSUB, BALANCED>(p, item, ct, s_tile[wave]);
+  run_unit<PREC, VEC, NSUB, BALANCED, MODE>(p, item, ct, s_tile[wave]);
+}
+
+// Unbalanced schedule for launches that cannot fill the GPU: one workgroup
+// per (window, column tile), whose four waves take a quarter of the window's
+// groups each; their tiles are added through LDS in wave order (a fixed one:
+// the result stays repeatable).  A window's serial chain of gathers becomes a
+// quarter as long.
+template <int PREC, int VEC, int NSUB, int MODE>
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, false>()))) void spmm_kernel_split(SPMM_KERNEL_ARGS) {
+  const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
+  constexpr int TW = 16 * VEC * NSUB;
+  __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
+  const int wave = wave_uniform(threadIdx.x >> 6);
+  const int lane = lane_id();
+  const int ct = blockIdx.x % p.n_ct;
+  const int w = blockIdx.x / p.n_ct;  // the grid is n_ct * num_windows
+  const int b1 = max(0, min(wave_uniform(p.rwo[w + 1]), p.num_blocks));
+  const int b0 = max(0, min(wave_uniform(p.rwo[w]), b1));
+  const int per = (b1 - b0 + kGroup * kWavesPerBlock - 1) / (kGroup * kWavesPerBlock) * kGroup;  // blocks per wave
+  const int b = min(b0 + wave * per, b1);
+  const int e = min(b + per, b1);
+  floatx4 acc[NSUB][VEC];
+  if (b < e) walk_blocks<PREC, VEC, NSUB, kSplit, MODE>(p, b, e, w, w + 1, 0, ct, s_tile[wave], -1, -1, acc);
+  else zero_acc<VEC, NSUB>(acc);
+  const Cols<NSUB> cols = lane_cols<VEC, NSUB>(ct, p.N);
+  const int g = lane >> 4;
+#pragma unroll
+  for (int s = 0; s < NSUB; ++s) {
+    const int lc = cols.c[s] - ct * TW;  // below 0: a moved-back lane's columns of the previous tile
+#pragma unroll
+    for (int v = 0; v < VEC; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (lc + v >= 0) s_tile[wave][(4 * g + i) * TW + lc + v] = acc[s][v][i];
+  }
+  __syncthreads();
+  // 16 x TW sums, consecutive threads on consecutive columns
+#pragma unroll
+  for (int k = threadIdx.x; k < kBlkH * TW; k += 256) {
+    const int col = ct * TW + k % TW;
+    const int64_t row = (int64_t)w * kBlkH + k / TW;
+    if (row < p.M && col < p.N) {
+      const float sum = (s_tile[0][k] + s_tile[1][k]) + (s_tile[2][k] + s_tile[3][k]);
+      __builtin_nontemporal_store(sum, p.C + row * p.N + col);
+    }
+  }
 }
 
 // Persistent variant of the balanced schedule: every wave pulls units from a
 // global counter until the list is exhausted.
-template <int PREC, int VEC, int NSUB>
+template <int PREC, int VEC, int NSUB, int MODE>
 __global__ __launch_bounds__(256) __attribute__((
     amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, true>()))) void spmm_kernel_persistent(SPMM_KERNEL_ARGS) {
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
@@ -753,7 +990,7 @@ __global__ __launch_bounds__(256) __attribute__((
     u = __shfl(u, 0, 64);
     u = wave_uniform(u);
     if (u >= total) break;
-    run_unit<PREC, VEC, NSUB, true>(p, u / p.n_ct, u % p.n_ct, s_tile[wave]);
+    run_unit<PREC, VEC, NSUB, true, MODE>(p, u / p.n_ct, u % p.n_ct, s_tile[wave]);
   }
 }
 
@@ -983,54 +1220,85 @@ struct Variant {
   int prec;  // DTC_PRECISION_* or a bf16-B scheme
   int vec;
   int nsub;
+  int mode;  // kPtr, kBuf or kDense
 };
 
-template <int PREC, int VEC, int NSUB>
+// Launch schedules of a kernel instance.
+constexpr int kRunWindows = 0, kRunBalanced = 1, kRunPersistent = 2, kRunSplit = 3;
+
+template <int PREC, int VEC, int NSUB, int MODE>
 KernelFn pick_schedule(int schedule) {
   switch (schedule) {
-    case 0: return spmm_kernel<PREC, VEC, NSUB, false>;
-    case 1: return spmm_kernel<PREC, VEC, NSUB, true>;
-    default: return spmm_kernel_persistent<PREC, VEC, NSUB>;
+    case kRunWindows: return spmm_kernel<PREC, VEC, NSUB, false, MODE>;
+    case kRunBalanced: return spmm_kernel<PREC, VEC, NSUB, true, MODE>;
+    case kRunPersistent: return spmm_kernel_persistent<PREC, VEC, NSUB, MODE == kDense ? kBuf : MODE>;
+    default: return spmm_kernel_split<PREC, VEC, NSUB, MODE>;
   }
 }
 
-template <int PREC>
-KernelFn pick_shape(int vec, int nsub, int schedule) {
-  if (vec == 4 && nsub == 2) return pick_schedule<PREC, 4, 2>(schedule);
-  if (vec == 4) return pick_schedule<PREC, 4, 1>(schedule);
-  if (vec == 2) return pick_schedule<PREC, 2, 1>(schedule);
-  return pick_schedule<PREC, 1, 1>(schedule);
+template <int PREC, int VEC, int NSUB>
+KernelFn pick_mode(const Variant &v, int schedule) {
+  return v.mode == kDense ? pick_schedule<PREC, VEC, NSUB, kDense>(schedule)
+                          : pick_schedule<PREC, VEC, NSUB, kBuf>(schedule);
 }
 
 template <int PREC>
-KernelFn pick_shape_bf16b(int vec, int schedule) {
-  if (vec == 8) return pick_schedule<PREC, 8, 1>(schedule);
-  return pick_schedule<PREC, 4, 1>(schedule);
+KernelFn pick_shape(const Variant &v, int schedule) {
+  if (v.mode == kPtr)
+    return v.vec == 4 ? pick_schedule<PREC, 4, 1, kPtr>(schedule) : pick_schedule<PREC, 1, 1, kPtr>(schedule);
+  if (v.vec == 4 && v.nsub == 2) return pick_mode<PREC, 4, 2>(v, schedule);
+  if (v.vec == 4) return pick_mode<PREC, 4, 1>(v, schedule);
+  if (v.vec == 2) return pick_mode<PREC, 2, 1>(v, schedule);
+  return pick_mode<PREC, 1, 1>(v, schedule);
+}
+
+template <int PREC>
+KernelFn pick_shape_bf16b(const Variant &v, int schedule) {
+  if (v.mode == kPtr) return pick_schedule<PREC, 4, 1, kPtr>(schedule);
+  if (v.vec == 8) return pick_mode<PREC, 8, 1>(v, schedule);
+  return pick_mode<PREC, 4, 1>(v, schedule);
 }
 
 KernelFn pick_kernel(const Variant &v, int schedule) {
   switch (v.prec) {
-    case DTC_PRECISION_FP32: return pick_shape<DTC_PRECISION_FP32>(v.vec, v.nsub, schedule);
-    case DTC_PRECISION_BF16: return pick_shape<DTC_PRECISION_BF16>(v.vec, v.nsub, schedule);
-    case DTC_PRECISION_FP16: return pick_shape<DTC_PRECISION_FP16>(v.vec, v.nsub, schedule);
-    case DTC_PRECISION_BF16X3: return pick_shape<DTC_PRECISION_BF16X3>(v.vec, v.nsub, schedule);
-    case kBf16B_A3: return pick_shape_bf16b<kBf16B_A3>(v.vec, schedule);
-    case kBf16B_A1: return pick_shape_bf16b<kBf16B_A1>(v.vec, schedule);
-    default: return pick_shape<DTC_PRECISION_BF16X6>(v.vec, v.nsub, schedule);
+    case DTC_PRECISION_FP32: return pick_shape<DTC_PRECISION_FP32>(v, schedule);
+    case DTC_PRECISION_BF16: return pick_shape<DTC_PRECISION_BF16>(v, schedule);
+    case DTC_PRECISION_FP16: return pick_shape<DTC_PRECISION_FP16>(v, schedule);
+    case DTC_PRECISION_BF16X3: return pick_shape<DTC_PRECISION_BF16X3>(v, schedule);
+    case kBf16B_A3: return pick_shape_bf16b<kBf16B_A3>(v, schedule);
+    case kBf16B_A1: return pick_shape_bf16b<kBf16B_A1>(v, schedule);
+    default: return pick_shape<DTC_PRECISION_BF16X6>(v, schedule);
   }
 }
 
-// Kernel scheme and lane shape from the options, N and operand alignment.
+// How the kernels read these operands.  Buffers need 32-bit byte offsets
+// (offsets of 2^31 and more lie past B's end) and 24-bit factors of a row's
+// offset.  The dense form pays where groups hold more than one load's 64
+// elements on average; it reads whole 4-element vectors, whose alignment
+// keeps the last one in the same 16 bytes as an element of the array.
+int operand_mode(int64_t b_rows, int64_t n, int64_t esz, int64_t nnz, int64_t num_blocks, const void *tile,
+                 const void *vals) {
+  const int64_t lim = (int64_t)1 << 31;
+  const bool fits = (b_rows + 1) * n * esz < lim && b_rows < (1 << 24) - 1 && n * esz < (1 << 24) &&
+                    nnz * 4 < lim - 64 && num_blocks * kBlkW * 4 < lim;
+  if (!fits) return kPtr;
+  const bool aligned = ((uintptr_t)tile & 3) == 0 && ((uintptr_t)vals & 15) == 0;
+  return aligned && nnz > 16 * num_blocks ? kDense : kBuf;
+}
+
+// Kernel scheme and lane shape from the options, N and operand alignment.  An
+// explicit vec must divide N and the base addresses; vec 0 takes any N of at
+// least its width (unaligned vectors, the last lanes moved back: lane_cols).
 // vec 0 for float32 B: 2 floats per lane (32-column tiles) in the balanced
-// schedule, 4 in the unbalanced one -- the widths measured fastest for each
-// across the selector's 2,000 training matrices -- or the widest narrower
-// width N and the alignment allow.
+// schedule, 4 in the unbalanced one, less where N is narrower.
 dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void *b, const float *c,
-                           bool balanced, Variant *out) {
+                           bool balanced, int mode, Variant *out) {
+  const bool wide = mode == kPtr;
   const int prec = opt ? opt->precision : DTC_PRECISION_FP32;
   const int bdt = opt ? opt->b_dtype : DTC_B_FLOAT32;
   int vec = opt ? opt->vec : 0;
   int nsub = opt ? opt->subtiles : 0;
+  out->mode = mode;
   if (bdt == DTC_B_BFLOAT16) {
     // bf16 B: 4 or 8 bf16 per lane (8 or 16 bytes), one subtile.
     if (vec != 0 && vec != 4 && vec != 8)
@@ -1038,14 +1306,18 @@ dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void 
     auto fits = [&](int v) {
       return n % v == 0 && ((uintptr_t)b % (2 * v)) == 0 && ((uintptr_t)c % (4 * v)) == 0;
     };
-    // Balanced: 128-column tiles, faster than 64 on R-MAT scales 18 and 20 (0.44 vs
-    // 0.49 ms and 1.89 vs 2.09 ms at chunk 64, N = 256); unbalanced: 64.
-    if (vec == 0) vec = (balanced && fits(8)) ? 8 : 4;
+    // 128-column tiles where N fills more than half of one
+    if (vec == 0) {
+      if (!fits(4))
+        return fail(DTC_ERROR_INVALID_VALUE,
+                    "bfloat16 B needs N to be a multiple of 4 and 8-byte aligned B/C rows");
+      vec = n > 64 ? 8 : 4;
+    } else
     if (!fits(vec))
       return fail(DTC_ERROR_INVALID_VALUE,
                   "bfloat16 B needs N to be a multiple of 4 and 8-byte aligned B/C rows");
     out->prec = (prec == DTC_PRECISION_BF16) ? kBf16B_A1 : kBf16B_A3;
-    out->vec = vec;
+    out->vec = wide ? 4 : vec;
     out->nsub = 1;
     return DTC_SUCCESS;
   }
@@ -1056,19 +1328,49 @@ dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void 
   auto fits = [&](int v) {
     return n % v == 0 && ((uintptr_t)b % (4 * v)) == 0 && ((uintptr_t)c % (4 * v)) == 0;
   };
-  if (vec == 0) {
-    const int pref = balanced ? 2 : 4;
-    vec = (pref >= 4 && fits(4)) ? 4 : (fits(2) ? 2 : 1);
-  }
-  if (!fits(vec))
+  if (vec != 0 && !fits(vec))
     return fail(DTC_ERROR_INVALID_VALUE,
                 "vec " + std::to_string(vec) + " needs N and the B/C base addresses to be multiples of it");
-  if (nsub == 0) nsub = 1;  // one 16*vec column tile per wave measured fastest on R-MAT and SBM
-  if (nsub == 2 && vec != 4) nsub = 1;
+  if (vec == 0) {
+    vec = n <= 16 ? 1 : n <= 32 ? 2 : 4;
+    // 128-column tiles (two 64-column subtiles) where 64-column ones would
+    // leave half of the last one empty, and for wide B in the unbalanced
+    // schedule
+    if (nsub == 0) nsub = (n % 128 > 64 && n % 128 <= 96) || (!balanced && n > 256) ? 2 : 1;
+  }
+  if (wide) vec = n >= 4 ? 4 : 1;
+  if (nsub == 0 || wide || vec != 4) nsub = 1;
   out->prec = prec;
   out->vec = vec;
   out->nsub = nsub;
   return DTC_SUCCESS;
+}
+
+// Whether the unbalanced schedule splits each window over a workgroup's four
+// waves: with at most one unit per SIMD (two when windows are long) the chip
+// idles while every wave walks its window's groups one after another.
+// Uniform matrices, 64-column tiles, us whole -> split: 128 windows of 57
+// blocks 17 -> 6.6, of 162 42 -> 13; 512 windows at 1,024 units, of 62 blocks
+// 19 -> 15.5, of 16 7.0 -> 7.5; at 2,048 units, of 62 28 -> 29, of 227 95 -> 85.
+bool split_windows(int64_t windows, int64_t n_ct, int64_t num_blocks) {
+  const int64_t units = windows * n_ct;
+  return (units <= 1024 && num_blocks > 5 * windows) || (units <= 2048 && num_blocks > 96 * windows);
+}
+
+// Consecutive windows per unit of the unbalanced schedule: short windows are
+// walked several to a wave, as one pipeline, while enough units remain.
+int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks) {
+  int32_t k = 1;
+  while (k < 32 && 2 * k * num_blocks <= 32 * windows && windows * n_ct >= 2 * k * 16384) k *= 2;
+  return k;
+}
+
+// Workgroups per column tile when the column tiles go one after another, 0
+// when they go side by side.  B beyond the 256 MB memory-side cache: one
+// slice at a time, so that most of its gathers hit there.
+int32_t column_order(const SpmmParams &p, int64_t esz) {
+  const int64_t b_bytes = (int64_t)p.b_rows * p.N * esz;
+  return p.n_ct > 1 && b_bytes > ((int64_t)256 << 20) ? (int32_t)ceil_div(p.num_items, kWavesPerBlock) : 0;
 }
 
 dtc_status_t check_common(const uint8_t *tile, const int32_t *off, const int32_t *atox,
@@ -1095,15 +1397,13 @@ dtc_status_t check_common(const uint8_t *tile, const int32_t *off, const int32_t
   return DTC_SUCCESS;
 }
 
-// Default balanced chunk: the largest power of two in [32, 512] that is at
-// most T / 8192, i.e. about 8K chunks (x column tiles) of work units once
-// the matrix is large enough.  On the selector's 400 held-out matrices this
-// rule is 12% slower than the per-matrix best variant on average, a fixed
-// 256 122% (small matrices leave most CUs idle with long chunks).
+// Default balanced chunk, in TC blocks: short chunks leave enough units on
+// small matrices, long ones cut fewer windows and start fewer units.
 int default_chunk_blocks(int32_t num_blocks) {
-  int c = 32;
-  while (c < 512 && (int64_t)c * 2 * 8192 <= (int64_t)num_blocks) c *= 2;
-  return c;
+  if (num_blocks < (1 << 15)) return 16;
+  if (num_blocks < (1 << 18)) return 32;
+  if (num_blocks < (1 << 21)) return 64;
+  return num_blocks < 6 * (1 << 20) ? 128 : 256;
 }
 
 // Cut span of the balanced schedule: options->cut_span_blocks, a positive
@@ -1179,7 +1479,7 @@ __global__ __launch_bounds__(256) void spmm_tcgnn_kernel(
   const int ct = blockIdx.x % p.n_ct;
   const int w = (blockIdx.x / p.n_ct) * kWavesPerBlock + wave;
   if (w >= W) return;
-  const int colbase = ct * 16 * VEC + (lane & 15) * VEC;  // this lane's columns, as in run_unit
+  const Cols<1> cols = lane_cols<VEC, 1>(ct, p.N);
   const int64_t r0 = (int64_t)w * kBlkH;
   const int ws = wave_uniform(rowptr[min(r0, (int64_t)p.M)]);
   const int we = wave_uniform(rowptr[min(r0 + kBlkH, (int64_t)p.M)]);
@@ -1217,15 +1517,14 @@ __global__ __launch_bounds__(256) void spmm_tcgnn_kernel(
       a[j + 4] = hi[j];
     }
     int rows[8];
-    const bool gv = g < nb - k0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) rows[j] = gv ? atox[g * kBlkW + j] : -1;
+    for (int j = 0; j < 8; ++j) rows[j] = atox[g * kBlkW + j];
     wave_lds_sync();
     breg_t<DTC_PRECISION_FP32, VEC> breg[1][8];
-    gather_b<DTC_PRECISION_FP32, VEC, 1>(p, rows, colbase, breg);
+    gather_ptr<DTC_PRECISION_FP32, VEC, 1>(p, rows, g < nb - k0, cols, breg);
     mfma_group<DTC_PRECISION_FP32, VEC, 1>(a, breg, acc, true);
   }
-  store_window<VEC, 1>(p, w, colbase, acc);
+  store_window<VEC, 1, true>(p, w, cols, acc);
 }
 
 }  // namespace dtc
@@ -1284,7 +1583,7 @@ dtc_status_t dtc_spmm_tcgnn(const int32_t *node_pointer, const int32_t *edge_lis
   o.vec = options ? options->vec : 0;
   o.subtiles = 1;
   Variant var;
-  dtc_status_t st = resolve_shape(&o, n, b, c, false, &var);
+  dtc_status_t st = resolve_shape(&o, n, b, c, false, kBuf, &var);
   if (st != DTC_SUCCESS) return st;
   const int32_t W = (int32_t)ceil_div(num_nodes, kBlkH);
   if (b_rows == 0) return zero_output(c, num_nodes, n, stream);
@@ -1335,7 +1634,9 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
     return fail(DTC_ERROR_INVALID_VALUE,
                 "Rowwindow_offset has " + std::to_string(num_windows) + " windows, fewer than num_nodes/16");
   Variant var;
-  st = resolve_shape(options, n, b, c, false, &var);
+  const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
+  const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
+  st = resolve_shape(options, n, b, c, false, mode, &var);
   if (st != DTC_SUCCESS) return st;
   // Only windows that hold output rows are processed.
   const int32_t W = (int32_t)std::min<int64_t>(num_windows, ceil_div(num_nodes, kBlkH));
@@ -1354,11 +1655,14 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   p.b_rows = b_rows;
   p.N = n;
   p.n_ct = (int32_t)ceil_div(n, 16 * var.vec * var.nsub);
-  p.num_items = W;
   p.num_blocks = num_blocks;
   p.nnz = nnz;
-  KernelFn fn = pick_kernel(var, 0);
-  const int64_t grid = (int64_t)p.n_ct * ceil_div(W, kWavesPerBlock);
+  const bool split = split_windows(W, p.n_ct, num_blocks);
+  p.chunk = split ? 1 : windows_per_unit(W, p.n_ct, num_blocks);
+  p.num_items = (int32_t)ceil_div(W, p.chunk);
+  p.ct_blocks = split ? 0 : column_order(p, esz);
+  KernelFn fn = pick_kernel(var, split ? kRunSplit : kRunWindows);
+  const int64_t grid = (int64_t)p.n_ct * (split ? W : ceil_div(p.num_items, kWavesPerBlock));
   if (grid > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "grid too large");
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, stream, p.rwo, p.rowid, p.tile, p.off,
                      p.atox, p.vals, p.B, p.C, p);
@@ -1403,7 +1707,9 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   if (num_blocks > 0 && (!tcblock_rowid || !tcblocktile_id || !sparse_atox))
     return fail(DTC_ERROR_INVALID_VALUE, "TCblock_rowid, TCblocktile_id and sparse_AToX_idx are required");
   Variant var;
-  st = resolve_shape(options, n, b, c, true, &var);
+  const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
+  const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
+  st = resolve_shape(options, n, b, c, true, mode, &var);
   if (st != DTC_SUCCESS) return st;
   const int chunk = (options && options->chunk_blocks > 0) ? options->chunk_blocks
                                                            : default_chunk_blocks(num_blocks);
@@ -1440,6 +1746,7 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   p.num_items = (int32_t)ceil_div(num_blocks, chunk);
   p.chunk = chunk;
   p.span = span;
+  p.ct_blocks = column_order(p, esz);
   p.queue = persistent ? static_cast<int32_t *>(workspace) : nullptr;
   int2 *runs = reinterpret_cast<int2 *>(static_cast<char *>(workspace) + kQueueBytes);
   p.runs = runs;
@@ -1451,7 +1758,7 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
       tcblock_rowid, num_blocks, num_nodes, n, chunk, span, p.num_items, c, p.queue, runs, det ? 0 : 1);
   DTC_LAUNCH_CHECK("balance_prep");
   if (!persistent) {
-    KernelFn fn = pick_kernel(var, 1);
+    KernelFn fn = pick_kernel(var, kRunBalanced);
     const int64_t grid = (int64_t)p.n_ct * ceil_div(p.num_items, kWavesPerBlock);
     if (grid > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "grid too large");
     hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, stream, p.rwo, p.rowid, p.tile, p.off,
@@ -1463,7 +1770,7 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
     const int64_t units = (int64_t)p.num_items * p.n_ct;
     const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(ceil_div(units, kWavesPerBlock),
                                                                 (int64_t)cus * 8));
-    KernelFn fn = pick_kernel(var, 2);
+    KernelFn fn = pick_kernel(var, kRunPersistent);
     hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, stream, p.rwo, p.rowid, p.tile, p.off,
                      p.atox, p.vals, p.B, p.C, p);
   }

@@ -1,0 +1,81 @@
+"""The SpMM kernels' forms at the sizes where they change: ragged widths, one
+to several element loads per group, windows split over a workgroup, several
+windows per wave; each against the float64 CSR product."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import say
+
+pytestmark = pytest.mark.gpu
+
+
+def random_csr(rng, rows, cols, lengths):
+    """Rows of the given lengths with distinct sorted columns."""
+    rowptr = np.zeros(rows + 1, np.int64)
+    rowptr[1:] = np.cumsum(lengths)
+    col = np.concatenate([np.sort(rng.choice(cols, k, replace=False)) for k in lengths] or [np.zeros(0, np.int64)])
+    values = rng.uniform(-1, 1, col.shape[0]).astype(np.float32)
+    return rowptr.astype(np.int32), col.astype(np.int32), values
+
+
+def check(rowptr, col, values, cols, n, schedule, **options):
+    """Componentwise: a float32 sum of k products is off by at most
+    (k + 4) 2^-24 of the sum of their magnitudes."""
+    from dtc.matrix import DTCMatrix
+    rows = rowptr.shape[0] - 1
+    A = DTCMatrix(rowptr, col, values, num_rows=rows, num_cols=cols)
+    B = np.random.default_rng(n).standard_normal((cols, n)).astype(np.float32)
+    out = torch.full((rows, n), float("nan"), device="cuda")
+    say("spmm path", rows, cols, n, schedule, options)
+    C = A.spmm(torch.from_numpy(B).cuda(), schedule=schedule, out=out, **options).cpu().numpy()
+    exact, mag = oracle.spmm_csr_f64(rowptr, col, values, B, rows, with_abs=True)
+    bound = (np.diff(rowptr)[:, None] + 4) * 2.0 ** -24 * mag
+    assert np.all(np.abs(C - exact) <= bound), (n, schedule, options)
+
+
+@pytest.mark.parametrize("schedule", ["windows", "balanced"])
+@pytest.mark.parametrize("n", [1, 3, 5, 15, 17, 31, 33, 47, 63, 65, 72, 97, 130, 191, 260])
+def test_ragged_widths(n, schedule):
+    """Widths that no vector divides: the last lanes of a row move back."""
+    rng = np.random.default_rng(n)
+    lengths = rng.integers(0, 20, 330)
+    lengths[160:200] = 0  # two empty windows
+    check(*random_csr(rng, 330, 200, lengths), 200, n, schedule)
+
+
+@pytest.mark.parametrize("schedule,options", [("windows", {}), ("balanced", {}), ("balanced", {"chunk_blocks": 5}),
+                                              ("balanced", {"deterministic": True, "chunk_blocks": 4})])
+@pytest.mark.parametrize("fill", [0.05, 0.2, 0.45, 0.7, 1.0])
+def test_elements_per_group(fill, schedule, options):
+    """Groups from a few elements to all 512: the first load's 64 (or 256),
+    the second's, and the loop past them."""
+    rng = np.random.default_rng(int(fill * 100))
+    lengths = np.full(150, int(fill * 96))
+    lengths[40:60] = 3  # a sparse window among them
+    check(*random_csr(rng, 150, 96, lengths), 96, 64, schedule, **options)
+
+
+@pytest.mark.parametrize("n", [16, 64, 100])
+@pytest.mark.parametrize("rows,long_row", [(16, 500), (15, 33), (1000, 900), (3000, 0)])
+def test_split_windows(rows, long_row, n):
+    """Few windows: each is shared by four waves, from none to many groups."""
+    rng = np.random.default_rng(rows)
+    lengths = rng.integers(4, 12, rows)
+    if rows > 100:
+        lengths[64:80] = 0
+        lengths[80:96] = 0
+        lengths[80] = 1  # a window of one entry
+    lengths[rows // 2] = max(long_row, lengths[rows // 2])
+    check(*random_csr(rng, rows, 1200, lengths), 1200, n, "windows")
+
+
+def test_several_windows_per_wave():
+    """Many short windows, empty ones among them, a ragged last one."""
+    rng = np.random.default_rng(9)
+    rows = 16 * 17000 + 5
+    lengths = rng.integers(0, 3, rows)
+    lengths[1600:4800] = 0
+    lengths[-21:] = 2
+    check(*random_csr(rng, rows, 500, lengths), 500, 260, "windows")
