@@ -57,6 +57,7 @@ class DTCMatrix:
         when a matrix is rebuilt from a cache file without ``__init__``)."""
         self._transpose = None
         self._perm_t = None
+        self._tc_edge_t = None
         self._max_window_blocks = None
 
     # ------------------------------------------------------------------ info
@@ -126,6 +127,17 @@ class DTCMatrix:
         self.transpose()
         return self._perm_t
 
+    @property
+    def tc_edge_t(self) -> torch.Tensor:
+        """CSR edge of A behind every TC position of A^T (perm_t after A^T's
+        tc_edge, composed once): A's CSR values reach A^T's TC order in one
+        gather."""
+        if self._tc_edge_t is None:
+            At = self.transpose()
+            # the gather moves 32-bit words whatever they hold
+            self._tc_edge_t = load_extension().gather(self._perm_t.view(torch.float32), At.tc_edge).view(torch.int32)
+        return self._tc_edge_t
+
     def transposed_operands(self, schedule: str = "windows", values: torch.Tensor | None = None) -> tuple:
         """A^T's ME-TCF operands as the reference's backward names take them in
         ``transposed`` (``backward_ptx_uint8_improved``, ``..._gcn``: schedule
@@ -137,7 +149,7 @@ class DTCMatrix:
         ext = load_extension()
         At = self.transpose()
         vals = values if values is not None else self.values
-        vals_t = None if vals is None else ext.gather(ext.gather(vals.contiguous(), self.perm_t), At.tc_edge)
+        vals_t = None if vals is None else ext.gather(vals.contiguous(), self.tc_edge_t)
         index = At.row_window_offset if schedule in ("windows", "unbalanced") else At.tcblock_rowid
         return (index, At.tcblocktile_id, At.tcblock_offset, At.sparse_atox, vals_t, At.num_rows)
 
@@ -165,8 +177,7 @@ class _SpMMFunction(torch.autograd.Function):
             d_values = ext.sddmm_csr(A.rowptr, A.col, dC, B.contiguous(), A.edge_to_row)
         if ctx.needs_input_grad[1]:
             At = A.transpose()
-            vals_t_csr = ext.gather(values.contiguous(), A.perm_t)
-            vals_t_tc = ext.gather(vals_t_csr, At.tc_edge)
+            vals_t_tc = ext.gather(values.contiguous(), A.tc_edge_t)
             d_B = At.spmm(dC, schedule=ctx.schedule, precision=ctx.precision, values_tc=vals_t_tc)
             # A^T has num_cols rows; B may have more (rows no column of A
             # reaches get zero gradient) or fewer (columns of A past B's rows
