@@ -626,6 +626,47 @@ Tensor gcn_transform(Tensor X, Tensor W_packed, int64_t F, bool relu) {
   return out;
 }
 
+// Gradients of act(X) W from dY float32: (dX or None, dW or None).
+py::tuple gcn_gradients(Tensor dY, Tensor X, Tensor W, bool relu, bool need_dx, bool need_dw) {
+  CHECK_INPUT(dY);
+  CHECK_INPUT(X);
+  CHECK_INPUT(W);
+  CHECK_DTYPE(dY, torch::kFloat32);
+  CHECK_DTYPE(W, torch::kBFloat16);
+  TORCH_CHECK(X.scalar_type() == torch::kFloat32 || X.scalar_type() == torch::kBFloat16,
+              "X must be float32 or bfloat16");
+  CHECK_SAME_DEVICE(X, dY);
+  CHECK_SAME_DEVICE(W, dY);
+  TORCH_CHECK(dY.dim() == 2 && X.dim() == 2 && W.dim() == 2, "dY, X and W must be 2-D");
+  const int64_t M = X.size(0), K = X.size(1), F = W.size(1);
+  TORCH_CHECK(W.size(0) == K && dY.size(0) == M && dY.size(1) == F, "inconsistent shapes");
+  TORCH_CHECK(M < INT32_MAX && K < INT32_MAX && F < INT32_MAX, "sizes out of range");
+  const int32_t xdt = X.scalar_type() == torch::kFloat32 ? DTC_GCN_X_FLOAT32 : DTC_GCN_X_BFLOAT16;
+  const c10::OptionalDeviceGuard guard(dY.device());
+  const auto u8 = dY.options().dtype(torch::kUInt8);
+  py::object dx = py::none(), dw = py::none();
+  if (need_dx) {
+    Tensor out = torch::empty_like(X);
+    Tensor ws = torch::empty({K * F * 2}, u8);
+    check_status(dtc_gcn_input_grad(dY.data_ptr<float>(), W.data_ptr(), X.data_ptr(), xdt, relu ? 1 : 0, (int32_t)M,
+                                    (int32_t)K, (int32_t)F, out.data_ptr(), ws.data_ptr(), (size_t)ws.numel(),
+                                    current_stream()),
+                 "gcn_gradients");
+    dx = py::cast(out);
+  }
+  if (need_dw) {
+    size_t bytes = 0;
+    check_status(dtc_gcn_weight_grad_workspace_size((int32_t)M, (int32_t)K, (int32_t)F, &bytes), "gcn_gradients");
+    Tensor out = torch::empty_like(W);
+    Tensor ws = torch::empty({(int64_t)bytes}, u8);
+    check_status(dtc_gcn_weight_grad(X.data_ptr(), xdt, relu ? 1 : 0, dY.data_ptr<float>(), (int32_t)M, (int32_t)K,
+                                     (int32_t)F, out.data_ptr(), ws.data_ptr(), bytes, current_stream()),
+                 "gcn_gradients");
+    dw = py::cast(out);
+  }
+  return py::make_tuple(dx, dw);
+}
+
 // ------------------------------------------------------------- selector
 
 void check_f32_2d(const Tensor &t, const char *name) {
@@ -910,6 +951,8 @@ PYBIND11_MODULE(DTCSpMM, m) {
   m.def("gather", &gather, "out[p] = values[index[p]]", py::arg("values"), py::arg("index"));
   m.def("gcn_pack_weights", &gcn_pack_weights, "W [K x F] bf16 -> the GCN transform's fragment order",
         py::arg("W"));
+  m.def("gcn_gradients", &gcn_gradients, "(dX or None, dW or None) of act(X) W from dY float32", py::arg("dY"),
+        py::arg("X"), py::arg("W"), py::arg("relu"), py::arg("need_dx"), py::arg("need_dw"));
   m.def("gcn_transform", &gcn_transform, "bf16(act(X) W) as the bf16 B of the SpMM", py::arg("X"),
         py::arg("W_packed"), py::arg("F"), py::arg("relu") = false);
   m.attr("BLK_H") = kBlkH;

