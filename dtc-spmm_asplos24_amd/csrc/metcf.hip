@@ -11,24 +11,27 @@
 //
 //   LDS path (16-row windows of 8-column blocks, E <= 16,384): one workgroup
 //   per window (five shapes, 1 to 16 waves, up to 512 ... 16,384 entries;
-//   windows of at most 64 entries take one wave each and bitonic sorts)
-//   sorts the window's (column, local index) pairs in LDS (LSD radix sort
-//   over the window's column span, ranks from LDS atomics in the first pass
-//   and from wave ballots in the stable later ones), numbers the distinct
-//   columns by a workgroup scan and writes every output sized by the CSR:
+//   windows of at most 64 entries take one wave each and bitonic sorts).  When
+//   every row's columns strictly increase, entries are numbered from bitmaps
+//   of the window's columns (k_window_bits); otherwise the window's (column,
+//   local index) pairs are sorted in LDS (LSD radix sort over the window's
+//   column span, ranks from LDS atomics in the first pass and from wave
+//   ballots in the stable later ones) and the distinct columns numbered by a
+//   workgroup scan (k_window_sort).  Both write every output sized by the CSR:
 //   edgeToRow, edgeToColumn, blockPartition, and the tile ids, values and
 //   edge indices in TC-block order, each entry at its block's start plus
 //   the number of the block's entries with a smaller CSR index (the
 //   reference's CSR-order placement inside a block, :291-300).
 //
 //   Global path (larger windows, and every window of other block shapes),
-//   on a side stream beside the LDS path: the windows are compacted and
-//   sorted by column, each within its own range (segmented radix sort of
-//   32-bit keys) when they average at least one sort tile, else together by
-//   (compacted window, column); the inclusive scan G of "key differs from
-//   its predecessor" gives every sorted element its unique-column number, so
-//   the rank of a column inside its window is G - G(window start), and
-//   edge-parallel kernels write the same outputs.
+//   on a side stream beside the LDS path.  16 x 8 windows whose rows strictly
+//   increase: bitmaps again, of column slices (k_slice_mark).  Others: the
+//   windows are compacted and sorted by column, each within its own range
+//   (segmented radix sort of 32-bit keys) when they average at least one sort
+//   tile, else together by (compacted window, column); the inclusive scan G of
+//   "key differs from its predecessor" gives every sorted element its
+//   unique-column number, so the rank of a column inside its window is
+//   G - G(window start), and edge-parallel kernels write the same outputs.
 //
 // Both paths leave per-window block data in the workspace (distinct columns,
 // block starts, |S_w|); after the caller has allocated the block-sized
@@ -52,7 +55,7 @@ namespace {
 constexpr int kWinH = 16;  // rows per window on the LDS path (the reference's BLK_H)
 constexpr int kWinW = 8;   // columns per TC block on the LDS path (BLK_W)
 // Class 0 (at most 64 entries) is one wave per window with bitonic sorts
-// (k_window_tiny); classes 1-5 are k_window_sort.
+// (k_window_tiny); classes 1-5 are k_window_bits and k_window_sort.
 constexpr int kClasses = 6;
 // (Measured against 2 x 16 and 4 x 16 for the middle classes, 2 x 4 for
 // class 1 and 16 x 8 for class 4 on power-law and block-model matrices.)
@@ -69,13 +72,23 @@ constexpr int kPathAuto = 0;
 constexpr int kPathGlobal = 1;
 constexpr int kPathClass0 = 2;
 
+// Columns of some rows that decide between bitmaps and sorts.  kRowsBig: a row
+// of the global path's windows (all are checked, unless there are too many)
+// does not strictly increase.  From the first row of every other window: one
+// descends (kRowsDown), or spans more columns than the bit kernel of class 1
+// (kRowsWide1) or of the larger classes (kRowsWide) takes.
+constexpr int kRowsBig = 1, kRowsDown = 2, kRowsWide1 = 4, kRowsWide = 8;
+constexpr int kSpanLog1 = 20, kSpanLog = 21;  // log2 of those spans
+
 constexpr int kMaxSlots = 16;  // the column maximum is spread over this many words
 struct MetcfHeader {
   int32_t flags;    // CSR check bits, see kBad*
   int32_t nnz_big;  // entries of the global-path windows
   int32_t cls_count[kClasses + 1];  // windows per LDS class; [kClasses]: global-path windows
   int32_t max_col[kMaxSlots];       // largest column index: the maximum of these
-  int32_t pad[64 - 2 - (kClasses + 1) - kMaxSlots];
+  int32_t rows;                     // what is known of the rows' columns, see kRows*
+  int32_t miss[kClasses];   // windows of each class that its bit kernel left
+  int32_t pad[64 - 3 - (kClasses + 1) - kMaxSlots - kClasses];
 };
 constexpr int kHeaderRead = 128;  // bytes of the header read by the host
 static_assert(sizeof(MetcfHeader) == 256, "header size");
@@ -98,6 +111,7 @@ struct MetcfWs {
   int32_t *wU;
   int32_t *lists;           // [kClasses + 1][W] windows of each class; the last row
                             // (global path) maps compacted window -> window
+  int32_t *miss;            // [kClasses][W] windows of each class that its bit kernel left
   int32_t *bstart;          // global path: first compacted entry of each of its blocks
   int32_t *cbb;             // global path: first block of each compacted window [n_big + 1]
   int32_t *csb;             // compacted window -> first compacted entry [n_big + 1]
@@ -128,6 +142,7 @@ MetcfWs carve(void *ws, int64_t nnz, int64_t W) {
   w.dcol = c.take<int32_t>(n);
   w.wU = c.take<int32_t>(nw);
   w.lists = c.take<int32_t>((kClasses + 1) * nw);
+  w.miss = c.take<int32_t>(kClasses * nw);
   w.bstart = c.take<int32_t>(n);
   w.cbb = c.take<int32_t>(nw + 1);
   w.csb = c.take<int32_t>(nw + 1);
@@ -176,6 +191,8 @@ __global__ void k_header_init(MetcfHeader *h) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     h->flags = 0;
     h->nnz_big = 0;
+    h->rows = 0;
+    for (int c = 0; c < kClasses; ++c) h->miss[c] = 0;
     for (int c = 0; c <= kClasses; ++c) h->cls_count[c] = 0;
     for (int c = 0; c < kMaxSlots; ++c) h->max_col[c] = 0;
   }
@@ -218,7 +235,8 @@ __device__ __forceinline__ int window_end(const int32_t *rowptr, int w, int blk_
 // Also writes row_window_offset[0] = 0.
 __device__ __forceinline__ void classify_part(const int32_t *rowptr, int32_t M, int32_t W,
                                               int32_t blk_h, int mode, const int32_t *bp,
-                                              int32_t *lists, int32_t *rwo, MetcfHeader *h) {
+                                              const int32_t *col, int32_t nnz, int32_t *lists,
+                                              int32_t *rwo, MetcfHeader *h) {
   constexpr int NC = kClasses + 1;
   __shared__ int s_cnt[NC], s_base[NC], s_big;
   const int w = blockIdx.x * blockDim.x + threadIdx.x;
@@ -242,6 +260,22 @@ __device__ __forceinline__ void classify_part(const int32_t *rowptr, int32_t M, 
     } else {
       bad = bp[w] != 0;
     }
+  }
+  // A look at one row of each window: unsorted and too wide ones go to the sort
+  // at once, instead of after the bit kernel has read them.
+  int rows = 0;
+  if (cls >= 0 && cls < kClasses) {
+    const int r0 = rowptr[(int64_t)w * blk_h], r1 = rowptr[min((int64_t)w * blk_h + 1, (int64_t)M)];
+    if (r0 >= 0 && r1 - r0 >= 2 && r1 <= nnz) {
+      const int64_t d = (int64_t)col[r1 - 1] - col[r0];
+      rows = d <= 0 ? kRowsDown
+                    : cls == 1 && d >> kSpanLog1 ? kRowsWide1 : cls > 1 && d >> kSpanLog ? kRowsWide : 0;
+    }
+  }
+  if (__ballot(rows != 0)) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) rows |= __shfl_xor(rows, d, 64);
+    if (lane == 0) atomicOr(&h->rows, rows);
   }
   if (w == 0) rwo[0] = 0;
   if (__ballot(bad) && lane == 0) atomicOr(&h->flags, kBadPartition);
@@ -280,10 +314,10 @@ __device__ __forceinline__ void classify_part(const int32_t *rowptr, int32_t M, 
 __global__ __launch_bounds__(256) void k_check_classify(const int32_t *rowptr, int32_t M,
                                                         int32_t nnz, int32_t W, int32_t blk_h,
                                                         int mode, const int32_t *bp,
-                                                        int32_t *lists, int32_t *rwo,
-                                                        MetcfHeader *h) {
+                                                        const int32_t *col, int32_t *lists,
+                                                        int32_t *rwo, MetcfHeader *h) {
   validate_part(rowptr, M, nnz, h);
-  classify_part(rowptr, M, W, blk_h, mode, bp, lists, rwo, h);
+  classify_part(rowptr, M, W, blk_h, mode, bp, col, nnz, lists, rwo, h);
 }
 
 // Exclusive prefix sum by one 1,024-thread workgroup, 16 items per thread
@@ -391,7 +425,9 @@ __global__ __launch_bounds__(1024) void k_big_offsets(const int32_t *rowptr, int
 // and negative columns there, read by tiles of `tile` entries as laid out by
 // k_big_offsets; with more than kOneGroupWindows such windows (their tiles
 // are laid out after the first host read) every column is read.  One atomic
-// pair per workgroup.
+// pair per workgroup.  For 16-row windows it also finds whether every row's
+// columns strictly increase (an entry not above its predecessor must be the
+// first of its row), which decides between the bitmaps and the sort.
 __global__ __launch_bounds__(256) void k_big_maxcol(const int32_t *rowptr, const int32_t *col,
                                                     int32_t M, int32_t nnz, int32_t blk_h,
                                                     const int32_t *wmap, const int32_t *csb,
@@ -400,17 +436,27 @@ __global__ __launch_bounds__(256) void k_big_maxcol(const int32_t *rowptr, const
   const int n_big = h->cls_count[kClasses];
   if (n_big == 0) return;  // workgroup-uniform
   int mx = 0, neg = 0;
+  bool unsorted = n_big > kOneGroupWindows;
   if (n_big <= kOneGroupWindows) {
     const int tiles = tb[n_big];
     for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
       const int k = tw[t];
-      const int s = window_begin(rowptr, wmap[k], blk_h, M);
+      const int w = wmap[k];
+      const int s = window_begin(rowptr, w, blk_h, M);
       const int off = (t - tb[k]) * tile;
       const int len = min(tile, csb[k + 1] - csb[k] - off);
+#pragma unroll 4
       for (int i = threadIdx.x; i < len; i += blockDim.x) {
-        const int c = col[s + off + i];
+        const int e = s + off + i;
+        const int c = col[e], before = col[max(e - 1, s)];
         mx = max(mx, c);
         neg |= c;
+        if (before >= c && e > s && blk_h == kWinH) {
+          bool starts = false;
+#pragma unroll
+          for (int r = 1; r < kWinH; ++r) starts |= rowptr[min((int64_t)w * kWinH + r, (int64_t)M)] == e;
+          unsorted |= !starts;
+        }
       }
     }
   } else {
@@ -444,7 +490,9 @@ __global__ __launch_bounds__(256) void k_big_maxcol(const int32_t *rowptr, const
     mx = max(mx, __shfl_xor(mx, d, 64));
   }
   __shared__ int s_m[4], s_n[4];
+  const bool any_unsorted = __ballot(unsorted) != 0;
   if ((threadIdx.x & 63) == 0) {
+    if (any_unsorted) atomicOr(&h->rows, kRowsBig);
     s_m[threadIdx.x >> 6] = mx;
     s_n[threadIdx.x >> 6] = neg;
   }
@@ -567,7 +615,325 @@ constexpr int win_cnt(int waves) {
 }
 constexpr bool win_wide(int waves, int items) { return 64 * waves * items <= 4096; }
 
-// Phase 1 of the LDS path, one workgroup per window of the class list.
+// ---- windows whose rows' columns strictly increase
+//
+// LDS of the bit kernels, one stage over the other.  Ranks: a bit for every
+// 32 columns of the span that hold an entry, then, for those only, a word with
+// a bit per column, both with the number of bits set before each word.
+// Positions: the occupancy of every TC block (16 rows x 8 slots, four words).
+// Outputs in their final order, so that they leave in runs.
+template <int WAVES, int ITEMS>
+struct BitLds {
+  static constexpr int kCap = 64 * WAVES * ITEMS;
+  static constexpr int kSpanLog = WAVES == 1 ? kSpanLog1 : dtc::kSpanLog;  // widest column span
+  static constexpr int kTop = 1 << (kSpanLog - 10);          // words of the 32-column bits
+  static constexpr int kWords = kCap < 8192 ? kCap : 8192;   // words of the column bits
+  static constexpr int kStage = kCap < 8192 ? kCap : 8192;   // 4-byte outputs staged at a time
+  union {
+    struct {
+      uint4 top[kTop / 4], word[kWords / 4];
+      ushort4 top_before[kTop / 4], word_before[kWords / 4];
+    };
+    struct {
+      uint4 occ[kCap / kWinW];
+      ushort4 occ_before[kCap / kWinW];
+    };
+    struct {
+      uint16_t edge[kCap];  // local entry at every TC-block position
+      uint8_t tile[kCap];
+    };
+    uint32_t stage[kStage];
+  };
+};
+
+__device__ __forceinline__ int popc4(uint4 m) { return __popc(m.x) + __popc(m.y) + __popc(m.z) + __popc(m.w); }
+
+// Keeps what is derived from x after this point from being computed before it:
+// carried from stage to stage, it takes several registers per slot.
+__device__ __forceinline__ void fresh(uint32_t &x) { asm volatile("" : "+v"(x)); }
+
+// Set bits of word i below bit b (0 .. 31) of a bitmap with its counts.
+__device__ __forceinline__ int bits_below(const uint4 *bits, const ushort4 *before, uint32_t i,
+                                          uint32_t b) {
+  const uint32_t m = reinterpret_cast<const uint32_t *>(bits)[i];
+  return __popc(m & ((1u << b) - 1u)) + reinterpret_cast<const uint16_t *>(before)[i];
+}
+
+// before = set bits of the words before each word of bits[0 .. groups);
+// returns all of them.  emit(g, bits before group g) runs once per group.
+// Every thread of the workgroup must call it; it starts and ends with a
+// barrier.
+template <int WAVES, class Emit>
+__device__ __forceinline__ int bits_before(const uint4 *bits, ushort4 *before, int groups,
+                                           int *s_scan, Emit emit) {
+  constexpr int NT = 64 * WAVES;
+  const int tid = threadIdx.x;
+  const int per = (groups + NT - 1) / NT;  // consecutive groups per thread
+  const int g0 = min(tid * per, groups), g1 = min(g0 + per, groups);
+  __syncthreads();
+  int sum = 0;
+  for (int g = g0; g < g1; ++g) sum += popc4(bits[g]);
+  const int inc = wave_inclusive_sum(sum);
+  int run = inc - sum, total = 0;
+  if (WAVES > 1) {
+    if ((tid & 63) == 63) s_scan[tid >> 6] = inc;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) {
+      const int t = s_scan[v];
+      run += v < (tid >> 6) ? t : 0;
+      total += t;
+    }
+  } else {
+    total = __builtin_amdgcn_readlane(inc, 63);
+  }
+  for (int g = g0; g < g1; ++g) {
+    const uint4 m = bits[g];
+    emit(g, run);
+    ushort4 b;
+    b.x = (uint16_t)run;
+    run += __popc(m.x);
+    b.y = (uint16_t)run;
+    run += __popc(m.y);
+    b.z = (uint16_t)run;
+    run += __popc(m.z);
+    b.w = (uint16_t)run;
+    run += __popc(m.w);
+    before[g] = b;
+  }
+  __syncthreads();
+  return total;
+}
+
+// Phase 1 of the LDS path for windows whose rows' columns strictly increase
+// (sorted and duplicate-free: what loaders produce) within a span of
+// 2^kSpanLog columns, one workgroup per window of the class list; the others
+// are listed in `miss`.  No sort: entries stay where they are (local CSR entry
+// q with wave q / (64 ITEMS), slot (q / 64) % ITEMS, lane q % 64).
+//   ranks   LDS atomics set the bit of every 32 columns that are used; counting
+//           the bits before each of their words numbers those 32-column pieces,
+//           so that a word per piece, a bit per column, holds the window's
+//           columns in as many words as it has entries at most; a column's
+//           rank is the number of bits below its own, and the entry that set
+//           the bit lists the column;
+//   blocks  entry (row, rank) is bit row * 8 + rank % 8 of block rank / 8;
+//           rows being sorted, the CSR order inside a block (the reference's
+//           placement) is the order of those bits.
+// Bound by vector instructions and the latency between its barriers (a sort
+// takes 3 to 5 times the instructions: nine ballots a digit).  Kernel times on
+// an R-MAT matrix of 2^20 rows and 31.4 M entries, sorted before and now, for
+// windows of up to 512 / 2,048 / 4,096 / 8,192 / 16,384 entries: 95 -> 70,
+// 120 -> 55, 163 -> 66, 67 -> 21, 258 -> 90 us (the last three sorts ran beside
+// the large windows').  The 32-column pieces are what makes the cost
+// independent of the span: bitmaps of 2^18 columns taken one after another
+// measured 119, 131, 40 and 157 us for the last four.  A span of 2^20 (one wave)
+// or 2^21 columns keeps three to four workgroups' LDS on a CU.
+template <int WAVES, int ITEMS>
+__global__ __launch_bounds__(64 * WAVES, ITEMS == 16 ? 4 : 8) void k_window_bits(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t M,
+    const int32_t *__restrict__ list, const float *__restrict__ values, int32_t *__restrict__ e2r,
+    int32_t *__restrict__ e2c, int32_t *__restrict__ bp, uint8_t *__restrict__ tile,
+    float *__restrict__ tcvalues, int32_t *__restrict__ tcedge, WinStage st, MetcfHeader *h,
+    int32_t *__restrict__ miss_count, int32_t *__restrict__ miss) {
+  typedef BitLds<WAVES, ITEMS> Bits;
+  constexpr int NT = 64 * WAVES;
+  __shared__ __align__(16) Bits l;
+  __shared__ int s_unsorted;  // some row's columns do not strictly increase
+  __shared__ int s_scan[16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int vbase = __builtin_amdgcn_readfirstlane(tid >> 6) * 64 * ITEMS;
+  const int w = list[blockIdx.x];
+  // lane r: start of row r of the window (r = 16: its end), window-relative
+  int rp = rowptr[min((int64_t)w * kWinH + min(lane, kWinH), (int64_t)M)];
+  const int s = __builtin_amdgcn_readlane(rp, 0);
+  const int E = __builtin_amdgcn_readlane(rp, kWinH) - s;
+  rp -= s;
+  if (E <= 0 || E > Bits::kCap) {  // the class list guarantees 0 < E <= kCap
+    if (tid == 0) atomicOr(&h->flags, kBadClass);
+    return;
+  }
+  // key[k]: column.  ix[k]: row (high half).  Branch-free loads (clamped to the
+  // window) so that all of them are in flight together; the last ones are the
+  // column before the wave's first, and the first and last column of row `lane`.
+  const int32_t *wcol = col + s;
+  uint32_t key[ITEMS], ix[ITEMS];
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) key[k] = (uint32_t)wcol[(uint32_t)min(vbase + k * 64 + lane, E - 1)];
+  const uint32_t prev_wave = (uint32_t)wcol[min(max(vbase - 1, 0), E - 1)];
+  const int row_end = __shfl_down(rp, 1, 64);
+  const bool has = lane < kWinH && row_end > rp;
+  int cmin = has ? wcol[(uint32_t)rp] : INT32_MAX;
+  int cmax = has ? wcol[(uint32_t)(row_end - 1)] : 0;
+#pragma unroll
+  for (int d = 1; d < kWinH; d <<= 1) {
+    cmin = min(cmin, __shfl_xor(cmin, d, 64));
+    cmax = max(cmax, __shfl_xor(cmax, d, 64));
+  }
+  cmin = __builtin_amdgcn_readfirstlane(cmin);
+  cmax = __builtin_amdgcn_readfirstlane(cmax);
+  const uint32_t span = (uint32_t)(cmax - cmin);
+  const int top_groups = (int)min(span >> 12, (uint32_t)(Bits::kTop / 4 - 1)) + 1;
+  const int word_groups = (min(E, Bits::kWords) + 3) / 4;
+  const uint4 zero = make_uint4(0, 0, 0, 0);
+  if (tid == 0) s_unsorted = 0;
+  for (int g = tid; g < top_groups; g += NT) l.top[g] = zero;
+  for (int g = tid; g < word_groups; g += NT) l.word[g] = zero;
+  __syncthreads();
+  unsigned *top = reinterpret_cast<unsigned *>(l.top), *word = reinterpret_cast<unsigned *>(l.word);
+  constexpr uint32_t kSpanMask = (1u << Bits::kSpanLog) - 1u;
+  bool unsorted = false;
+  {
+    int row = 0;                                     // rows started at or before the slot, less one
+    int next = __builtin_amdgcn_readlane(rp, 1);     // start of row + 1
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      const int q = vbase + k * 64 + lane;
+      ix[k] = 0;
+      if (vbase + k * 64 < E) {  // wave-uniform
+        uint32_t before = __shfl_up(key[k], 1, 64);
+        if (lane == 0)
+          before = k > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)key[k > 0 ? k - 1 : 0], 63) : prev_wave;
+        bool starts = q == 0;
+        int r = row;
+        while (row < kWinH - 1 && next < vbase + k * 64 + 64) {  // wave-uniform
+          r += q >= next;
+          starts |= q == next;
+          ++row;
+          next = __builtin_amdgcn_readlane(rp, row + 1);
+        }
+        ix[k] = (uint32_t)r << 16;
+        if (q < E) {
+          (e2r + s)[(uint32_t)q] = w * kWinH + r;
+          unsorted |= !starts && (int)key[k] <= (int)before;  // (signed: a negative column too)
+        }
+      }
+      // (a clamped slot repeats the window's last entry, and so do its bits)
+      key[k] = (key[k] - (uint32_t)cmin) & kSpanMask;
+      if (vbase + k * 64 < E) {
+        const uint32_t p = min(key[k] >> 5, (uint32_t)top_groups * 128u - 1u);
+        atomicOr(&top[p >> 5], 1u << (p & 31));
+      }
+    }
+  }
+  if (__ballot(unsorted) != 0 && lane == 0) s_unsorted = 1;
+  if (tid == 0 && cmin < 0) atomicOr(&h->flags, kBadColumn);  // reported after phase 1
+  const int pieces = bits_before<WAVES>(l.top, l.top_before, top_groups, s_scan, [](int, int) {});
+  if (s_unsorted || span > kSpanMask || pieces > Bits::kWords) {  // workgroup-uniform
+    if (tid == 0) {
+      miss[atomicAdd(miss_count, 1)] = w;
+      bp[w] = 0;  // until then
+    }
+    return;
+  }
+  uint32_t lists = 0;  // slots whose entry set its column's bit
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    fresh(key[k]);
+    if (vbase + k * 64 + lane < E) {
+      const uint32_t p = (uint32_t)bits_below(l.top, l.top_before, key[k] >> 10, (key[k] >> 5) & 31);
+      const uint32_t bit = 1u << (key[k] & 31);
+      ix[k] |= p;
+      lists |= (atomicOr(&word[p], bit) & bit) ? 0u : 1u << k;
+    }
+    if (k % 4 == 3) asm volatile("" ::: "memory");  // four slots' LDS reads in flight, not all
+  }
+  const int U = bits_before<WAVES>(l.word, l.word_before, (pieces + 3) / 4, s_scan, [](int, int) {});
+  const int nb = (U + kWinW - 1) / kWinW;
+  if (tid == 0) {
+    bp[w] = nb;
+    st.wU[w] = U;
+  }
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int q = vbase + k * 64 + lane;
+    fresh(key[k]);
+    fresh(ix[k]);
+    if (q < E) {
+      const int rank = bits_below(l.word, l.word_before, ix[k] & 0xffffu, key[k] & 31);
+      ix[k] = (ix[k] & 0xffff0000u) | (uint32_t)rank;
+      (e2c + s)[(uint32_t)q] = rank;
+    }
+    if (k % 4 == 3) asm volatile("" ::: "memory");
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int r0 = 0; r0 < U; r0 += Bits::kStage) {
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      fresh(ix[k]);
+      const uint32_t r = (ix[k] & 0xffffu) - (uint32_t)r0;
+      if (((lists >> k) & 1u) && r < (uint32_t)Bits::kStage) l.stage[r] = key[k];
+    }
+    __syncthreads();
+    for (int r = tid; r < min(Bits::kStage, U - r0); r += NT)
+      st.dcol[s + r0 + r] = cmin + (int)l.stage[r];
+    __syncthreads();
+  }
+  // the values, branch-free (one latency for all slots), into the keys' place
+  if (tcvalues && values) {
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k)
+      key[k] = __float_as_uint((values + s)[(uint32_t)min(vbase + k * 64 + lane, E - 1)]);
+  }
+  unsigned *occ = reinterpret_cast<unsigned *>(l.occ);
+  for (int g = tid; g < nb; g += NT) l.occ[g] = zero;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    fresh(ix[k]);
+    if (vbase + k * 64 + lane < E) {
+      const uint32_t r = ix[k] >> 16, rank = ix[k] & 0xffffu;
+      atomicOr(&occ[rank / kWinW * 4 + r / 4], 1u << (r % 4 * kWinW + rank % kWinW));
+    }
+  }
+  bits_before<WAVES>(l.occ, l.occ_before, nb, s_scan, [&](int g, int run) { st.boff[s + g] = run; });
+  // ix: TC-block position (low half) and tile id
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    fresh(ix[k]);
+    if (vbase + k * 64 + lane < E) {
+      const uint32_t r = ix[k] >> 16, rank = ix[k] & 0xffffu;
+      ix[k] = (uint32_t)bits_below(l.occ, l.occ_before, rank / kWinW * 4 + r / 4,
+                                   r % 4 * kWinW + rank % kWinW) |
+              (r * kWinW + rank % kWinW) << 16;
+    }
+    if (k % 4 == 3) asm volatile("" ::: "memory");
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int q = vbase + k * 64 + lane;
+    fresh(ix[k]);
+    if (q < E) {
+      l.edge[ix[k] & 0xffffu] = (uint16_t)q;
+      l.tile[ix[k] & 0xffffu] = (uint8_t)(ix[k] >> 16);
+    }
+  }
+  __syncthreads();
+  for (int p = tid; p < E; p += NT) {
+    tile[s + p] = l.tile[p];
+    if (tcedge) tcedge[s + p] = s + l.edge[p];
+    if (tcvalues && !values) tcvalues[s + p] = 1.0f;
+  }
+  if (!tcvalues || !values) return;
+#pragma unroll 1
+  for (int p0 = 0; p0 < E; p0 += Bits::kStage) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      fresh(ix[k]);
+      const uint32_t p = (ix[k] & 0xffffu) - (uint32_t)p0;
+      if (vbase + k * 64 + lane < E && p < (uint32_t)Bits::kStage) l.stage[p] = key[k];
+    }
+    __syncthreads();
+    for (int p = tid; p < min(Bits::kStage, E - p0); p += NT)
+      tcvalues[s + p0 + p] = __uint_as_float(l.stage[p]);
+  }
+}
+
+// Phase 1 of the LDS path for any columns, one workgroup per window of the
+// list: the windows that the bit kernels leave, and every window of a class
+// whose columns may span more than they take.
 // Local CSR entry q is held by wave q / (64 ITEMS), slot (q / 64) % ITEMS,
 // lane q % 64; after the sort the same layout holds sorted position p.
 //   sort   LSD radix sort of (column - window minimum, q) over the window's
@@ -1209,6 +1575,293 @@ __global__ __launch_bounds__(256) void k_big_keys(const int32_t *rowptr, const i
   }
 }
 
+// ---- global-path windows whose rows' columns strictly increase
+//
+// The same numbering without a sort (16 x 8 windows): three kernels over
+// pieces of windows.  Rows are sorted, so a piece given by two columns is one
+// range of every row, found by a 17-way search (rows in parallel, four rounds
+// of loads for 80,000 entries), and a piece never shares a bitmap with another
+// workgroup.
+//   k_slice_mark   a slice of 2^16 columns: its column bits in LDS, kept in
+//                  the workspace with their count and the slice's row ranges;
+//   k_slice_rank   the same slice, its first rank known from the counts: every
+//                  entry's rank (the set bits below its own), the distinct
+//                  columns;
+//   k_run_out      a run of 256 TC blocks: the blocks' occupancies in LDS,
+//                  the entries' places in TC-block order, the outputs.
+// 6.1 M entries in 137 windows of an R-MAT matrix of 2^20 rows: 61 + 76 + 95 us
+// alone, where keys, three passes of the segmented sort, its scan and the
+// passes after it took 760 us.  Bound by the latency of short pieces: a slice of
+// 2^16 columns holds 2,800 of these entries, a run 2,600.
+constexpr int kSliceLog = 16;                       // columns of a slice
+constexpr int kSpanGroups = 1 << (kSliceLog - 7);    // 128-bit groups of it
+constexpr int kSpanThreads = 512;                   // one group per thread
+constexpr int kRunBlocks = 256;                     // TC blocks of a run, one per thread
+constexpr int kRunStage = 8192;                     // entries staged at a time
+static_assert(kSpanGroups == kSpanThreads, "one group per thread");
+
+// Workspace of the three kernels (over the sort's buffers).
+struct SpanWs {
+  uint4 *bits;     // [n_big][slices][kSpanGroups]
+  int32_t *count;  // [n_big][slices] distinct columns
+  int32_t *lo;     // [n_big][slices][kWinH] first entry of each row in the slice
+  int32_t slices;
+};
+
+// Set bits of m below bit b (0 .. 127).
+__device__ __forceinline__ int popc_below(uint4 m, int b) {
+  const uint32_t below = (1u << (b & 31)) - 1u;
+  const int wi = b >> 5;
+  int n = __popc((wi == 0 ? m.x : wi == 1 ? m.y : wi == 2 ? m.z : m.w) & below);
+  n += wi > 0 ? __popc(m.x) : 0;
+  n += wi > 1 ? __popc(m.y) : 0;
+  n += wi > 2 ? __popc(m.z) : 0;
+  return n;
+}
+
+// The first entry in [lo, hi) with col >= key, found by the 16 lanes of a
+// group of consecutive lanes: 16 probes cut the range into 17 parts.
+__device__ __forceinline__ int group_lower_bound(const int32_t *__restrict__ col, int lo, int hi,
+                                                 int64_t key) {
+  const int l = threadIdx.x & 15, shift = threadIdx.x & 48;
+  while (__ballot(lo < hi)) {  // wave-uniform
+    const int stride = (hi - lo) / 17 + 1;
+    const int64_t p = lo + (int64_t)(l + 1) * stride - 1;
+    const bool below = p < hi && col[p] < key;
+    const int n = __popcll((__ballot(below) >> shift) & 0xffffull);
+    // (probe n is past the range or not below the key)
+    const int64_t end = lo + (int64_t)(n + 1) * stride - 1;
+    lo += n * stride;
+    hi = n < 16 ? (int)min((int64_t)hi, end) : hi;
+  }
+  return lo;
+}
+
+// s_from[r]: first entry of row r in the piece; s_pre[r]: entries of the
+// piece in rows before r (s_pre[16]: all).  The first 16 threads call it.
+__device__ __forceinline__ void row_ranges(int *s_from, int *s_pre, int r, int lo, int hi) {
+  s_from[r] = lo;
+  int inc = max(hi - lo, 0);
+#pragma unroll
+  for (int d = 1; d < kWinH; d <<= 1) {
+    const int t = __shfl_up(inc, d, kWinH);
+    if (r >= d) inc += t;
+  }
+  if (r == 0) s_pre[0] = 0;
+  s_pre[r + 1] = inc;
+}
+
+// One workgroup per slice of a window (grid: windows x slices).
+__global__ __launch_bounds__(kSpanThreads) void k_slice_mark(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t M,
+    const int32_t *__restrict__ wmap, SpanWs sw) {
+  __shared__ uint4 s_bits[kSpanGroups];
+  __shared__ int s_lo[2 * kWinH], s_from[kWinH], s_pre[kWinH + 1], s_sum[kSpanThreads / 64];
+  const int tid = threadIdx.x;
+  const int wp = blockIdx.x / sw.slices, sl = blockIdx.x % sw.slices;
+  const int w = wmap[wp];
+  s_bits[tid] = make_uint4(0, 0, 0, 0);
+  {
+    const int g = tid >> 4;  // 32 groups: 16 rows at the slice's first column and at its end
+    const int64_t row = (int64_t)w * kWinH + (g & 15);
+    const int r0 = rowptr[min(row, (int64_t)M)], r1 = rowptr[min(row + 1, (int64_t)M)];
+    const int p = group_lower_bound(col, r0, r1, (int64_t)(sl + (g >> 4)) << kSliceLog);
+    if ((tid & 15) == 0) s_lo[g] = p;
+  }
+  __syncthreads();
+  if (tid < kWinH) {
+    row_ranges(s_from, s_pre, tid, s_lo[tid], s_lo[kWinH + tid]);
+    sw.lo[(int64_t)blockIdx.x * kWinH + tid] = s_lo[tid];
+  }
+  __syncthreads();
+  unsigned *words = reinterpret_cast<unsigned *>(s_bits);
+  const int n = s_pre[kWinH];
+#pragma unroll 4
+  for (int f = tid; f < n; f += kSpanThreads) {
+    const int r = row_of(s_pre, f);
+    const uint32_t c = (uint32_t)col[s_from[r] + f - s_pre[r]] & ((1u << kSliceLog) - 1);
+    atomicOr(&words[c >> 5], 1u << (c & 31));
+  }
+  __syncthreads();
+  const uint4 m = s_bits[tid];
+  sw.bits[(int64_t)blockIdx.x * kSpanGroups + tid] = m;
+  const int sum = wave_sum(popc4(m));
+  if ((tid & 63) == 0) s_sum[tid >> 6] = sum;
+  __syncthreads();
+  if (tid == 0) {
+    int total = 0;
+#pragma unroll
+    for (int v = 0; v < kSpanThreads / 64; ++v) total += s_sum[v];
+    sw.count[blockIdx.x] = total;
+  }
+}
+
+// One workgroup per slice again.
+__global__ __launch_bounds__(kSpanThreads) void k_slice_rank(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t M,
+    const int32_t *__restrict__ wmap, SpanWs sw, int32_t *__restrict__ e2r,
+    int32_t *__restrict__ e2c, int32_t *__restrict__ bp, WinStage st) {
+  __shared__ uint4 s_bits[kSpanGroups];
+  __shared__ int s_before[kSpanGroups];
+  __shared__ int s_from[kWinH], s_pre[kWinH + 1], s_sum[kSpanThreads / 64], s_base[kSpanThreads / 64];
+  const int tid = threadIdx.x;
+  const int wp = blockIdx.x / sw.slices, sl = blockIdx.x % sw.slices;
+  const int w = wmap[wp];
+  const uint4 m = sw.bits[(int64_t)blockIdx.x * kSpanGroups + tid];
+  s_bits[tid] = m;
+  int first = 0;  // distinct columns of the slices before this one
+  for (int k = tid; k < sl; k += kSpanThreads) first += sw.count[(int64_t)wp * sw.slices + k];
+  if (tid < kWinH) {
+    const int64_t at = (int64_t)blockIdx.x * kWinH + tid;
+    const int hi = sl + 1 < sw.slices ? sw.lo[at + kWinH]
+                                      : rowptr[min((int64_t)w * kWinH + tid + 1, (int64_t)M)];
+    row_ranges(s_from, s_pre, tid, sw.lo[at], hi);
+  }
+  const int inc = wave_inclusive_sum(popc4(m));
+  const int base_sum = wave_sum(first);
+  if ((tid & 63) == 63) s_sum[tid >> 6] = inc;
+  if ((tid & 63) == 0) s_base[tid >> 6] = base_sum;
+  __syncthreads();
+  int run = inc - popc4(m), base = 0, total = 0;
+#pragma unroll
+  for (int v = 0; v < kSpanThreads / 64; ++v) {
+    run += v < (tid >> 6) ? s_sum[v] : 0;
+    total += s_sum[v];
+    base += s_base[v];
+  }
+  run += base;  // rank of the group's first column
+  s_before[tid] = run;
+  const int s = rowptr[(int64_t)w * kWinH];
+  {
+    int32_t *d = st.dcol + s + run;
+    const int c0 = (int)(((int64_t)sl << kSliceLog) + tid * 128);
+    auto list = [&](uint32_t bits, int c) {
+      for (; bits; bits &= bits - 1) *d++ = c + (int)__builtin_ctz(bits);
+    };
+    list(m.x, c0);
+    list(m.y, c0 + 32);
+    list(m.z, c0 + 64);
+    list(m.w, c0 + 96);
+  }
+  if (sl + 1 == sw.slices && tid == 0) {
+    bp[w] = (base + total + kWinW - 1) / kWinW;
+    st.wU[w] = base + total;
+  }
+  __syncthreads();
+  const int n = s_pre[kWinH];
+#pragma unroll 4
+  for (int f = tid; f < n; f += kSpanThreads) {
+    const int r = row_of(s_pre, f);
+    const int e = s_from[r] + f - s_pre[r];
+    const uint32_t c = (uint32_t)col[e] & ((1u << kSliceLog) - 1);
+    e2r[e] = w * kWinH + r;
+    e2c[e] = s_before[c >> 7] + popc_below(s_bits[c >> 7], (int)(c & 127));
+  }
+}
+
+// One workgroup per run of kRunBlocks TC blocks; a window of E entries has a
+// run for every kWinW * kRunBlocks of them, as many as it can fill (grid: the
+// sort tiles x runs per tile).  An entry (row, rank) is bit row * 8 + rank % 8
+// of its block, and the CSR order inside a block (the reference's placement)
+// is the order of those bits.  The outputs are staged so that they leave in
+// order; a run's entries of up to kRunStage (its usual number is 2,000 to
+// 4,000, its largest 32,768) take one turn of that.
+__global__ __launch_bounds__(kRunBlocks) void k_run_out(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t M,
+    const int32_t *__restrict__ wmap, const int32_t *__restrict__ tb,
+    const int32_t *__restrict__ tw, int32_t n_big, int32_t runs_per_tile,
+    const float *__restrict__ values, const int32_t *__restrict__ e2c, WinStage st,
+    uint8_t *__restrict__ tile, float *__restrict__ tcvalues, int32_t *__restrict__ tcedge) {
+  __shared__ uint4 s_occ[kRunBlocks];
+  __shared__ int s_before[kRunBlocks];
+  __shared__ int s_lo[2 * kWinH], s_from[kWinH], s_pre[kWinH + 1], s_sum[kRunBlocks / 64];
+  __shared__ int s_start;  // the run's first TC-block position, window-relative
+  __shared__ uint16_t s_f[kRunStage];
+  __shared__ uint8_t s_tile[kRunStage];
+  const int tid = threadIdx.x;
+  const int t = blockIdx.x / runs_per_tile;
+  if (t >= tb[n_big]) return;  // workgroup-uniform
+  const int wp = tw[t];
+  const int w = wmap[wp];
+  const int U = st.wU[w];
+  const int nb = (U + kWinW - 1) / kWinW;
+  const int64_t kb64 = ((int64_t)(t - tb[wp]) * runs_per_tile + blockIdx.x % runs_per_tile) * kRunBlocks;
+  if (kb64 >= nb) return;  // workgroup-uniform
+  const int kb0 = (int)kb64, kb1 = min(kb0 + kRunBlocks, nb);
+  const int s = rowptr[(int64_t)w * kWinH];
+  s_occ[tid] = make_uint4(0, 0, 0, 0);
+  const bool last = kb1 == nb;
+  const int c0 = st.dcol[s + kb0 * kWinW];
+  const int64_t c1 = last ? (int64_t)1 << 32 : st.dcol[s + kb1 * kWinW];
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {  // 16 rows at the run's first column, then at its end
+    const int64_t row = (int64_t)w * kWinH + (tid >> 4);
+    const int r0 = rowptr[min(row, (int64_t)M)], r1 = rowptr[min(row + 1, (int64_t)M)];
+    const int p = group_lower_bound(col, r0, half && last ? r0 : r1, half ? c1 : c0);
+    if ((tid & 15) == 0) s_lo[half * kWinH + (tid >> 4)] = half && last ? r1 : p;
+  }
+  __syncthreads();
+  if (tid < kWinH) {
+    row_ranges(s_from, s_pre, tid, s_lo[tid], s_lo[kWinH + tid]);
+    int before = s_lo[tid] - rowptr[min((int64_t)w * kWinH + tid, (int64_t)M)];
+#pragma unroll
+    for (int d = 1; d < kWinH; d <<= 1) before += __shfl_xor(before, d, kWinH);
+    if (tid == 0) s_start = before;
+  }
+  __syncthreads();
+  const int n = s_pre[kWinH];
+  const uint32_t rank0 = (uint32_t)kb0 * kWinW;
+  constexpr uint32_t kRankMask = kRunBlocks * kWinW - 1;  // ranks of the run, less rank0
+  unsigned *words = reinterpret_cast<unsigned *>(s_occ);
+#pragma unroll 4
+  for (int f = tid; f < n; f += kRunBlocks) {
+    const int r = row_of(s_pre, f);
+    const uint32_t k = ((uint32_t)e2c[s_from[r] + f - s_pre[r]] - rank0) & kRankMask;
+    const uint32_t bit = (uint32_t)r * kWinW + k % kWinW;
+    atomicOr(&words[k / kWinW * 4 + (bit >> 5)], 1u << (bit & 31));
+  }
+  __syncthreads();
+  {
+    const int sum = popc4(s_occ[tid]);
+    const int inc = wave_inclusive_sum(sum);
+    if ((tid & 63) == 63) s_sum[tid >> 6] = inc;
+    __syncthreads();
+    int run = inc - sum;
+#pragma unroll
+    for (int v = 0; v < kRunBlocks / 64; ++v) run += v < (tid >> 6) ? s_sum[v] : 0;
+    s_before[tid] = run;
+    if (kb0 + tid < kb1) st.boff[s + kb0 + tid] = s_start + run;
+  }
+  __syncthreads();
+  const int64_t out = (int64_t)s + s_start;
+  for (int p0 = 0; p0 < n; p0 += kRunStage) {
+#pragma unroll 4
+    for (int f = tid; f < n; f += kRunBlocks) {
+      const int r = row_of(s_pre, f);
+      const uint32_t k = ((uint32_t)e2c[s_from[r] + f - s_pre[r]] - rank0) & kRankMask;
+      const uint32_t bit = (uint32_t)r * kWinW + k % kWinW;
+      const uint32_t p = (uint32_t)(s_before[k / kWinW] + popc_below(s_occ[k / kWinW], (int)bit) - p0);
+      if (p < kRunStage) {
+        s_f[p] = (uint16_t)f;
+        s_tile[p] = (uint8_t)bit;
+      }
+    }
+    __syncthreads();
+    const int len = min(n - p0, kRunStage);
+#pragma unroll 4
+    for (int p = tid; p < len; p += kRunBlocks) {
+      const int f = s_f[p];
+      const int r = s_tile[p] / kWinW;
+      const int e = s_from[r] + f - s_pre[r];
+      const int64_t dst = out + p0 + p;
+      tile[dst] = s_tile[p];
+      if (tcvalues) tcvalues[dst] = values ? values[e] : 1.0f;
+      if (tcedge) tcedge[dst] = e;
+    }
+    __syncthreads();
+  }
+}
+
 struct BigView {
   const uint32_t *keys32;  // segmented sort
   const uint64_t *keys64;  // sort of the whole range
@@ -1410,17 +2063,57 @@ dtc_status_t side_stream(SideStream **out) {
   return DTC_SUCCESS;
 }
 
+// What the window kernels of one build read and write.
+struct WindowArgs {
+  const int32_t *rowptr, *col;
+  int32_t M;
+  const float *values;
+  int32_t *e2r, *e2c, *bp;
+  uint8_t *tile;
+  float *tcvalues;
+  int32_t *tcedge;
+  MetcfWs ws;
+  int64_t W;
+};
+
+// The windows of class C from its list: without a sort (`bits`), or sorted;
+// or the ones that the bit kernel left, sorted (`missed`).
 template <int C>
-dtc_status_t launch_window_sort(const int32_t *rowptr, const int32_t *col, int32_t M, int count,
-                                const MetcfWs &ws, int64_t W, const float *values, int32_t *e2r,
-                                int32_t *e2c, int32_t *bp, uint8_t *tile, float *tcvalues,
-                                int32_t *tcedge, hipStream_t stream) {
-  if (count <= 0) return DTC_SUCCESS;
-  k_window_sort<kClassWaves[C], kClassItems[C]><<<(unsigned)count, 64 * kClassWaves[C], 0, stream>>>(
-      rowptr, col, M, ws.lists + (int64_t)C * W, values, e2r, e2c, bp, tile, tcvalues, tcedge,
-      win_stage(ws), ws.hdr);
-  DTC_LAUNCH_CHECK("window_sort");
+dtc_status_t launch_windows(const WindowArgs &a, int count, bool bits, bool missed,
+                            hipStream_t stream) {
+  constexpr int NT = 64 * kClassWaves[C];
+  const int32_t *list = a.ws.lists + (int64_t)C * a.W;
+  int32_t *miss = a.ws.miss + (int64_t)C * a.W;
+  if (bits)
+    k_window_bits<kClassWaves[C], kClassItems[C]><<<(unsigned)count, NT, 0, stream>>>(
+        a.rowptr, a.col, a.M, list, a.values, a.e2r, a.e2c, a.bp, a.tile, a.tcvalues, a.tcedge,
+        win_stage(a.ws), a.ws.hdr, &a.ws.hdr->miss[C], miss);
+  else
+    k_window_sort<kClassWaves[C], kClassItems[C]><<<(unsigned)count, NT, 0, stream>>>(
+        a.rowptr, a.col, a.M, missed ? miss : list, a.values, a.e2r, a.e2c, a.bp, a.tile,
+        a.tcvalues, a.tcedge, win_stage(a.ws), a.ws.hdr);
+  DTC_LAUNCH_CHECK(bits ? "window_bits" : "window_sort");
   return DTC_SUCCESS;
+}
+
+// Without a sort, unless the rows looked at need one.
+dtc_status_t launch_class(int c, const WindowArgs &a, int count, int rows, bool missed,
+                          hipStream_t stream) {
+  if (count <= 0) return DTC_SUCCESS;
+  const bool bits = !missed && !(rows & (kRowsDown | (c == 1 ? kRowsWide1 : kRowsWide)));
+  switch (c) {
+    case 0:
+      k_window_tiny<<<grid_for(count, 4), 256, 0, stream>>>(
+          a.rowptr, a.col, a.M, a.ws.lists, count, a.values, a.e2r, a.e2c, a.bp, a.tile,
+          a.tcvalues, a.tcedge, win_stage(a.ws), a.ws.hdr);
+      DTC_LAUNCH_CHECK("window_tiny");
+      return DTC_SUCCESS;
+    case 1: return launch_windows<1>(a, count, bits, missed, stream);
+    case 2: return launch_windows<2>(a, count, bits, missed, stream);
+    case 3: return launch_windows<3>(a, count, bits, missed, stream);
+    case 4: return launch_windows<4>(a, count, bits, missed, stream);
+    default: return launch_windows<5>(a, count, bits, missed, stream);
+  }
 }
 
 }  // namespace
@@ -1476,7 +2169,7 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
     const unsigned grid = (unsigned)std::max<int64_t>(
         std::min<int64_t>(1024, grid_for(num_nodes, 256)), grid_for(W, 256));
     k_check_classify<<<grid, 256, 0, stream>>>(node_pointer, num_nodes, nnz, (int32_t)W, blk_h,
-                                               mode, block_partition, ws.lists,
+                                               mode, block_partition, edge_list, ws.lists,
                                                row_window_offset, ws.hdr);
     DTC_LAUNCH_CHECK("check_classify");
   }
@@ -1571,8 +2264,33 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
     DTC_LAUNCH_CHECK("big_tilemap");
   }
 
+  // Windows of strictly increasing rows: column bitmaps instead of the sort,
+  // when they fit the sort's key buffers (a bit per column of the matrix and
+  // window, at most 16 bytes per entry).
+  const int64_t slices = (max_col >> kSliceLog) + 1;
+  const int64_t pieces = n_big * slices;
+  const bool bitmaps = nnz_big > 0 && blk_h == kWinH && blk_w == kWinW && !(host.rows & kRowsBig) &&
+                       pieces * kSpanGroups <= nnz_big && pieces <= INT32_MAX;
   const bool segmented = n_big > 0 && nnz_big / n_big >= seg_radix_tile_size();
-  if (nnz_big > 0 && segmented) {
+  if (bitmaps) {
+    SpanWs sw;
+    sw.bits = reinterpret_cast<uint4 *>(ws.keys0);
+    sw.count = ws.vals0;
+    sw.lo = ws.vals1;
+    sw.slices = (int32_t)slices;
+    k_slice_mark<<<(unsigned)pieces, kSpanThreads, 0, gs>>>(node_pointer, edge_list, num_nodes,
+                                                            wmap, sw);
+    DTC_LAUNCH_CHECK("slice_mark");
+    k_slice_rank<<<(unsigned)pieces, kSpanThreads, 0, gs>>>(node_pointer, edge_list, num_nodes,
+                                                            wmap, sw, edge_to_row, edge_to_column,
+                                                            block_partition, win_stage(ws));
+    DTC_LAUNCH_CHECK("slice_rank");
+    const int64_t tile = seg_radix_tile_size(), per = ceil_div(tile, kRunBlocks * kWinW);
+    k_run_out<<<(unsigned)((ceil_div(nnz_big, tile) + n_big) * per), kRunBlocks, 0, gs>>>(
+        node_pointer, edge_list, num_nodes, wmap, ws.tb, ws.tw, n_big, (int32_t)per, values,
+        edge_to_column, win_stage(ws), tcblocktile_id, tcblock_values, tcblock_edge);
+    DTC_LAUNCH_CHECK("run_out");
+  } else if (nnz_big > 0 && segmented) {
     k_big_keys<uint32_t><<<grid_for(nnz_big, kBigChunk), 256, 0, gs>>>(
         node_pointer, edge_list, num_nodes, blk_h, colbits, n_big, nnz_big, wmap, ws.csb,
         edge_to_row, ws.k32_0, ws.vals0, ws.wpos);
@@ -1587,38 +2305,23 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
   // 4. LDS path (every output of the window sized by its entries, and its
   //    block data for phase 2): the largest class now, the others after the
   //    global path's launches.
-  auto launch_class = [&](int c) -> dtc_status_t {
-    const int n = host.cls_count[c];
-    if (n <= 0) return DTC_SUCCESS;
-    switch (c) {
-      case 0:
-        k_window_tiny<<<grid_for(n, 4), 256, 0, stream>>>(
-            node_pointer, edge_list, num_nodes, ws.lists, n, values, edge_to_row,
-            edge_to_column, block_partition, tcblocktile_id, tcblock_values, tcblock_edge,
-            win_stage(ws), ws.hdr);
-        DTC_LAUNCH_CHECK("window_tiny");
-        return DTC_SUCCESS;
-      case 5: return launch_window_sort<5>(node_pointer, edge_list, num_nodes, n, ws, W, values, edge_to_row, edge_to_column, block_partition, tcblocktile_id, tcblock_values, tcblock_edge, stream);
-      case 4: return launch_window_sort<4>(node_pointer, edge_list, num_nodes, n, ws, W, values, edge_to_row, edge_to_column, block_partition, tcblocktile_id, tcblock_values, tcblock_edge, stream);
-      case 3: return launch_window_sort<3>(node_pointer, edge_list, num_nodes, n, ws, W, values, edge_to_row, edge_to_column, block_partition, tcblocktile_id, tcblock_values, tcblock_edge, stream);
-      case 2: return launch_window_sort<2>(node_pointer, edge_list, num_nodes, n, ws, W, values, edge_to_row, edge_to_column, block_partition, tcblocktile_id, tcblock_values, tcblock_edge, stream);
-      default: return launch_window_sort<1>(node_pointer, edge_list, num_nodes, n, ws, W, values, edge_to_row, edge_to_column, block_partition, tcblocktile_id, tcblock_values, tcblock_edge, stream);
-    }
-  };
+  const WindowArgs args = {node_pointer,    edge_list,      num_nodes,       values,
+                           edge_to_row,     edge_to_column, block_partition, tcblocktile_id,
+                           tcblock_values,  tcblock_edge,   ws,              W};
   // The two largest classes now (a few hundred µs of work queued on the
   // caller's stream while the host issues the global path), the third after
   // the sort, the rest after the global path.
   bool issued[kClasses] = {};
   auto issue = [&](int c) -> dtc_status_t {
     issued[c] = true;
-    return launch_class(c);
+    return launch_class(c, args, host.cls_count[c], host.rows, false, stream);
   };
   st = issue(kClasses - 1);
   if (st == DTC_SUCCESS) st = issue(kClasses - 2);
   if (st != DTC_SUCCESS) return st;
   // 5. Global path, continued: sort, unique-column numbering;
   //    blockPartition, edgeToColumn, block data, tile ids; then join.
-  if (nnz_big > 0) {
+  if (nnz_big > 0 && !bitmaps) {
     bool in_1 = false;
     BigView bv;
     if (segmented) {
@@ -1678,24 +2381,35 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
     side_lock.unlock();
   }
 
-  // 7. Window offsets (row_window_offset[0] was written by k_check_classify).
-  st = scan_i32(block_partition, row_window_offset + 1, W, true, ws.tmp, stream);
-  if (st != DTC_SUCCESS) return st;
-  k_chunk_windows<<<grid_for(W, 256), 256, 0, stream>>>(row_window_offset, (int32_t)W, ws.cw,
-                                                         ws.cw + ws.cw_stride);
-  DTC_LAUNCH_CHECK("chunk_windows");
-
-  // 8. Block count (second host synchronisation).
+  // 7. Window offsets (row_window_offset[0] was written by k_check_classify)
+  //    and block count (second host synchronisation); then once more if the
+  //    bit kernels left windows to the sort.
   int32_t T = 0;
-  {
-    std::lock_guard<std::mutex> g(dev_state->read_mu);
-    DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned, ws.hdr, kHeaderRead, hipMemcpyDeviceToHost,
-                                 stream));
-    DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned + kHeaderRead, row_window_offset + W,
-                                 sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-    DTC_HIP_CHECK(hipStreamSynchronize(stream));
-    std::memcpy(&host, dev_state->pinned, kHeaderRead);
-    std::memcpy(&T, dev_state->pinned + kHeaderRead, sizeof(int32_t));
+  bool missed = false;
+  for (bool again = true; again;) {
+    st = scan_i32(block_partition, row_window_offset + 1, W, true, ws.tmp, stream);
+    if (st != DTC_SUCCESS) return st;
+    k_chunk_windows<<<grid_for(W, 256), 256, 0, stream>>>(row_window_offset, (int32_t)W, ws.cw,
+                                                           ws.cw + ws.cw_stride);
+    DTC_LAUNCH_CHECK("chunk_windows");
+    {
+      std::lock_guard<std::mutex> g(dev_state->read_mu);
+      DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned, ws.hdr, kHeaderRead, hipMemcpyDeviceToHost,
+                                   stream));
+      DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned + kHeaderRead, row_window_offset + W,
+                                   sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+      DTC_HIP_CHECK(hipStreamSynchronize(stream));
+      std::memcpy(&host, dev_state->pinned, kHeaderRead);
+      std::memcpy(&T, dev_state->pinned + kHeaderRead, sizeof(int32_t));
+    }
+    again = false;
+    for (int c = 1; c < kClasses && !(host.flags & (kBadColumn | kBadClass)); ++c) {
+      if (missed || host.miss[c] <= 0) continue;
+      again = true;
+      st = launch_class(c, args, host.miss[c], host.rows, true, stream);
+      if (st != DTC_SUCCESS) return st;
+    }
+    missed = true;
   }
   if (host.flags & kBadColumn)  // found by the window kernels
     return fail(DTC_ERROR_INVALID_CSR, "invalid CSR: negative column index;");

@@ -38,9 +38,11 @@ class DTCMatrix:
             self.values = torch.as_tensor(values, dtype=torch.float32).to(self.device).contiguous()
         W = (self.num_rows + BLK_H - 1) // BLK_H
         self.num_windows = W
+        # The build writes every edge; block_partition of empty windows it only
+        # checks for zero.
         self.block_partition = torch.zeros(W, dtype=torch.int32, device=self.device)
-        self.edge_to_column = torch.zeros(self.nnz, dtype=torch.int32, device=self.device)
-        self.edge_to_row = torch.zeros(self.nnz, dtype=torch.int32, device=self.device)
+        self.edge_to_column = torch.empty(self.nnz, dtype=torch.int32, device=self.device)
+        self.edge_to_row = torch.empty(self.nnz, dtype=torch.int32, device=self.device)
         # the values are reordered into TC-block order by the build itself (the
         # tile-id pass), not by a separate gather over tc_edge
         out = ext.preprocess_gpu(self.col, self.rowptr, self.num_rows, BLK_H, BLK_W,
