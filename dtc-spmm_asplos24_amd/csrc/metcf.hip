@@ -729,7 +729,7 @@ __device__ __forceinline__ int bits_before(const uint4 *bits, ushort4 *before, i
 // measured 119, 131, 40 and 157 us for the last four.  A span of 2^20 (one wave)
 // or 2^21 columns keeps three to four workgroups' LDS on a CU.
 template <int WAVES, int ITEMS>
-__global__ __launch_bounds__(64 * WAVES, ITEMS == 16 ? 4 : 8) void k_window_bits(
+__global__ __launch_bounds__(64 * WAVES, ITEMS == 16 ? 4 : 6) void k_window_bits(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t M,
     const int32_t *__restrict__ list, const float *__restrict__ values, int32_t *__restrict__ e2r,
     int32_t *__restrict__ e2c, int32_t *__restrict__ bp, uint8_t *__restrict__ tile,
