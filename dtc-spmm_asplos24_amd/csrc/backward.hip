@@ -15,76 +15,6 @@
 namespace dtc {
 namespace {
 
-struct TransposeWs {
-  int32_t *flags;
-  uint64_t *keys0, *keys1;
-  int32_t *vals0, *vals1;
-  int32_t *e2r;
-  void *tmp;
-  size_t bytes;
-};
-
-TransposeWs carve_t(void *ws, int64_t nnz) {
-  Carver c(ws);
-  TransposeWs t;
-  t.flags = c.take<int32_t>(64);
-  const size_t n = (size_t)std::max<int64_t>(nnz, 1);
-  t.keys0 = c.take<uint64_t>(n);
-  t.keys1 = c.take<uint64_t>(n);
-  t.vals0 = c.take<int32_t>(n);
-  t.vals1 = c.take<int32_t>(n);
-  t.e2r = c.take<int32_t>(n);
-  t.tmp = c.take<char>(radix_sort_workspace_bytes(nnz));
-  t.bytes = c.used();
-  return t;
-}
-
-__global__ void k_flags_init(int32_t *f) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) f[0] = 0;
-}
-
-__global__ __launch_bounds__(256) void k_check_csr(const int32_t *rowptr, const int32_t *col,
-                                                   int32_t M, int32_t K, int32_t nnz,
-                                                   int32_t *flags) {
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  int f = 0;
-  for (int64_t r = tid; r < M; r += stride)
-    if (rowptr[r] > rowptr[r + 1]) f |= 1;
-  for (int64_t e = tid; e < nnz; e += stride) {
-    const int c = col[e];
-    if (c < 0 || c >= K) f |= 2;
-  }
-  if (tid == 0 && (rowptr[0] != 0 || rowptr[M] != nnz)) f |= 4;
-  if (f) atomicOr(flags, f);
-}
-
-// Row, key (the column) and value (the CSR index) of every edge, edge-balanced.
-__global__ __launch_bounds__(256) void k_transpose_keys(const int32_t *rowptr,
-                                                        const int32_t *col, int32_t M,
-                                                        int32_t nnz, int32_t *e2r,
-                                                        uint64_t *keys, int32_t *vals) {
-  for_each_edge_row(rowptr, M, nnz, [&](int idx, int row) {
-    e2r[idx] = row;
-    keys[idx] = (uint32_t)col[idx];
-    vals[idx] = idx;
-  });
-}
-
-__global__ __launch_bounds__(256) void k_transpose_fill(const uint64_t *skeys,
-                                                        const int32_t *svals,
-                                                        const int32_t *e2r, int32_t nnz,
-                                                        int32_t K, int32_t *rowptr_t,
-                                                        int32_t *col_t, int32_t *perm) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nnz) {
-    const int src = svals[i];
-    perm[i] = src;
-    col_t[i] = e2r[src];
-  }
-  if (i <= K) rowptr_t[i] = lower_bound_dev<uint64_t>(skeys, 0, nnz, (uint64_t)i);
-}
-
 // out[e] = x[row(e)] . y[col(e)], edge-parallel: every wavefront takes 8
 // consecutive edges at a time (CSR order), all 64 lanes reading VEC floats of
 // each edge's two rows (one 1 KB row per edge at n = 256 and VEC = 4), so a
@@ -499,7 +429,7 @@ dtc_status_t dtc_csr_transpose_workspace_size(int32_t num_rows, int32_t num_cols
   if (!bytes) return fail(DTC_ERROR_INVALID_VALUE, "bytes is NULL");
   if (num_rows < 0 || num_cols < 0 || nnz < 0)
     return fail(DTC_ERROR_INVALID_VALUE, "sizes must be >= 0");
-  *bytes = carve_t(nullptr, nnz).bytes;
+  *bytes = transpose_workspace_bytes(nnz);
   return DTC_SUCCESS;
 }
 
@@ -515,38 +445,11 @@ dtc_status_t dtc_csr_transpose(const int32_t *node_pointer, const int32_t *edge_
     return fail(DTC_ERROR_INVALID_VALUE, "row pointers are required");
   if (nnz > 0 && (!edge_list || !edge_list_t || !perm))
     return fail(DTC_ERROR_INVALID_VALUE, "edge arrays are required when nnz > 0");
-  TransposeWs ws = carve_t(workspace, nnz);
-  if (!workspace || workspace_bytes < ws.bytes)
-    return fail(DTC_ERROR_WORKSPACE, "transpose workspace needs " + std::to_string(ws.bytes) + " bytes");
-  k_flags_init<<<1, 64, 0, stream>>>(ws.flags);
-  DTC_LAUNCH_CHECK("flags_init");
-  const int64_t work = std::max<int64_t>(std::max<int64_t>(num_rows, nnz), 1);
-  k_check_csr<<<(unsigned)std::min<int64_t>(4096, ceil_div(work, 256)), 256, 0, stream>>>(
-      node_pointer, edge_list, num_rows, num_cols, nnz, ws.flags);
-  DTC_LAUNCH_CHECK("check_csr");
-  int32_t flags = 0;
-  DTC_HIP_CHECK(hipMemcpyAsync(&flags, ws.flags, 4, hipMemcpyDeviceToHost, stream));
-  DTC_HIP_CHECK(hipStreamSynchronize(stream));
-  if (flags)
-    return fail(DTC_ERROR_INVALID_CSR, "invalid CSR for transpose (flags " + std::to_string(flags) + ")");
-  if (nnz > 0) {
-    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(65536, ceil_div(nnz, 4096)));
-    k_transpose_keys<<<grid, 256, 0, stream>>>(node_pointer, edge_list, num_rows, nnz, ws.e2r,
-                                               ws.keys0, ws.vals0);
-    DTC_LAUNCH_CHECK("transpose_keys");
-  }
-  int key_bits = 1;
-  while (key_bits < 31 && (int64_t(1) << key_bits) < num_cols) ++key_bits;
-  bool in_1 = false;
-  dtc_status_t st = radix_sort_pairs(ws.keys0, ws.vals0, ws.keys1, ws.vals1, nnz, key_bits,
-                                     &in_1, ws.tmp, stream);
-  if (st != DTC_SUCCESS) return st;
-  const int64_t n = std::max<int64_t>(nnz, (int64_t)num_cols + 1);
-  k_transpose_fill<<<(unsigned)ceil_div(n, 256), 256, 0, stream>>>(
-      in_1 ? ws.keys1 : ws.keys0, in_1 ? ws.vals1 : ws.vals0, ws.e2r, nnz, num_cols,
-      node_pointer_t, edge_list_t, perm);
-  DTC_LAUNCH_CHECK("transpose_fill");
-  return DTC_SUCCESS;
+  const size_t need = transpose_workspace_bytes(nnz);
+  if (!workspace || workspace_bytes < need)
+    return fail(DTC_ERROR_WORKSPACE, "transpose workspace needs " + std::to_string(need) + " bytes");
+  return transpose_edges(node_pointer, edge_list, num_rows, num_cols, nnz, node_pointer_t,
+                         edge_list_t, perm, workspace, stream);
 }
 
 dtc_status_t dtc_sddmm_csr(const int32_t *node_pointer, const int32_t *edge_list,

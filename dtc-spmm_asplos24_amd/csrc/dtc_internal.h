@@ -146,60 +146,6 @@ __device__ __forceinline__ int wave_lower_bound(const T *a, int lo, int hi, T ke
   return lo + __popcll(__ballot(less));
 }
 
-// Calls emit(idx, row) once for every edge idx of a CSR with M rows, the
-// edges cut into equal ranges over all waves of the grid (a long row is
-// shared by many waves instead of walked by one).  The wave finds the row of
-// its first edge by one search, then takes up to 64 edges per step, each
-// lane locating its edge's row among the next 64 row ends held in lanes.
-// Must be called by whole waves with the same arguments.
-// As for_each_edge_row, with a per-edge value loaded at the start of each
-// step together with the row ends (one memory round trip per step instead of
-// two): load(e) for the step's edge e = p + lane (clamped to the range), and
-// emit(idx, row, value) gets the value of its own edge.
-template <class Load, class Emit>
-__device__ __forceinline__ void for_each_edge_row_load(const int32_t *rowptr, int32_t M, int32_t nnz,
-                                                       Load load, Emit emit) {
-  const int lane = lane_id();
-  const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
-  const int64_t w = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave_uniform(threadIdx.x >> 6);
-  const int e_begin = (int)((int64_t)nnz * w / nw);
-  const int e_end = (int)((int64_t)nnz * (w + 1) / nw);
-  if (e_begin >= e_end) return;
-  // the row of e_begin: the last r with rowptr[r] <= e_begin
-  int r = wave_uniform(wave_lower_bound<int32_t>(rowptr, 0, M + 1, e_begin + 1) - 1);
-  int p = e_begin;
-  while (p < e_end) {
-    const auto val = load(min(p + lane, e_end - 1));
-    const int64_t bi = (int64_t)r + 1 + lane;
-    const int bnd = bi <= M ? rowptr[bi] : INT32_MAX;
-    const uint64_t past = __ballot(bnd > p);
-    if (past == 0) {  // rows r .. r+63 all end at or before p (empty rows)
-      r += kWave;
-      continue;
-    }
-    const int last = __builtin_amdgcn_readlane(bnd, kWave - 1);  // > p
-    const int cnt = min(min(kWave, e_end - p), last - p);
-    const int idx = p + min(lane, cnt - 1);
-    int lo = 0, hi = kWave - 1;  // first lane whose row end exceeds idx (lane 63's does)
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (__shfl(bnd, mid, kWave) > idx) hi = mid;
-      else lo = mid + 1;
-    }
-    const int row = r + lo;
-    if (lane < cnt) emit(idx, row, val);  // idx = p + lane here: val is its own edge's
-    r = wave_uniform(__shfl(row, cnt - 1, kWave));  // row of the step's last edge
-    p += cnt;
-  }
-}
-
-template <class Emit>
-__device__ __forceinline__ void for_each_edge_row(const int32_t *rowptr, int32_t M, int32_t nnz,
-                                                  Emit emit) {
-  for_each_edge_row_load(
-      rowptr, M, nnz, [](int) { return 0; }, [&](int idx, int row, int) { emit(idx, row); });
-}
-
 // ----------------------------------------------------- device-wide pieces
 // (implemented in primitives.hip)
 
@@ -220,5 +166,12 @@ size_t radix_sort_workspace_bytes(int64_t n);
 dtc_status_t radix_sort_pairs(uint64_t *keys0, int32_t *vals0, uint64_t *keys1,
                               int32_t *vals1, int64_t n, int key_bits, bool *result_in_1,
                               void *ws, hipStream_t stream);
+
+// Checks the CSR (M rows, K columns; one host synchronisation), then the CSR
+// of its transpose with, for every edge of that, the edge it was.
+size_t transpose_workspace_bytes(int64_t nnz);
+dtc_status_t transpose_edges(const int32_t *rowptr, const int32_t *col, int32_t M, int32_t K,
+                             int32_t nnz, int32_t *rowptr_t, int32_t *col_t, int32_t *perm,
+                             void *ws, hipStream_t stream);
 
 }  // namespace dtc

@@ -202,11 +202,14 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const Key *key
   int64_t start, hbase;
   int len, hstride;
   tiles.get(blockIdx.x, start, len, hbase, hstride);
-#pragma unroll 4
-  for (int k = 0; k < kSortItems; ++k) {
-    const int i = k * kSortThreads + threadIdx.x;
-    if (i < len) atomicAdd(&cnt[(int)((keys[start + i] >> shift) & (kRadix - 1))], 1);
-  }
+  Key kreg[kSortItems];  // all loads in flight before the first count
+#pragma unroll
+  for (int k = 0; k < kSortItems; ++k)
+    kreg[k] = keys[start + min(k * kSortThreads + (int)threadIdx.x, len - 1)];
+#pragma unroll
+  for (int k = 0; k < kSortItems; ++k)
+    if (k * kSortThreads + (int)threadIdx.x < len)
+      atomicAdd(&cnt[(int)((kreg[k] >> shift) & (kRadix - 1))], 1);
   __syncthreads();
   hist[hbase + (int64_t)threadIdx.x * hstride] = cnt[threadIdx.x];
 }
@@ -229,16 +232,41 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const Key *key
 constexpr int kSortWaves = kSortThreads / 64;
 constexpr int kWaveItems = kSortTile / kSortWaves;  // 1,024 elements per wave
 
-template <class Key, class Tiles>
-__global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
-    const Key *kin, const int32_t *vin, Key *kout, int32_t *vout, int shift,
-    const int32_t *offsets, Tiles tiles) {
+//
+// In gives the key and the value words of element i, the first kComputed of
+// them from i alone; Out takes them at their place.  Keys and words go through
+// the same LDS buffer one after another (a 16 KB buffer instead of one for each
+// keeps four to six workgroups on a CU instead of two).
+template <class Key>
+struct PairIn {
+  typedef Key key_type;
+  static constexpr int kWords = 1, kComputed = 0;
+  const Key *k;
+  const int32_t *v;
+  __device__ __forceinline__ void tile(int64_t, int, int32_t *, int *) const {}
+  __device__ __forceinline__ Key key(int64_t i) const { return k[i]; }
+  __device__ __forceinline__ int32_t word(int, int64_t i, int, const int32_t *) const { return v[i]; }
+};
+template <class Key>
+struct PairOut {
+  Key *k;
+  int32_t *v;
+  __device__ __forceinline__ void key(int64_t i, Key x) const { k[i] = x; }
+  __device__ __forceinline__ void word(int, int64_t i, int32_t x) const { v[i] = x; }
+};
+
+template <class In, class Out, class Tiles>
+__global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(In in, Out out, int shift,
+                                                                      const int32_t *offsets,
+                                                                      Tiles tiles) {
+  typedef typename In::key_type Key;
+  constexpr int NW = In::kWords;
   __shared__ int s_off[kRadix];             // global position of the tile's first element of digit d
   __shared__ int s_loc[kRadix];             // local position of the same element
   __shared__ int s_wcnt[kSortWaves][kRadix];  // per-wave digit counts, then per-wave prefixes
   __shared__ int s_scan[kSortWaves];
   __shared__ Key s_keys[kSortTile];
-  __shared__ int32_t s_vals[kSortTile];
+  int32_t *s_word = reinterpret_cast<int32_t *>(s_keys);
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
@@ -251,12 +279,15 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
   // All of the wave's keys and values are loaded up front (one memory
   // latency for the whole tile).
   Key kreg[kSortItems];
-  int32_t vreg[kSortItems];
+  int32_t vreg[NW][kSortItems];
+  in.tile(start, len, s_word, s_scan);
 #pragma unroll
   for (int r = 0; r < kSortItems; ++r) {
     const int i = wbase + r * 64 + lane;
-    kreg[r] = i < len ? kin[start + i] : (Key)0;
-    vreg[r] = i < len ? vin[start + i] : 0;
+    kreg[r] = i < len ? in.key(start + i) : (Key)0;
+#pragma unroll
+    for (int w = In::kComputed; w < NW; ++w)
+      vreg[w][r] = i < len ? in.word(w, start + i, i, s_word) : 0;
   }
   s_off[tid] = offsets[hbase + (int64_t)tid * hstride];
 #pragma unroll
@@ -298,22 +329,41 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
   for (int w = 0; w < kSortWaves; ++w) pre += w < wave ? s_scan[w] : 0;
   s_loc[tid] = pre + inc - cnt;
   __syncthreads();
+  // lrank: place in the tile's layout; pos: place in the output of the element
+  // that this thread writes
+  int pos[kSortItems];
 #pragma unroll
   for (int r = 0; r < kSortItems; ++r) {
     if (wbase + r * 64 + lane < len) {
       const int d = (int)((kreg[r] >> shift) & (kRadix - 1));
-      const int lp = s_loc[d] + s_wcnt[wave][d] + lrank[r];
-      s_keys[lp] = kreg[r];
-      s_vals[lp] = vreg[r];
+      lrank[r] += s_loc[d] + s_wcnt[wave][d];
+      s_keys[lrank[r]] = kreg[r];
     }
   }
   __syncthreads();
-  for (int j = tid; j < len; j += kSortThreads) {
-    const Key key = s_keys[j];
-    const int d = (int)((key >> shift) & (kRadix - 1));
-    const int64_t pos = (int64_t)s_off[d] + (j - s_loc[d]);
-    kout[pos] = key;
-    vout[pos] = s_vals[j];
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int j = r * kSortThreads + tid;
+    if (j < len) {
+      const Key key = s_keys[j];
+      const int d = (int)((key >> shift) & (kRadix - 1));
+      pos[r] = s_off[d] + (j - s_loc[d]);
+      out.key(pos[r], key);
+    }
+  }
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+      if (wbase + r * 64 + lane < len)
+        s_word[lrank[r]] = w < In::kComputed
+                               ? in.word(w, start + wbase + r * 64 + lane, 0, nullptr)
+                               : vreg[w][r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSortItems; ++r)
+      if (r * kSortThreads + tid < len) out.word(w, pos[r], s_word[r * kSortThreads + tid]);
   }
 }
 
@@ -343,8 +393,8 @@ dtc_status_t radix_sort_pairs(uint64_t *keys0, int32_t *vals0, uint64_t *keys1,
     DTC_LAUNCH_CHECK("radix_hist");
     dtc_status_t st = scan_i32(hist, hist, ntiles * kRadix, false, scan_ws, stream);
     if (st != DTC_SUCCESS) return st;
-    radix_scatter_kernel<uint64_t, PlainTiles>
-        <<<(unsigned)ntiles, kSortThreads, 0, stream>>>(kin, vin, kout, vout, shift, hist, tiles);
+    radix_scatter_kernel<<<(unsigned)ntiles, kSortThreads, 0, stream>>>(
+        PairIn<uint64_t>{kin, vin}, PairOut<uint64_t>{kout, vout}, shift, hist, tiles);
     DTC_LAUNCH_CHECK("radix_scatter");
     std::swap(kin, kout);
     std::swap(vin, vout);
@@ -383,14 +433,223 @@ dtc_status_t seg_radix_sort_pairs_u32(uint32_t *keys0, int32_t *vals0, uint32_t 
     DTC_LAUNCH_CHECK("radix_hist");
     dtc_status_t st = scan_i32(hist, hist, ntiles * kRadix, false, scan_ws, stream);
     if (st != DTC_SUCCESS) return st;
-    radix_scatter_kernel<uint32_t, SegTiles>
-        <<<(unsigned)ntiles, kSortThreads, 0, stream>>>(kin, vin, kout, vout, shift, hist, tiles);
+    radix_scatter_kernel<<<(unsigned)ntiles, kSortThreads, 0, stream>>>(
+        PairIn<uint32_t>{kin, vin}, PairOut<uint32_t>{kout, vout}, shift, hist, tiles);
     DTC_LAUNCH_CHECK("radix_scatter");
     std::swap(kin, kout);
     std::swap(vin, vout);
     in_1 = !in_1;
   }
   *result_in_1 = in_1;
+  return DTC_SUCCESS;
+}
+
+// ------------------------------------------------------------ CSR transpose
+//
+// Stable sort of the edges by column, carrying (edge, row).  The first pass
+// reads the columns themselves and makes edge and row on the way, the last one
+// writes the transposed arrays, so that an edge moves 4 + 12 bytes in the first
+// pass and 12 + 12 in each other one.  12.2 M edges of 60,000 columns: check and
+// counts 19 us, passes 103 and 86 (3.4 TB/s: runs of 16 elements), counts 21,
+// row pointer 14; with 64-bit keys, a kernel that made them and one that looked
+// every edge's row up at the end it took 420 us.
+
+// Edges in CSR order.  The row of every edge of the tile: each row that starts
+// in the tile marks its first entry (a later one overrides an empty one before
+// it), and an entry's row is the largest mark up to it.
+struct EdgeIn {
+  typedef uint32_t key_type;
+  static constexpr int kWords = 2, kComputed = 1;
+  const int32_t *col, *rowptr;
+  int32_t M;
+  __device__ __forceinline__ void tile(int64_t start, int len, int32_t *s_row, int *s_scan) const {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int4 none = make_int4(0, 0, 0, 0);
+    int4 *mine = reinterpret_cast<int4 *>(s_row) + tid * (kSortItems / 4);
+#pragma unroll
+    for (int k = 0; k < kSortItems / 4; ++k) mine[k] = none;
+    // rows of the tile's first and last entry: the last r with rowptr[r] <= e
+    const int e0 = (int)start, e1 = (int)start + len - 1;
+    const int r0 = wave_lower_bound<int32_t>(rowptr, 0, M + 1, e0 + 1) - 1;
+    const int r1 = wave_lower_bound<int32_t>(rowptr, r0 + 1, M + 1, e1 + 1) - 1;
+    __syncthreads();
+    for (int64_t r = (int64_t)r0 + 1 + tid; r <= r1; r += kSortThreads)
+      atomicMax(&s_row[rowptr[r] - e0], (int)r);
+    __syncthreads();
+    int m[kSortItems];
+    int top = r0;
+#pragma unroll
+    for (int k = 0; k < kSortItems / 4; ++k) {
+      const int4 v = mine[k];
+      m[4 * k] = top = max(top, v.x);
+      m[4 * k + 1] = top = max(top, v.y);
+      m[4 * k + 2] = top = max(top, v.z);
+      m[4 * k + 3] = top = max(top, v.w);
+    }
+    int up = top;  // largest mark of this and the lower lanes
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int t = __shfl_up(up, d, kWave);
+      if (lane >= d) up = max(up, t);
+    }
+    if (lane == kWave - 1) s_scan[tid >> 6] = up;
+    int below = __shfl_up(up, 1, kWave);
+    if (lane == 0) below = r0;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w)
+      if (w < (tid >> 6)) below = max(below, s_scan[w]);
+#pragma unroll
+    for (int k = 0; k < kSortItems / 4; ++k)
+      mine[k] = make_int4(max(m[4 * k], below), max(m[4 * k + 1], below), max(m[4 * k + 2], below),
+                          max(m[4 * k + 3], below));
+    __syncthreads();
+  }
+  __device__ __forceinline__ uint32_t key(int64_t i) const { return (uint32_t)col[i]; }
+  __device__ __forceinline__ int32_t word(int w, int64_t i, int j, const int32_t *s_row) const {
+    return w == 0 ? (int32_t)i : s_row[j];
+  }
+};
+struct EdgePairIn {
+  typedef uint32_t key_type;
+  static constexpr int kWords = 2, kComputed = 0;
+  const uint32_t *k;
+  const int32_t *edge, *row;
+  __device__ __forceinline__ void tile(int64_t, int, int32_t *, int *) const {}
+  __device__ __forceinline__ uint32_t key(int64_t i) const { return k[i]; }
+  __device__ __forceinline__ int32_t word(int w, int64_t i, int, const int32_t *) const {
+    return w == 0 ? edge[i] : row[i];
+  }
+};
+struct EdgePairOut {
+  uint32_t *k;
+  int32_t *edge, *row;
+  __device__ __forceinline__ void key(int64_t i, uint32_t x) const { k[i] = x; }
+  __device__ __forceinline__ void word(int w, int64_t i, int32_t x) const {
+    if (w == 0) edge[i] = x;
+    else row[i] = x;
+  }
+};
+
+__global__ void transpose_flags_kernel(int32_t *f) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) f[0] = 0;
+}
+
+// The digit counts of the first pass together with the checks of the CSR: 1
+// row pointer decreases, 2 column outside [0, K), 4 its ends.
+__global__ __launch_bounds__(kSortThreads) void transpose_check_kernel(
+    const int32_t *rowptr, const int32_t *col, int32_t M, int32_t K, int32_t nnz, int32_t ntiles,
+    int32_t *hist, int32_t *flags) {
+  __shared__ int cnt[kRadix];
+  const int64_t tid = (int64_t)blockIdx.x * kSortThreads + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * kSortThreads;
+  int f = 0;
+  for (int64_t r = tid; r < M; r += stride)
+    if (rowptr[r] > rowptr[r + 1]) f |= 1;
+  if (tid == 0 && (rowptr[0] != 0 || rowptr[M] != nnz)) f |= 4;
+  if ((int)blockIdx.x < ntiles) {  // workgroup-uniform
+    cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t start = (int64_t)blockIdx.x * kSortTile;
+    const int len = (int)min<int64_t>(kSortTile, nnz - start);
+    int c[kSortItems];
+#pragma unroll
+    for (int k = 0; k < kSortItems; ++k)
+      c[k] = col[start + min(k * kSortThreads + (int)threadIdx.x, len - 1)];
+#pragma unroll
+    for (int k = 0; k < kSortItems; ++k) {
+      if (c[k] < 0 || c[k] >= K) f |= 2;
+      if (k * kSortThreads + (int)threadIdx.x < len) atomicAdd(&cnt[c[k] & (kRadix - 1)], 1);
+    }
+    __syncthreads();
+    hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = cnt[threadIdx.x];
+  }
+  if (f) atomicOr(flags, f);
+}
+
+// rowptr_t[c] = edges of columns below c.
+__global__ __launch_bounds__(kSortThreads) void transpose_rowptr_kernel(const uint32_t *keys,
+                                                                        int32_t nnz, int32_t K,
+                                                                        int32_t *rowptr_t) {
+  const int64_t i = (int64_t)blockIdx.x * kSortThreads + threadIdx.x;
+  if (i <= K) rowptr_t[i] = lower_bound_dev<uint32_t>(keys, 0, nnz, (uint32_t)i);
+}
+
+struct TransposeWs {
+  int32_t *flags, *hist;
+  uint32_t *keys[2];
+  int32_t *edge, *row;  // of the passes between the first and the last
+  int32_t *edge1, *row1;
+  void *scan;
+  size_t bytes;
+};
+
+static TransposeWs carve_transpose(void *ws, int64_t nnz) {
+  Carver c(ws);
+  TransposeWs t;
+  const size_t n = (size_t)std::max<int64_t>(nnz, 1);
+  const int64_t counts = ceil_div((int64_t)n, kSortTile) * kRadix;
+  t.flags = c.take<int32_t>(64);
+  for (int i = 0; i < 2; ++i) t.keys[i] = c.take<uint32_t>(n);
+  t.edge = c.take<int32_t>(n);
+  t.row = c.take<int32_t>(n);
+  t.edge1 = c.take<int32_t>(n);
+  t.row1 = c.take<int32_t>(n);
+  t.hist = c.take<int32_t>((size_t)counts);
+  t.scan = c.take<char>(scan_workspace_bytes(counts));
+  t.bytes = c.used();
+  return t;
+}
+
+size_t transpose_workspace_bytes(int64_t nnz) { return carve_transpose(nullptr, nnz).bytes; }
+
+dtc_status_t transpose_edges(const int32_t *rowptr, const int32_t *col, int32_t M, int32_t K,
+                             int32_t nnz, int32_t *rowptr_t, int32_t *col_t, int32_t *perm,
+                             void *workspace, hipStream_t stream) {
+  const TransposeWs t = carve_transpose(workspace, nnz);
+  const int64_t ntiles = ceil_div(nnz, kSortTile);
+  if (ntiles * kRadix > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "sort too large");
+  transpose_flags_kernel<<<1, 64, 0, stream>>>(t.flags);
+  DTC_LAUNCH_CHECK("flags_init");
+  const unsigned check = (unsigned)std::max<int64_t>(std::max<int64_t>(ntiles, 1),
+                                                     std::min<int64_t>(1024, ceil_div(M, kSortThreads)));
+  transpose_check_kernel<<<check, kSortThreads, 0, stream>>>(rowptr, col, M, K, nnz, (int32_t)ntiles,
+                                                             t.hist, t.flags);
+  DTC_LAUNCH_CHECK("transpose_check");
+  int32_t flags = 0;
+  DTC_HIP_CHECK(hipMemcpyAsync(&flags, t.flags, 4, hipMemcpyDeviceToHost, stream));
+  DTC_HIP_CHECK(hipStreamSynchronize(stream));
+  if (flags)
+    return fail(DTC_ERROR_INVALID_CSR, "invalid CSR for transpose (flags " + std::to_string(flags) + ")");
+  int key_bits = 1;
+  while (key_bits < 31 && (int64_t(1) << key_bits) < K) ++key_bits;
+  const PlainTiles tiles{nnz, (int)ntiles};
+  int at = 0;  // keys[at]: the passes' keys so far
+  for (int shift = 0; shift < key_bits && nnz > 0; shift += 8) {
+    const bool last = shift + 8 >= key_bits;
+    uint32_t *kin = t.keys[at], *kout = t.keys[at ^ 1];
+    int32_t *ein = at ? t.edge1 : t.edge, *rin = at ? t.row1 : t.row;
+    const EdgePairOut out = {kout, last ? perm : at ? t.edge : t.edge1,
+                             last ? col_t : at ? t.row : t.row1};
+    if (shift > 0) {
+      radix_hist_kernel<uint32_t, PlainTiles>
+          <<<(unsigned)ntiles, kSortThreads, 0, stream>>>(kin, shift, t.hist, tiles);
+      DTC_LAUNCH_CHECK("radix_hist");
+    }
+    dtc_status_t st = scan_i32(t.hist, t.hist, ntiles * kRadix, false, t.scan, stream);
+    if (st != DTC_SUCCESS) return st;
+    if (shift == 0)
+      radix_scatter_kernel<<<(unsigned)ntiles, kSortThreads, 0, stream>>>(
+          EdgeIn{col, rowptr, M}, out, shift, t.hist, tiles);
+    else
+      radix_scatter_kernel<<<(unsigned)ntiles, kSortThreads, 0, stream>>>(
+          EdgePairIn{kin, ein, rin}, out, shift, t.hist, tiles);
+    DTC_LAUNCH_CHECK("radix_scatter");
+    at ^= 1;
+  }
+  transpose_rowptr_kernel<<<(unsigned)ceil_div((int64_t)K + 1, kSortThreads), kSortThreads, 0,
+                            stream>>>(t.keys[at], nnz, K, rowptr_t);
+  DTC_LAUNCH_CHECK("transpose_rowptr");
   return DTC_SUCCESS;
 }
 
