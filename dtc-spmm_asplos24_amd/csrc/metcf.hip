@@ -97,6 +97,7 @@ static_assert(offsetof(MetcfHeader, pad) <= kHeaderRead, "header read size");
 constexpr int kBadFirst = 1;     // rowptr[0] != 0
 constexpr int kBadLast = 2;      // rowptr[M] != nnz
 constexpr int kBadOrder = 4;     // rowptr decreases
+constexpr int kBadRowptr = kBadFirst | kBadLast | kBadOrder;
 constexpr int kBadColumn = 8;    // negative column index
 constexpr int kBadClass = 16;    // a window larger than its class (internal)
 constexpr int kBadPartition = 32;  // blockPartition of an empty window is not zero
@@ -187,7 +188,7 @@ bool one_stream() {
   return e && !std::strcmp(e, "1");
 }
 
-__global__ void k_header_init(MetcfHeader *h) {
+__device__ __forceinline__ void header_init(MetcfHeader *h) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     h->flags = 0;
     h->nnz_big = 0;
@@ -198,6 +199,18 @@ __global__ void k_header_init(MetcfHeader *h) {
   }
 }
 
+__global__ void k_header_init(MetcfHeader *h) { header_init(h); }
+
+// What the host reads, written by the kernel that has it last straight to
+// pinned host memory (a copy would be a launch and a kernel more): the header,
+// then the block count.  Called by one workgroup, after a barrier.
+__device__ __forceinline__ void report_header(MetcfHeader *h, int32_t *host) {
+  int32_t *words = reinterpret_cast<int32_t *>(h);
+  if (threadIdx.x < kHeaderRead / 4)
+    host[threadIdx.x] = __hip_atomic_load(&words[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void k_report(MetcfHeader *h, int32_t *host) { report_header(h, host); }
 
 // Checks rowptr[0] == 0, rowptr[M] == nnz and rowptr non-decreasing, which
 // keeps every window's entries inside the edge arrays.  (Columns are checked
@@ -232,14 +245,14 @@ __device__ __forceinline__ int window_end(const int32_t *rowptr, int w, int blk_
 // does not affect any output): an LDS class, or the global path (list
 // kClasses, whose entries are summed into nnz_big).  Empty windows must have
 // blockPartition 0 (the caller zero-fills it; empty windows are not written).
-// Also writes row_window_offset[0] = 0.
-__device__ __forceinline__ void classify_part(const int32_t *rowptr, int32_t M, int32_t W,
+// Also writes row_window_offset[0] = 0.  One window per thread (w64, none past W).
+__device__ __forceinline__ void classify_part(int64_t w64, const int32_t *rowptr, int32_t M, int32_t W,
                                               int32_t blk_h, int mode, const int32_t *bp,
                                               const int32_t *col, int32_t nnz, int32_t *lists,
                                               int32_t *rwo, MetcfHeader *h) {
   constexpr int NC = kClasses + 1;
   __shared__ int s_cnt[NC], s_base[NC], s_big;
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  const int w = (int)min(w64, (int64_t)W);
   const int lane = threadIdx.x & 63;
   if (threadIdx.x < NC) s_cnt[threadIdx.x] = 0;
   if (threadIdx.x == 0) s_big = 0;
@@ -317,7 +330,7 @@ __global__ __launch_bounds__(256) void k_check_classify(const int32_t *rowptr, i
                                                         const int32_t *col, int32_t *lists,
                                                         int32_t *rwo, MetcfHeader *h) {
   validate_part(rowptr, M, nnz, h);
-  classify_part(rowptr, M, W, blk_h, mode, bp, col, nnz, lists, rwo, h);
+  classify_part((int64_t)blockIdx.x * blockDim.x + threadIdx.x, rowptr, M, W, blk_h, mode, bp, col, nnz, lists, rwo, h);
 }
 
 // Exclusive prefix sum by one 1,024-thread workgroup, 16 items per thread
@@ -370,13 +383,11 @@ __device__ __forceinline__ int wg1024_exclusive_scan(Load load, Store store, int
 // leaves the work to the multi-workgroup kernels when it exceeds
 // kOneGroupWindows.
 constexpr int kOneGroupWindows = 4096;  // up to this many: one-workgroup kernels
-__global__ __launch_bounds__(1024) void k_big_offsets(const int32_t *rowptr, int32_t M,
-                                                      int32_t blk_h, const int32_t *wmap,
-                                                      const MetcfHeader *h, int32_t tile,
-                                                      int32_t *csb, int32_t *tb, int32_t *tw) {
+__device__ __forceinline__ void big_offsets_part(int n_big, const int32_t *rowptr, int32_t M,
+                                                 int32_t blk_h, const int32_t *wmap, int32_t tile,
+                                                 int32_t *csb, int32_t *tb, int32_t *tw) {
   constexpr int IT = kOneGroupWindows / 1024;  // windows per thread
   __shared__ int s_e[16], s_t[16];
-  const int n_big = h->cls_count[kClasses];
   if (n_big == 0 || n_big > kOneGroupWindows) return;  // workgroup-uniform
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   // entries and sort tiles of this thread's windows, loaded once
@@ -421,6 +432,50 @@ __global__ __launch_bounds__(1024) void k_big_offsets(const int32_t *rowptr, int
   }
 }
 
+__global__ __launch_bounds__(1024) void k_big_offsets(const int32_t *rowptr, int32_t M,
+                                                      int32_t blk_h, const int32_t *wmap,
+                                                      const MetcfHeader *h, int32_t tile,
+                                                      int32_t *csb, int32_t *tb, int32_t *tw) {
+  if (h->flags & kBadRowptr) return;  // the windows' ranges may lie outside the edge arrays
+  big_offsets_part(h->cls_count[kClasses], rowptr, M, blk_h, wmap, tile, csb, tb, tw);
+}
+
+// Everything before the first host read in one workgroup, for up to
+// kOnePlanWindows windows: header, row-pointer check, classes, offsets of the
+// global path's windows, report.  (A dozen launches were most of a small build:
+// with k_window_offsets and without the copies, 4,096 rows of 16 entries went
+// from 106 to 57 us.  Whole builds with this kernel and with the launches it
+// replaces, 8 entries a row: 256 windows 56 and 64 us, 1,024 60 and 64, 2,048
+// 68 and 67, 4,096 86 and 72.)
+constexpr int kOnePlanWindows = 1024;
+__global__ __launch_bounds__(1024) void k_plan(const int32_t *rowptr, int32_t M, int32_t nnz,
+                                               int32_t W, int32_t blk_h, int mode,
+                                               const int32_t *bp, const int32_t *col,
+                                               int32_t *lists, int32_t *rwo, int32_t tile,
+                                               int32_t *csb, int32_t *tb, int32_t *tw,
+                                               MetcfHeader *h, int32_t *host) {
+  __shared__ MetcfHeader s_h;
+  header_init(&s_h);
+  __syncthreads();
+  validate_part(rowptr, M, nnz, &s_h);
+  __syncthreads();
+  if (s_h.flags == 0) {  // else the windows' ranges may lie outside the edge arrays
+    for (int w = 0; w < W; w += blockDim.x) {
+      __syncthreads();
+      classify_part(w + threadIdx.x, rowptr, M, W, blk_h, mode, bp, col, nnz, lists, rwo, &s_h);
+    }
+    __syncthreads();
+    big_offsets_part(s_h.cls_count[kClasses], rowptr, M, blk_h, lists + (int64_t)kClasses * W, tile,
+                     csb, tb, tw);
+  }
+  __syncthreads();
+  const int32_t *words = reinterpret_cast<const int32_t *>(&s_h);
+  if (threadIdx.x < kHeaderRead / 4) {
+    reinterpret_cast<int32_t *>(h)[threadIdx.x] = words[threadIdx.x];
+    host[threadIdx.x] = words[threadIdx.x];
+  }
+}
+
 // Largest column of the global path's windows (the width of its sort keys)
 // and negative columns there, read by tiles of `tile` entries as laid out by
 // k_big_offsets; with more than kOneGroupWindows such windows (their tiles
@@ -434,7 +489,7 @@ __global__ __launch_bounds__(256) void k_big_maxcol(const int32_t *rowptr, const
                                                     const int32_t *tb, const int32_t *tw,
                                                     int32_t tile, MetcfHeader *h) {
   const int n_big = h->cls_count[kClasses];
-  if (n_big == 0) return;  // workgroup-uniform
+  if (n_big == 0 || (h->flags & kBadRowptr)) return;  // workgroup-uniform
   int mx = 0, neg = 0;
   bool unsorted = n_big > kOneGroupWindows;
   if (n_big <= kOneGroupWindows) {
@@ -1403,21 +1458,55 @@ constexpr int kOutWin = 1024;  // row-window offsets kept in LDS
 // T))), so that its workgroups start without a search.  One thread per
 // window; a window writes the chunks whose first or last block it holds
 // (every block has at least one entry, so T <= nnz and c < cw_stride).
-__global__ __launch_bounds__(256) void k_chunk_windows(const int32_t *__restrict__ rwo, int32_t W,
-                                                       int32_t *__restrict__ cw_first,
-                                                       int32_t *__restrict__ cw_last) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= W) return;
-  const int64_t b0 = rwo[w], b1 = rwo[w + 1];
+__device__ __forceinline__ void chunk_windows_part(int w, int32_t b0, int64_t b1, int64_t T,
+                                                   int32_t *__restrict__ cw_first,
+                                                   int32_t *__restrict__ cw_last) {
   if (b0 >= b1) return;  // empty window: no block
-  const int64_t T = rwo[W];
-  for (int64_t c = (b0 + kOutBlocks - 1) / kOutBlocks; c * kOutBlocks < b1; ++c)
+  for (int64_t c = ((int64_t)b0 + kOutBlocks - 1) / kOutBlocks; c * kOutBlocks < b1; ++c)
     cw_first[c] = w;
   for (int64_t c = b0 / kOutBlocks; c <= (b1 - 1) / kOutBlocks; ++c) {
     const int64_t last = std::min(c * kOutBlocks + kOutBlocks, T) - 1;
     if (last >= b0 && last < b1) cw_last[c] = w;
   }
 }
+
+// (also reports the header and the block count)
+__global__ __launch_bounds__(256) void k_chunk_windows(const int32_t *__restrict__ rwo, int32_t W,
+                                                       int32_t *__restrict__ cw_first,
+                                                       int32_t *__restrict__ cw_last,
+                                                       MetcfHeader *h, int32_t *host) {
+  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w < W) chunk_windows_part(w, rwo[w], rwo[w + 1], rwo[W], cw_first, cw_last);
+  if (blockIdx.x == 0) {
+    report_header(h, host);
+    if (threadIdx.x == 0) host[kHeaderRead / 4] = rwo[W];
+  }
+}
+
+// The window offsets and what k_chunk_windows makes of them in one workgroup,
+// for up to kOneScanWindows windows.  (Whole builds with it and with the four
+// kernels it replaces: 256 windows 56 and 60 us, 4,096 72 and 76, 8,192 90 and
+// 87, 16,384 120 and 103.)
+constexpr int kOneScanWindows = 4096;
+__global__ __launch_bounds__(1024) void k_window_offsets(const int32_t *__restrict__ bp, int32_t W,
+                                                         int32_t *rwo,
+                                                         int32_t *__restrict__ cw_first,
+                                                         int32_t *__restrict__ cw_last,
+                                                         MetcfHeader *h, int32_t *host) {
+  __shared__ int s_tmp[16];
+  const int T = wg1024_exclusive_scan([&](int w) { return bp[w]; },
+                                      [&](int w, int x) { rwo[w] = x; }, W, s_tmp);
+  if (threadIdx.x == 0) {
+    rwo[W] = T;
+    host[kHeaderRead / 4] = T;
+  }
+  report_header(h, host);
+  __threadfence_block();
+  __syncthreads();
+  for (int w = threadIdx.x; w < W; w += 1024)
+    chunk_windows_part(w, rwo[w], (int64_t)rwo[w] + bp[w], T, cw_first, cw_last);
+}
+
 __global__ __launch_bounds__(256) void k_blocks_out(const int32_t *__restrict__ rowptr, int32_t M,
                                                     int32_t W, int32_t blk_h, int32_t blk_w,
                                                     int32_t T, int32_t nnz, WinStage st,
@@ -2030,15 +2119,15 @@ WinStage win_stage(const MetcfWs &ws) {
 }
 
 // The global path runs on a library-owned stream of the current device
-// (default priority, created once), forked from and joined back to the
-// caller's stream with events, so that it overlaps the LDS path: the two
-// write disjoint windows.  `mu` is held from the fork to the join of one
+// (default priority, created once), started when the caller's stream is idle
+// and joined back to it with an event, so that it overlaps the LDS path: the
+// two write disjoint windows.  `mu` is held from the start to the join of one
 // build so that concurrent builds do not interleave their event records.
 struct SideStream {
   hipStream_t s = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
+  hipEvent_t join = nullptr;
   std::mutex mu;
-  // pinned host words for the build's device-to-host reads (header, block
+  // pinned host words that the build's kernels report to (header, block
   // count), guarded by `read_mu`
   char *pinned = nullptr;
   std::mutex read_mu;
@@ -2054,7 +2143,6 @@ dtc_status_t side_stream(SideStream **out) {
   if (!per_dev[dev]) {
     SideStream *x = new SideStream;
     DTC_HIP_CHECK(hipStreamCreateWithFlags(&x->s, hipStreamNonBlocking));
-    DTC_HIP_CHECK(hipEventCreateWithFlags(&x->fork, hipEventDisableTiming));
     DTC_HIP_CHECK(hipEventCreateWithFlags(&x->join, hipEventDisableTiming));
     DTC_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&x->pinned), 256, hipHostMallocDefault));
     per_dev[dev] = x;
@@ -2161,49 +2249,59 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
   // 1. Row-pointer check, window classes, the global path's largest column
   //    (negative columns are flagged where they are read) (first host
   //    synchronisation).
-  k_header_init<<<1, 64, 0, stream>>>(ws.hdr);
-  DTC_LAUNCH_CHECK("header_init");
-  {
-    // up to 1,024 workgroups for the row check, and one per 256 windows for
-    // the classes
-    const unsigned grid = (unsigned)std::max<int64_t>(
-        std::min<int64_t>(1024, grid_for(num_nodes, 256)), grid_for(W, 256));
-    k_check_classify<<<grid, 256, 0, stream>>>(node_pointer, num_nodes, nnz, (int32_t)W, blk_h,
-                                               mode, block_partition, edge_list, ws.lists,
-                                               row_window_offset, ws.hdr);
-    DTC_LAUNCH_CHECK("check_classify");
-  }
-  if (W > 0) {
-    // offsets and sort tiles of up to kOneGroupWindows global-path windows
-    k_big_offsets<<<1, 1024, 0, stream>>>(node_pointer, num_nodes, blk_h,
-                                          ws.lists + (int64_t)kClasses * W, ws.hdr,
-                                          (int32_t)seg_radix_tile_size(), ws.csb, ws.tb, ws.tw);
-    DTC_LAUNCH_CHECK("big_offsets");
-    k_big_maxcol<<<1024, 256, 0, stream>>>(node_pointer, edge_list, num_nodes, nnz, blk_h,
-                                           ws.lists + (int64_t)kClasses * W, ws.csb, ws.tb,
-                                           ws.tw, (int32_t)seg_radix_tile_size(), ws.hdr);
-    DTC_LAUNCH_CHECK("big_maxcol");
-  }
   SideStream *dev_state = nullptr;
   st = side_stream(&dev_state);
   if (st != DTC_SUCCESS) return st;
-  // The side stream is forked here, before the first host synchronisation,
-  // so that the global path's first kernel starts as soon as it is issued;
-  // the lock keeps other builds on this device off the side stream until
-  // the join.
-  std::unique_lock<std::mutex> side_lock(dev_state->mu);
-  if (W > 0) {
-    DTC_HIP_CHECK(hipEventRecord(dev_state->fork, stream));
-    DTC_HIP_CHECK(hipStreamWaitEvent(dev_state->s, dev_state->fork, 0));
-  }
+  int32_t *report = reinterpret_cast<int32_t *>(dev_state->pinned);
+  const int32_t *big_list = ws.lists + (int64_t)kClasses * W;
+  const int32_t sort_tile = (int32_t)seg_radix_tile_size();
   MetcfHeader host{};
   {
+    // held from the launch of the kernel that reports to the read
     std::lock_guard<std::mutex> g(dev_state->read_mu);
-    DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned, ws.hdr, kHeaderRead, hipMemcpyDeviceToHost,
-                                 stream));
-    DTC_HIP_CHECK(hipStreamSynchronize(stream));
-    std::memcpy(&host, dev_state->pinned, kHeaderRead);
+    auto big_maxcol = [&]() -> dtc_status_t {
+      k_big_maxcol<<<1024, 256, 0, stream>>>(node_pointer, edge_list, num_nodes, nnz, blk_h,
+                                             big_list, ws.csb, ws.tb, ws.tw, sort_tile, ws.hdr);
+      DTC_LAUNCH_CHECK("big_maxcol");
+      k_report<<<1, 64, 0, stream>>>(ws.hdr, report);
+      DTC_LAUNCH_CHECK("report");
+      return DTC_SUCCESS;
+    };
+    auto read = [&]() -> dtc_status_t {
+      DTC_HIP_CHECK(hipStreamSynchronize(stream));
+      std::memcpy(&host, dev_state->pinned, kHeaderRead);
+      return DTC_SUCCESS;
+    };
+    if (W <= kOnePlanWindows) {
+      k_plan<<<1, 1024, 0, stream>>>(node_pointer, num_nodes, nnz, (int32_t)W, blk_h, mode,
+                                     block_partition, edge_list, ws.lists, row_window_offset,
+                                     sort_tile, ws.csb, ws.tb, ws.tw, ws.hdr, report);
+      DTC_LAUNCH_CHECK("plan");
+      st = read();
+      if (st == DTC_SUCCESS && !host.flags && host.cls_count[kClasses] > 0) {
+        st = big_maxcol();
+        if (st == DTC_SUCCESS) st = read();
+      }
+    } else {
+      k_header_init<<<1, 64, 0, stream>>>(ws.hdr);
+      DTC_LAUNCH_CHECK("header_init");
+      // up to 1,024 workgroups for the row check, and one per 256 windows for
+      // the classes
+      const unsigned grid = (unsigned)std::max<int64_t>(
+          std::min<int64_t>(1024, grid_for(num_nodes, 256)), grid_for(W, 256));
+      k_check_classify<<<grid, 256, 0, stream>>>(node_pointer, num_nodes, nnz, (int32_t)W, blk_h,
+                                                 mode, block_partition, edge_list, ws.lists,
+                                                 row_window_offset, ws.hdr);
+      DTC_LAUNCH_CHECK("check_classify");
+      // offsets and sort tiles of up to kOneGroupWindows global-path windows
+      k_big_offsets<<<1, 1024, 0, stream>>>(node_pointer, num_nodes, blk_h, big_list, ws.hdr,
+                                            sort_tile, ws.csb, ws.tb, ws.tw);
+      DTC_LAUNCH_CHECK("big_offsets");
+      st = big_maxcol();
+      if (st == DTC_SUCCESS) st = read();
+    }
   }
+  if (st != DTC_SUCCESS) return st;
   int max_col = 0;
   for (int c = 0; c < kMaxSlots; ++c) max_col = std::max(max_col, host.max_col[c]);
   if (host.flags) {
@@ -2226,7 +2324,7 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
   const int colbits = std::max(1, bits_for(max_col));
   const int n_big = host.cls_count[kClasses];
   const int nnz_big = host.nnz_big;
-  const int32_t *wmap = ws.lists + (int64_t)kClasses * W;
+  const int32_t *wmap = big_list;
 
   // 2. The global path goes to the side stream when the LDS path also has
   //    work.  Issue order: the global path's keys, the two largest LDS
@@ -2236,13 +2334,16 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
   //    launches on the other.
   int n_lds = 0;
   for (int c = 0; c < kClasses; ++c) n_lds += host.cls_count[c];
+  //    (The caller's stream is idle here, so there is nothing that the side
+  //    stream would have to wait for.)  The lock keeps other builds on this
+  //    device off the side stream until the join.
+  std::unique_lock<std::mutex> side_lock(dev_state->mu, std::defer_lock);
   SideStream *side = nullptr;
   hipStream_t gs = stream;
   if (nnz_big > 0 && n_lds > 0 && !one_stream()) {
+    side_lock.lock();
     side = dev_state;
     gs = side->s;
-  } else {
-    side_lock.unlock();
   }
   // 3. Global path, first steps (issued before the LDS path so that the
   //    side stream starts at once): window offsets and sort tiles of many
@@ -2387,17 +2488,19 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
   int32_t T = 0;
   bool missed = false;
   for (bool again = true; again;) {
-    st = scan_i32(block_partition, row_window_offset + 1, W, true, ws.tmp, stream);
-    if (st != DTC_SUCCESS) return st;
-    k_chunk_windows<<<grid_for(W, 256), 256, 0, stream>>>(row_window_offset, (int32_t)W, ws.cw,
-                                                           ws.cw + ws.cw_stride);
-    DTC_LAUNCH_CHECK("chunk_windows");
     {
       std::lock_guard<std::mutex> g(dev_state->read_mu);
-      DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned, ws.hdr, kHeaderRead, hipMemcpyDeviceToHost,
-                                   stream));
-      DTC_HIP_CHECK(hipMemcpyAsync(dev_state->pinned + kHeaderRead, row_window_offset + W,
-                                   sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+      if (W <= kOneScanWindows) {
+        k_window_offsets<<<1, 1024, 0, stream>>>(block_partition, (int32_t)W, row_window_offset,
+                                                 ws.cw, ws.cw + ws.cw_stride, ws.hdr, report);
+        DTC_LAUNCH_CHECK("window_offsets");
+      } else {
+        st = scan_i32(block_partition, row_window_offset + 1, W, true, ws.tmp, stream);
+        if (st != DTC_SUCCESS) return st;
+        k_chunk_windows<<<grid_for(W, 256), 256, 0, stream>>>(
+            row_window_offset, (int32_t)W, ws.cw, ws.cw + ws.cw_stride, ws.hdr, report);
+        DTC_LAUNCH_CHECK("chunk_windows");
+      }
       DTC_HIP_CHECK(hipStreamSynchronize(stream));
       std::memcpy(&host, dev_state->pinned, kHeaderRead);
       std::memcpy(&T, dev_state->pinned + kHeaderRead, sizeof(int32_t));

@@ -151,3 +151,30 @@ def test_negative_column_inside_a_row(ext, monkeypatch):
     rowptr, col = csr(rows)
     with pytest.raises(RuntimeError, match="negative column"):
         gpu_metcf(ext, rowptr, col, 16, 16, 8)
+
+
+@pytest.mark.parametrize("windows", [1, 64, 1023, 1024, 1025, 4095, 4096, 4097])
+def test_window_counts(ext, monkeypatch, windows):
+    """Builds at the edges of the one-workgroup plan (1,024 windows) and of the
+    one-workgroup offsets (4,096), with empty windows, a last window of one row,
+    one window of each LDS class and one beyond them."""
+    monkeypatch.setenv("DTC_METCF_PATH", "auto")
+    rng = np.random.default_rng(windows)
+    M = windows * 16 - 15
+    rows = [np.sort(rng.choice(60000, n, replace=False)) for n in rng.integers(0, 3, M)]
+    for i in range(min(windows, 200)):  # empty windows
+        w = int(rng.integers(0, windows))
+        rows[w * 16:w * 16 + 16] = [[] for _ in rows[w * 16:w * 16 + 16]]
+    for n in (300, 1500, 3000, 7000, 15000, 40000):
+        rows[int(rng.integers(0, M))] = np.sort(rng.choice(60000, n, replace=False))
+    check(ext, rows, f"{windows} windows")
+
+
+@pytest.mark.parametrize("windows", [40, 2000])
+def test_row_pointer_beyond_the_edges(ext, windows):
+    """A row pointer that would put a window's entries far outside the edge
+    arrays is refused before anything reads them."""
+    rowptr = np.arange(windows * 16 + 1, dtype=np.int32)
+    rowptr[100] = 2_000_000_000
+    with pytest.raises(RuntimeError, match="nodePointer decreases"):
+        gpu_metcf(ext, rowptr, np.zeros(windows * 16, np.int32), windows * 16, 16, 8)
