@@ -97,6 +97,7 @@ struct SpmmParams {
   float *parts;        // balanced, deterministic merge: partial-tile slots (NULL: atomics)
   int32_t span;        // balanced cut span in TC blocks (a multiple of chunk)
   int32_t ct_blocks;   // workgroups per column tile when column tiles go one after another, 0: side by side
+  int32_t long_blocks; // unbalanced: windows of more blocks are shared out to the workgroup
 };
 
 // Kernels take the arrays as restrict-qualified arguments: the compiler may
@@ -111,7 +112,8 @@ struct SpmmParams {
   SpmmParams {                                                                             \
     a_rwo, a_rowid, a_tile, a_off, a_atox, a_vals, a_B, a_C, a_p.num_windows,              \
         a_p.num_blocks, a_p.M, a_p.b_rows, a_p.N, a_p.nnz, a_p.n_ct, a_p.num_items,        \
-        a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span, a_p.ct_blocks                                \
+        a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span, a_p.ct_blocks, \
+        a_p.long_blocks                                                                    \
   }
 
 template <int VEC>
@@ -869,17 +871,10 @@ __device__ __forceinline__ int window_start_from(const int32_t *rowid, int b, in
   return wave_lower_bound<int32_t>(rowid, 0, b - 64, w);
 }
 
-template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
+template <int PREC, int VEC, int NSUB, int MODE>
 __device__ __forceinline__ void run_unit(const SpmmParams &p, int item, int ct, float *lds) {
   floatx4 acc[NSUB][VEC];
-  if constexpr (!BALANCED) {
-    const int w0 = item * p.chunk;
-    const int w1 = min(w0 + p.chunk, p.num_windows);
-    // Offsets are clamped to the blocks actually passed in.
-    const int rwo = max(0, min(p.rwo[min(w0 + lane_id(), w1)], p.num_blocks));
-    const int end = __builtin_amdgcn_readlane(rwo, w1 - w0);
-    walk_blocks<PREC, VEC, NSUB, kWindows, MODE>(p, 0, end, w0, w1, rwo, ct, lds, -1, -1, acc);
-  } else {
+  {
     // The chunk's run and the windows it merges atomically were worked out
     // by the preparation kernel (k_balance_prep).
     const int2 r = p.runs[item];
@@ -909,39 +904,16 @@ constexpr int spmm_waves_per_eu() {
   return VEC * NSUB <= 2 ? 6 : VEC * NSUB == 4 ? 5 : 1;
 }
 
-// Workgroup i serves column tile i % n_ct: workgroups are dispatched to the
-// 8 XCDs round robin, so when n_ct divides 8 every XCD (and its L2) only
-// sees one column tile of B.  With ct_blocks set, the column tiles go one
-// after another instead (workgroup i serves tile i / ct_blocks): all XCDs
-// then gather from the same column slice of B at a time.
-template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
-__global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED>()))) void spmm_kernel(SPMM_KERNEL_ARGS) {
-  const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
-  __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
-  const int wave = wave_uniform(threadIdx.x >> 6);
-  const int ct = p.ct_blocks ? blockIdx.x / p.ct_blocks : blockIdx.x % p.n_ct;
-  const int group = p.ct_blocks ? blockIdx.x % p.ct_blocks : blockIdx.x / p.n_ct;
-  const int item = group * kWavesPerBlock + wave;
-  if (item >= p.num_items) return;
-  run_unit<PREC, VEC, NSUB, BALANCED, MODE>(p, item, ct, s_tile[wave]);
-}
-
-// Unbalanced schedule for launches that cannot fill the GPU: one workgroup
-// per (window, column tile), whose four waves take a quarter of the window's
-// groups each; their tiles are added through LDS in wave order (a fixed one:
-// the result stays repeatable).  A window's serial chain of gathers becomes a
-// quarter as long.
+// Window w by the workgroup's four waves: each takes a quarter of its groups,
+// and their tiles are added through LDS in wave order (a fixed one: the result
+// stays repeatable).  The window's serial chain of gathers becomes a quarter as
+// long.
 template <int PREC, int VEC, int NSUB, int MODE>
-__global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, false>()))) void spmm_kernel_split(SPMM_KERNEL_ARGS) {
-  const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
+__device__ __forceinline__ void split_window(const SpmmParams &p, int w, int ct,
+                                             float (*s_tile)[wave_lds_words<VEC, NSUB>()]) {
   constexpr int TW = 16 * VEC * NSUB;
-  __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   const int wave = wave_uniform(threadIdx.x >> 6);
   const int lane = lane_id();
-  const int ct = blockIdx.x % p.n_ct;
-  const int w = blockIdx.x / p.n_ct;  // the grid is n_ct * num_windows
   const int b1 = max(0, min(wave_uniform(p.rwo[w + 1]), p.num_blocks));
   const int b0 = max(0, min(wave_uniform(p.rwo[w]), b1));
   const int per = (b1 - b0 + kGroup * kWavesPerBlock - 1) / (kGroup * kWavesPerBlock) * kGroup;  // blocks per wave
@@ -974,6 +946,85 @@ __global__ __launch_bounds__(256) __attribute__((
   }
 }
 
+// The unbalanced schedule's unit: p.chunk consecutive windows per wave, except
+// those of more than p.long_blocks blocks, which the workgroup's four waves
+// then take together: one hub window is otherwise the whole launch (R-MAT of
+// 761,088 rows, N = 48: a window of 5,585 blocks at 0.29 us each).
+template <int PREC, int VEC, int NSUB, int MODE>
+__device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int ct,
+                                            float (*s_tile)[wave_lds_words<VEC, NSUB>()], uint32_t *s_long) {
+  const int wave = wave_uniform(threadIdx.x >> 6);
+  const int lane = lane_id();
+  const int g0 = group * kWavesPerBlock * p.chunk;  // the workgroup's windows (g0 < num_windows)
+  const int g1 = min(g0 + kWavesPerBlock * p.chunk, p.num_windows);
+  const int w0 = min(g0 + wave * p.chunk, g1);
+  const int w1 = min(w0 + p.chunk, g1);
+  // Lane l (at most 32): start of window w0 + l; lanes 62 and 63: the
+  // workgroup's first block and end.  Offsets are clamped to the blocks
+  // actually passed in.
+  int rwo = max(0, min(p.rwo[lane == 62 ? g0 : lane == 63 ? g1 : min(w0 + lane, w1)], p.num_blocks));
+  const bool any_long =
+      __builtin_amdgcn_readlane(rwo, 63) - __builtin_amdgcn_readlane(rwo, 62) > p.long_blocks;
+  uint32_t longs = 0;  // this wave's long windows, a bit each
+  if (any_long) {
+    const int blocks = __shfl_down(rwo, 1, 64) - rwo;
+    longs = (uint32_t)__ballot(w0 + lane < w1 && blocks > p.long_blocks);
+  }
+  if (any_long && lane == 0) s_long[wave] = longs;
+  floatx4 acc[NSUB][VEC];
+  for (int a = w0; a < w1;) {
+    const int n = min(w1 - a, longs ? (int)__builtin_ctz(longs) : 32);  // windows up to the next long one
+    if (n > 0)
+      walk_blocks<PREC, VEC, NSUB, kWindows, MODE>(p, 0, __builtin_amdgcn_readlane(rwo, n), a, a + n, rwo, ct,
+                                                   s_tile[wave], -1, -1, acc);
+    if (!longs) break;
+    a += n + 1;
+    longs = n + 1 < 32 ? longs >> (n + 1) : 0;
+    rwo = __shfl(rwo, lane + n + 1, 64);
+  }
+  if (!any_long) return;  // workgroup-uniform
+  __syncthreads();
+  for (int v = 0; v < kWavesPerBlock; ++v) {
+    for (uint32_t m = wave_uniform((int)s_long[v]); m; m &= m - 1) {
+      split_window<PREC, VEC, NSUB, MODE>(p, g0 + v * p.chunk + (int)__builtin_ctz(m), ct, s_tile);
+      __syncthreads();  // its tiles are read
+    }
+  }
+}
+
+// Workgroup i serves column tile i % n_ct: workgroups are dispatched to the
+// 8 XCDs round robin, so when n_ct divides 8 every XCD (and its L2) only
+// sees one column tile of B.  With ct_blocks set, the column tiles go one
+// after another instead (workgroup i serves tile i / ct_blocks): all XCDs
+// then gather from the same column slice of B at a time.
+template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED>()))) void spmm_kernel(SPMM_KERNEL_ARGS) {
+  const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
+  __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
+  const int wave = wave_uniform(threadIdx.x >> 6);
+  const int ct = p.ct_blocks ? blockIdx.x / p.ct_blocks : blockIdx.x % p.n_ct;
+  const int group = p.ct_blocks ? blockIdx.x % p.ct_blocks : blockIdx.x / p.n_ct;
+  if constexpr (BALANCED) {
+    const int item = group * kWavesPerBlock + wave;
+    if (item >= p.num_items) return;
+    run_unit<PREC, VEC, NSUB, MODE>(p, item, ct, s_tile[wave]);
+  } else {
+    __shared__ uint32_t s_long[kWavesPerBlock];
+    run_windows<PREC, VEC, NSUB, MODE>(p, group, ct, s_tile, s_long);
+  }
+}
+
+// Unbalanced schedule for launches that cannot fill the GPU: one workgroup
+// per (window, column tile).
+template <int PREC, int VEC, int NSUB, int MODE>
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, false>()))) void spmm_kernel_split(SPMM_KERNEL_ARGS) {
+  const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
+  __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
+  split_window<PREC, VEC, NSUB, MODE>(p, blockIdx.x / p.n_ct, blockIdx.x % p.n_ct, s_tile);  // grid: n_ct * num_windows
+}
+
 // Persistent variant of the balanced schedule: every wave pulls units from a
 // global counter until the list is exhausted.
 template <int PREC, int VEC, int NSUB, int MODE>
@@ -990,7 +1041,7 @@ __global__ __launch_bounds__(256) __attribute__((
     u = __shfl(u, 0, 64);
     u = wave_uniform(u);
     if (u >= total) break;
-    run_unit<PREC, VEC, NSUB, true, MODE>(p, u / p.n_ct, u % p.n_ct, s_tile[wave]);
+    run_unit<PREC, VEC, NSUB, MODE>(p, u / p.n_ct, u % p.n_ct, s_tile[wave]);
   }
 }
 
@@ -1365,6 +1416,16 @@ int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks) {
   return k;
 }
 
+// Blocks from which the unbalanced schedule shares a window out to a workgroup:
+// windows far longer than the others, whose chains would outlast the launch.
+// (R-MAT, us before and after: 761,088 rows, N = 48, longest window 5,585
+// blocks 1,840 -> 1,320; 262,144, N = 128 1,470 -> 910; 100,000, N = 32 621 ->
+// 288; 20,000, N = 64 196 -> 93.  Block model and band, whose windows are near
+// their average, are unchanged.)
+int32_t long_window(int64_t windows, int64_t num_blocks) {
+  return (int32_t)std::min<int64_t>(std::max<int64_t>(128, 8 * num_blocks / windows), INT32_MAX);
+}
+
 // Workgroups per column tile when the column tiles go one after another, 0
 // when they go side by side.  B beyond the 256 MB memory-side cache: one
 // slice at a time, so that most of its gathers hit there.
@@ -1661,6 +1722,7 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   p.chunk = split ? 1 : windows_per_unit(W, p.n_ct, num_blocks);
   p.num_items = (int32_t)ceil_div(W, p.chunk);
   p.ct_blocks = split ? 0 : column_order(p, esz);
+  p.long_blocks = long_window(W, num_blocks);
   KernelFn fn = pick_kernel(var, split ? kRunSplit : kRunWindows);
   const int64_t grid = (int64_t)p.n_ct * (split ? W : ceil_div(p.num_items, kWavesPerBlock));
   if (grid > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "grid too large");

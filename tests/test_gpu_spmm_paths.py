@@ -79,3 +79,20 @@ def test_several_windows_per_wave():
     lengths[1600:4800] = 0
     lengths[-21:] = 2
     check(*random_csr(rng, rows, 500, lengths), 500, 260, "windows")
+
+
+@pytest.mark.parametrize("n", [16, 33, 64, 96, 320])
+@pytest.mark.parametrize("windows", [2301, 40000])
+def test_long_windows(n, windows):
+    """Hub windows among short ones (several short ones per wave at 40,000
+    windows): below, at and above the 128 blocks from which a workgroup shares
+    a window, neighbours, the first and the last window."""
+    rng = np.random.default_rng(windows + n)
+    cols = 3000 if windows < 10000 else 1300
+    rows = windows * 16 - 3
+    lengths = rng.integers(0, 2, rows)
+    lengths[16 * 8:16 * 10] = 0
+    for w, blocks in ((0, 160), (5, 127), (20, 128), (21, 129), (22, 130), (40, 132), (41, 160), (windows - 1, 159)):
+        lengths[16 * w:16 * (w + 1)] = 0
+        lengths[min(16 * w + 7, rows - 1)] = 8 * blocks - 3
+    check(*random_csr(rng, rows, cols, lengths), cols, n, "windows")
