@@ -1340,10 +1340,10 @@ int operand_mode(int64_t b_rows, int64_t n, int64_t esz, int64_t nnz, int64_t nu
 // Kernel scheme and lane shape from the options, N and operand alignment.  An
 // explicit vec must divide N and the base addresses; vec 0 takes any N of at
 // least its width (unaligned vectors, the last lanes moved back: lane_cols).
-// vec 0 for float32 B: 2 floats per lane (32-column tiles) in the balanced
-// schedule, 4 in the unbalanced one, less where N is narrower.
+// vec 0 for float32 B: 4 floats per lane (64-column tiles), less where N is
+// narrower.
 dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void *b, const float *c,
-                           bool balanced, int mode, Variant *out) {
+                           bool balanced, bool dense, int mode, Variant *out) {
   const bool wide = mode == kPtr;
   const int prec = opt ? opt->precision : DTC_PRECISION_FP32;
   const int bdt = opt ? opt->b_dtype : DTC_B_FLOAT32;
@@ -1384,10 +1384,16 @@ dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void 
                 "vec " + std::to_string(vec) + " needs N and the B/C base addresses to be multiples of it");
   if (vec == 0) {
     vec = n <= 16 ? 1 : n <= 32 ? 2 : 4;
-    // 128-column tiles (two 64-column subtiles) where 64-column ones would
-    // leave half of the last one empty, and for wide B in the unbalanced
-    // schedule
-    if (nsub == 0) nsub = (n % 128 > 64 && n % 128 <= 96) || (!balanced && n > 256) ? 2 : 1;
+    // Where 64-column tiles would leave half of the last one empty: one of 128
+    // (two subtiles) in the unbalanced schedule and for dense blocks (each tile
+    // builds its A again), else three of 32 in the balanced one (N = 96, us: 46,000
+    // blocks 40 against 47 and 55, 157,000 96 / 108 / 121, 1.08 M 476 / 526 / 539;
+    // block model of 958,000 blocks of 13 382 / 397 / 372, band of 55 a block 66 and
+    // 60).  128-column tiles also
+    // for wide B in the unbalanced schedule.
+    const bool half = n % 128 > 64 && n % 128 <= 96;
+    if (nsub == 0 && balanced && half && n < 128 && !dense) vec = 2;
+    if (nsub == 0) nsub = (half && (!balanced || dense)) || (!balanced && n > 256) ? 2 : 1;
   }
   if (wide) vec = n >= 4 ? 4 : 1;
   if (nsub == 0 || wide || vec != 4) nsub = 1;
@@ -1458,13 +1464,38 @@ dtc_status_t check_common(const uint8_t *tile, const int32_t *off, const int32_t
   return DTC_SUCCESS;
 }
 
-// Default balanced chunk, in TC blocks: short chunks leave enough units on
-// small matrices, long ones cut fewer windows and start fewer units.
-int default_chunk_blocks(int32_t num_blocks) {
-  if (num_blocks < (1 << 15)) return 16;
-  if (num_blocks < (1 << 18)) return 32;
-  if (num_blocks < (1 << 21)) return 64;
-  return num_blocks < 6 * (1 << 20) ? 128 : 256;
+// Longest default of a balanced chunk, in TC blocks: the one that a cut span is
+// measured against, and the one for a fixed workspace that short chunks exceed.
+int long_chunk_blocks(int32_t num_blocks) {
+  int c = 32;
+  while (c < 512 && (int64_t)c * 2 * 8192 <= (int64_t)num_blocks) c *= 2;
+  return c;
+}
+
+// Balanced chunk: options->chunk_blocks, or with 0 the power of two in [8, 256]
+// that leaves some 550 * chunk units (chunks x 64-column tiles): a small launch
+// is as long as one unit's chain, a large one pays for every unit's start and
+// every cut window's merge.  Best and next chunks measured, us, R-MAT: 4,100
+// blocks, N = 64 (8) 15 (16) 21; 18,700, N = 48 (8) 22 (32) 25, N = 192 (32) 33
+// (16) 35; 46,000, N = 48 (16) 34 (32) 43, N = 256 (32) 70 (16) 73; 157,000, N =
+// 64 (32) 71 (16) 77, N = 256 (64) 179 (32) 187; 432,000, N = 32 (32) 98 (64)
+// 108, N = 128 (64) 240 (32) 246; 1.08 M, N = 128 (64) 565 (128) 586; block model
+// of 958,000 blocks, N = 256 (128) 761 (64) 825.
+// Dense blocks take longer chunks (more work a block, and windows of one length,
+// most of which a short chunk cuts in two): half as many units per chunk beyond
+// 11 entries a block, and beyond 24 at least 32 blocks unless the launch is small.
+// Block model of 99,700 blocks of 12.5, N = 64, (32) 46 (16) 50; band of 55 a
+// block, 53,000 blocks, N = 64 (32) 37 (16) 44, 106,000, N = 256 (32) 164 (64)
+// 187, 8,750, N = 128 (8) 19.6 (16) 21.3.
+// nnz 0: not known, the shortest chunk it could be.
+int resolve_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n) {
+  if (opt && opt->chunk_blocks > 0) return opt->chunk_blocks;
+  if (opt && opt->cut_span_blocks != 0) return long_chunk_blocks(num_blocks);
+  const bool dense = nnz > 24 * (int64_t)num_blocks;
+  const int64_t k = !dense && nnz > 11 * (int64_t)num_blocks ? 275 : 550;
+  int c = dense && num_blocks >= 1 << 15 ? 32 : 8;
+  while (c < 256 && (int64_t)num_blocks * ceil_div(std::max(n, 1), 64) > k * c * c) c *= 2;
+  return c;
 }
 
 // Cut span of the balanced schedule: options->cut_span_blocks, a positive
@@ -1644,7 +1675,7 @@ dtc_status_t dtc_spmm_tcgnn(const int32_t *node_pointer, const int32_t *edge_lis
   o.vec = options ? options->vec : 0;
   o.subtiles = 1;
   Variant var;
-  dtc_status_t st = resolve_shape(&o, n, b, c, false, kBuf, &var);
+  dtc_status_t st = resolve_shape(&o, n, b, c, false, false, kBuf, &var);
   if (st != DTC_SUCCESS) return st;
   const int32_t W = (int32_t)ceil_div(num_nodes, kBlkH);
   if (b_rows == 0) return zero_output(c, num_nodes, n, stream);
@@ -1697,7 +1728,7 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   Variant var;
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
-  st = resolve_shape(options, n, b, c, false, mode, &var);
+  st = resolve_shape(options, n, b, c, false, false, mode, &var);
   if (st != DTC_SUCCESS) return st;
   // Only windows that hold output rows are processed.
   const int32_t W = (int32_t)std::min<int64_t>(num_windows, ceil_div(num_nodes, kBlkH));
@@ -1749,8 +1780,7 @@ dtc_status_t dtc_spmm_balanced_workspace_size_ex(int32_t num_blocks, int32_t n,
   if (options && options->chunk_blocks < 0)
     return fail(DTC_ERROR_INVALID_VALUE, "chunk_blocks must be >= 0");
   const bool det = options && options->deterministic;
-  const int chunk = (options && options->chunk_blocks > 0) ? options->chunk_blocks
-                                                           : default_chunk_blocks(num_blocks);
+  const int chunk = resolve_chunk(options, num_blocks, 0, n);
   *bytes = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
   return DTC_SUCCESS;
 }
@@ -1771,10 +1801,9 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   Variant var;
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
-  st = resolve_shape(options, n, b, c, true, mode, &var);
+  st = resolve_shape(options, n, b, c, true, nnz > (num_blocks >= (1 << 19) ? 11 : 24) * (int64_t)num_blocks, mode, &var);
   if (st != DTC_SUCCESS) return st;
-  const int chunk = (options && options->chunk_blocks > 0) ? options->chunk_blocks
-                                                           : default_chunk_blocks(num_blocks);
+  const int chunk = resolve_chunk(options, num_blocks, nnz, n);
   int span = chunk;
   st = resolve_cut_span(options, chunk, &span);
   if (st != DTC_SUCCESS) return st;
@@ -1861,9 +1890,15 @@ dtc_status_t dtc_spmm_balanced_noalloc(const int32_t *tcblock_rowid, const uint8
   if (options && options->chunk_blocks < 0)
     return fail(DTC_ERROR_INVALID_VALUE, "chunk_blocks must be >= 0");
   const bool det = options && options->deterministic;
-  const int chunk = (options && options->chunk_blocks > 0) ? options->chunk_blocks
-                                                           : default_chunk_blocks(num_blocks);
-  const size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
+  dtc_spmm_options_t o{};
+  if (options) o = *options;
+  int chunk = resolve_chunk(options, num_blocks, nnz, n);
+  size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
+  if (need > kNoAllocScratchBytes && o.chunk_blocks == 0) {
+    chunk = std::max(chunk, long_chunk_blocks(num_blocks));
+    need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
+  }
+  o.chunk_blocks = chunk;
   if (need > kNoAllocScratchBytes)
     return fail(DTC_ERROR_UNSUPPORTED,
                 "this SpMM needs " + std::to_string(need) + " bytes of workspace, more than the " +
@@ -1873,7 +1908,7 @@ dtc_status_t dtc_spmm_balanced_noalloc(const int32_t *tcblock_rowid, const uint8
   dtc_status_t st = noalloc_scratch(&ws);
   if (st != DTC_SUCCESS) return st;
   return dtc_spmm_balanced(tcblock_rowid, tcblocktile_id, tcblock_offset, sparse_atox, tcblock_values,
-                           num_blocks, nnz, num_nodes, b, b_rows, n, c, options, ws, kNoAllocScratchBytes,
+                           num_blocks, nnz, num_nodes, b, b_rows, n, c, &o, ws, kNoAllocScratchBytes,
                            stream);
 }
 

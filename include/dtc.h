@@ -54,13 +54,15 @@ typedef enum dtc_b_dtype {
 typedef struct dtc_spmm_options {
   int32_t precision;    /* dtc_precision_t */
   int32_t vec;          /* B elements per lane per gathered row: 1, 2, 4 (float32 B);
-                           4, 8 (bfloat16 B); 0 = float32 B: 2 (balanced) or 4
-                           (unbalanced), narrower where N or the alignment need it;
-                           bfloat16 B: 8 (balanced; 4 where N or the alignment need
-                           it) or 4 (unbalanced) */
-  int32_t subtiles;     /* 1 or 2 column tiles of 16*vec per wave (0 = 1; float32 B) */
-  int32_t chunk_blocks; /* balanced schedule: TC blocks per work chunk (0 = the largest
-                           power of two in [32, 512] at most num_blocks / 8192) */
+                           4, 8 (bfloat16 B); 0 = float32 B: 4, less for N <= 32 and
+                           for some N <= 96 of the balanced schedule, any N and
+                           alignment; bfloat16 B: 8 for N > 64, else 4 */
+  int32_t subtiles;     /* 1 or 2 column tiles of 16*vec per wave (0 = chosen from N;
+                           float32 B) */
+  int32_t chunk_blocks; /* balanced schedule: TC blocks per work chunk (0 = a power of two
+                           in [8, 256] that grows with num_blocks and N; with
+                           cut_span_blocks the largest power of two in [32, 512] at most
+                           num_blocks / 8192) */
   int32_t persistent;   /* balanced schedule: 1 = persistent waves pulling chunks from a queue */
   int32_t b_dtype;      /* dtc_b_dtype_t */
   int32_t deterministic; /* balanced schedule: 1 = windows cut across chunks are merged in a
@@ -184,8 +186,9 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
  * workspace (required when num_blocks > 0) holds each chunk's block run,
  * worked out by a preparation kernel, the work counter of the persistent
  * variant and, with options->deterministic, the partial tiles; its size is
- * dtc_spmm_balanced_workspace_size_ex for these options and N (exactly
- * 256 + 8 * ceil(num_blocks / chunk) bytes without the deterministic merge),
+ * dtc_spmm_balanced_workspace_size_ex for these options and N
+ * (256 + 8 * ceil(num_blocks / chunk) bytes without the deterministic merge;
+ * for the default chunk, the shortest that num_blocks and N can have),
  * or dtc_spmm_balanced_workspace_size (256 + 8 * num_blocks bytes, enough for
  * any chunk size without the deterministic merge).
  */

@@ -96,3 +96,42 @@ def test_long_windows(n, windows):
         lengths[16 * w:16 * (w + 1)] = 0
         lengths[min(16 * w + 7, rows - 1)] = 8 * blocks - 3
     check(*random_csr(rng, rows, cols, lengths), cols, n, "windows")
+
+
+@pytest.mark.parametrize("n", [48, 64, 65, 96, 97, 224])
+@pytest.mark.parametrize("blocks", [8800, 8801, 17600, 17601, 35200, 35201])
+def test_default_chunks(n, blocks):
+    """Balanced runs with the default chunk and lane shape, at block counts
+    where the chunk doubles from 8 to 16 for four, two and one 64 columns."""
+    rng = np.random.default_rng(blocks + n)
+    rows = 16 * (blocks // 4)
+    lengths = np.zeros(rows, np.int64)
+    lengths[::16] = 25  # four blocks a window
+    lengths[16 * 3] = 24 + 8 * (blocks % 4) + 1
+    check(*random_csr(rng, rows, 400, lengths), 400, n, "balanced")
+
+
+def test_noalloc_default_chunk():
+    """The allocation-free entry point with the default chunk: the ordered merge
+    of 12,000 blocks at N = 128 exceeds its scratch in chunks of 8 and fits it in
+    chunks of 32."""
+    from dtc.capi import Library
+    from dtc.matrix import DTCMatrix
+    lib = Library()
+    rng = np.random.default_rng(8)
+    rows, n = 16 * 3000, 128
+    lengths = np.zeros(rows, np.int64)
+    lengths[::16] = 32
+    rowptr, col, values = random_csr(rng, rows, 400, lengths)
+    A = DTCMatrix(rowptr, col, values, num_rows=rows, num_cols=400)
+    B = rng.standard_normal((400, n)).astype(np.float32)
+    C = torch.full((rows, n), float("nan"), device="cuda")
+    Bd = torch.from_numpy(B).cuda()
+    opt = lib.options(deterministic=True)
+    say("noalloc default chunk", A.block_count)
+    lib.spmm_balanced_noalloc(A.tcblock_rowid.data_ptr(), A.tcblocktile_id.data_ptr(), A.tcblock_offset.data_ptr(),
+                              A.sparse_atox.data_ptr(), A.values_tc.data_ptr(), A.block_count, A.nnz, rows,
+                              Bd.data_ptr(), 400, n, C.data_ptr(), options=opt,
+                              stream=torch.cuda.current_stream().cuda_stream)
+    exact, mag = oracle.spmm_csr_f64(rowptr, col, values, B, rows, with_abs=True)
+    assert np.all(np.abs(C.cpu().numpy() - exact) <= 36 * 2.0 ** -24 * mag)
