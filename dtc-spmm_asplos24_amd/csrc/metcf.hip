@@ -1678,16 +1678,20 @@ __global__ __launch_bounds__(256) void k_big_keys(const int32_t *rowptr, const i
 //                  columns;
 //   k_run_out      a run of 256 TC blocks: the blocks' occupancies in LDS,
 //                  the entries' places in TC-block order, the outputs.
-// 6.1 M entries in 137 windows of an R-MAT matrix of 2^20 rows: 61 + 76 + 95 us
-// alone, where keys, three passes of the segmented sort, its scan and the
-// passes after it took 760 us.  Bound by the latency of short pieces: a slice of
-// 2^16 columns holds 2,800 of these entries, a run 2,600.
+// 6.1 M entries in 137 windows of an R-MAT matrix of 2^20 rows: 42 + 80 + 115 us
+// beside the LDS path's kernels, where keys, three passes of the segmented sort,
+// its scan and the passes after it took 760 us.  Bound by the latency of short
+// pieces (a slice of 2^16 columns holds 2,800 of these entries, a run 2,600) and
+// by the longest one (85,000 entries): 1,024 threads a slice and four loads in
+// flight a thread instead of 512 and one, and nine workgroups a CU of the runs
+// instead of five, took the build from 651 to 636 us.
 constexpr int kSliceLog = 16;                       // columns of a slice
 constexpr int kSpanGroups = 1 << (kSliceLog - 7);    // 128-bit groups of it
-constexpr int kSpanThreads = 512;                   // one group per thread
+constexpr int kSpanThreads = 1024;
 constexpr int kRunBlocks = 256;                     // TC blocks of a run, one per thread
-constexpr int kRunStage = 8192;                     // entries staged at a time
-static_assert(kSpanGroups == kSpanThreads, "one group per thread");
+constexpr int kRunStage = 4096;                     // entries staged at a time
+constexpr int kFlight = 4;                          // entries of a thread in flight
+static_assert(kSpanGroups <= kSpanThreads && kSpanGroups % 64 == 0, "at most a group per thread");
 
 // Workspace of the three kernels (over the sort's buffers).
 struct SpanWs {
@@ -1740,6 +1744,28 @@ __device__ __forceinline__ void row_ranges(int *s_from, int *s_pre, int r, int l
   s_pre[r + 1] = inc;
 }
 
+// body(f, r, e, load(e)) for every entry f of a piece, the thread's next
+// kFlight loads issued together (clamped to the piece: past its end they repeat
+// its last entry); r is the entry's row in the window, e the entry.
+template <int NT, class Load, class Body>
+__device__ __forceinline__ void for_each_entry(const int *s_from, const int *s_pre, Load load, Body body) {
+  const int n = s_pre[kWinH];
+  for (int f0 = threadIdx.x; f0 < n; f0 += NT * kFlight) {
+    int r[kFlight], e[kFlight], v[kFlight];
+#pragma unroll
+    for (int k = 0; k < kFlight; ++k) {
+      const int f = min(f0 + k * NT, n - 1);
+      r[k] = row_of(s_pre, f);
+      e[k] = s_from[r[k]] + f - s_pre[r[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < kFlight; ++k) v[k] = load(e[k]);
+#pragma unroll
+    for (int k = 0; k < kFlight; ++k)
+      if (f0 + k * NT < n) body(f0 + k * NT, r[k], e[k], v[k]);
+  }
+}
+
 // One workgroup per slice of a window (grid: windows x slices).
 __global__ __launch_bounds__(kSpanThreads) void k_slice_mark(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int32_t M,
@@ -1749,9 +1775,9 @@ __global__ __launch_bounds__(kSpanThreads) void k_slice_mark(
   const int tid = threadIdx.x;
   const int wp = blockIdx.x / sw.slices, sl = blockIdx.x % sw.slices;
   const int w = wmap[wp];
-  s_bits[tid] = make_uint4(0, 0, 0, 0);
-  {
-    const int g = tid >> 4;  // 32 groups: 16 rows at the slice's first column and at its end
+  if (tid < kSpanGroups) s_bits[tid] = make_uint4(0, 0, 0, 0);
+  if (tid < 32 * 16) {  // 32 groups: 16 rows at the slice's first column and at its end
+    const int g = tid >> 4;
     const int64_t row = (int64_t)w * kWinH + (g & 15);
     const int r0 = rowptr[min(row, (int64_t)M)], r1 = rowptr[min(row + 1, (int64_t)M)];
     const int p = group_lower_bound(col, r0, r1, (int64_t)(sl + (g >> 4)) << kSliceLog);
@@ -1764,16 +1790,16 @@ __global__ __launch_bounds__(kSpanThreads) void k_slice_mark(
   }
   __syncthreads();
   unsigned *words = reinterpret_cast<unsigned *>(s_bits);
-  const int n = s_pre[kWinH];
-#pragma unroll 4
-  for (int f = tid; f < n; f += kSpanThreads) {
-    const int r = row_of(s_pre, f);
-    const uint32_t c = (uint32_t)col[s_from[r] + f - s_pre[r]] & ((1u << kSliceLog) - 1);
+  for_each_entry<kSpanThreads>(s_from, s_pre, [&](int e) { return col[e]; }, [&](int, int, int, int v) {
+    const uint32_t c = (uint32_t)v & ((1u << kSliceLog) - 1);
     atomicOr(&words[c >> 5], 1u << (c & 31));
-  }
+  });
   __syncthreads();
-  const uint4 m = s_bits[tid];
-  sw.bits[(int64_t)blockIdx.x * kSpanGroups + tid] = m;
+  uint4 m = make_uint4(0, 0, 0, 0);
+  if (tid < kSpanGroups) {
+    m = s_bits[tid];
+    sw.bits[(int64_t)blockIdx.x * kSpanGroups + tid] = m;
+  }
   const int sum = wave_sum(popc4(m));
   if ((tid & 63) == 0) s_sum[tid >> 6] = sum;
   __syncthreads();
@@ -1796,8 +1822,11 @@ __global__ __launch_bounds__(kSpanThreads) void k_slice_rank(
   const int tid = threadIdx.x;
   const int wp = blockIdx.x / sw.slices, sl = blockIdx.x % sw.slices;
   const int w = wmap[wp];
-  const uint4 m = sw.bits[(int64_t)blockIdx.x * kSpanGroups + tid];
-  s_bits[tid] = m;
+  uint4 m = make_uint4(0, 0, 0, 0);
+  if (tid < kSpanGroups) {
+    m = sw.bits[(int64_t)blockIdx.x * kSpanGroups + tid];
+    s_bits[tid] = m;
+  }
   int first = 0;  // distinct columns of the slices before this one
   for (int k = tid; k < sl; k += kSpanThreads) first += sw.count[(int64_t)wp * sw.slices + k];
   if (tid < kWinH) {
@@ -1819,7 +1848,7 @@ __global__ __launch_bounds__(kSpanThreads) void k_slice_rank(
     base += s_base[v];
   }
   run += base;  // rank of the group's first column
-  s_before[tid] = run;
+  if (tid < kSpanGroups) s_before[tid] = run;
   const int s = rowptr[(int64_t)w * kWinH];
   {
     int32_t *d = st.dcol + s + run;
@@ -1837,15 +1866,11 @@ __global__ __launch_bounds__(kSpanThreads) void k_slice_rank(
     st.wU[w] = base + total;
   }
   __syncthreads();
-  const int n = s_pre[kWinH];
-#pragma unroll 4
-  for (int f = tid; f < n; f += kSpanThreads) {
-    const int r = row_of(s_pre, f);
-    const int e = s_from[r] + f - s_pre[r];
-    const uint32_t c = (uint32_t)col[e] & ((1u << kSliceLog) - 1);
+  for_each_entry<kSpanThreads>(s_from, s_pre, [&](int e) { return col[e]; }, [&](int, int r, int e, int v) {
+    const uint32_t c = (uint32_t)v & ((1u << kSliceLog) - 1);
     e2r[e] = w * kWinH + r;
     e2c[e] = s_before[c >> 7] + popc_below(s_bits[c >> 7], (int)(c & 127));
-  }
+  });
 }
 
 // One workgroup per run of kRunBlocks TC blocks; a window of E entries has a
@@ -1902,13 +1927,11 @@ __global__ __launch_bounds__(kRunBlocks) void k_run_out(
   const uint32_t rank0 = (uint32_t)kb0 * kWinW;
   constexpr uint32_t kRankMask = kRunBlocks * kWinW - 1;  // ranks of the run, less rank0
   unsigned *words = reinterpret_cast<unsigned *>(s_occ);
-#pragma unroll 4
-  for (int f = tid; f < n; f += kRunBlocks) {
-    const int r = row_of(s_pre, f);
-    const uint32_t k = ((uint32_t)e2c[s_from[r] + f - s_pre[r]] - rank0) & kRankMask;
+  for_each_entry<kRunBlocks>(s_from, s_pre, [&](int e) { return e2c[e]; }, [&](int, int r, int, int v) {
+    const uint32_t k = ((uint32_t)v - rank0) & kRankMask;
     const uint32_t bit = (uint32_t)r * kWinW + k % kWinW;
     atomicOr(&words[k / kWinW * 4 + (bit >> 5)], 1u << (bit & 31));
-  }
+  });
   __syncthreads();
   {
     const int sum = popc4(s_occ[tid]);
@@ -1924,17 +1947,15 @@ __global__ __launch_bounds__(kRunBlocks) void k_run_out(
   __syncthreads();
   const int64_t out = (int64_t)s + s_start;
   for (int p0 = 0; p0 < n; p0 += kRunStage) {
-#pragma unroll 4
-    for (int f = tid; f < n; f += kRunBlocks) {
-      const int r = row_of(s_pre, f);
-      const uint32_t k = ((uint32_t)e2c[s_from[r] + f - s_pre[r]] - rank0) & kRankMask;
+    for_each_entry<kRunBlocks>(s_from, s_pre, [&](int e) { return e2c[e]; }, [&](int f, int r, int, int v) {
+      const uint32_t k = ((uint32_t)v - rank0) & kRankMask;
       const uint32_t bit = (uint32_t)r * kWinW + k % kWinW;
       const uint32_t p = (uint32_t)(s_before[k / kWinW] + popc_below(s_occ[k / kWinW], (int)bit) - p0);
       if (p < kRunStage) {
         s_f[p] = (uint16_t)f;
         s_tile[p] = (uint8_t)bit;
       }
-    }
+    });
     __syncthreads();
     const int len = min(n - p0, kRunStage);
 #pragma unroll 4
