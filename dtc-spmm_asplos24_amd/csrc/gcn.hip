@@ -12,10 +12,10 @@
 // The product is HBM-bound (X read once, B written once: 128 flop per byte at
 // K = F = 256, against MI355X's 2.5 PFLOP/s over 8 TB/s = 312), so the
 // kernel is built to read X once and keep W in L2:
-//   * a workgroup computes 128 rows x 256 columns: 4 waves, 64 columns each
-//     (4 MFMA column tiles), 8 row tiles of 16 each -- 128 accumulator VGPRs;
-//   * X's 128 rows are staged in LDS as bf16, 128 columns of K at a time
-//     (32 KB, rows padded by 16 bytes), shared by the four waves;
+//   * a workgroup computes 64 rows x 256 columns: 4 waves, 64 columns each
+//     (4 MFMA column tiles), 4 row tiles of 16 each -- 64 accumulator VGPRs;
+//   * X's 64 rows are staged in LDS as bf16, 128 columns of K at a time
+//     (16 KB, rows padded by 16 bytes), shared by the four waves;
 //   * W is packed once per call into MFMA fragment order (K/32 x F/16 groups
 //     of 64 lanes x 8 bf16), so each B fragment is one contiguous 1 KB read,
 //     served by L2 (W is 128 KB at K = F = 256);

@@ -778,7 +778,7 @@ __device__ __forceinline__ int bits_before(const uint4 *bits, ushort4 *before, i
 // takes 3 to 5 times the instructions: nine ballots a digit).  Kernel times on
 // an R-MAT matrix of 2^20 rows and 31.4 M entries, sorted before and now, for
 // windows of up to 512 / 2,048 / 4,096 / 8,192 / 16,384 entries: 95 -> 70,
-// 120 -> 55, 163 -> 66, 67 -> 21, 258 -> 90 us (the last three sorts ran beside
+// 120 -> 54, 163 -> 57, 67 -> 21, 258 -> 91 us (the last three sorts ran beside
 // the large windows').  The 32-column pieces are what makes the cost
 // independent of the span: bitmaps of 2^18 columns taken one after another
 // measured 119, 131, 40 and 157 us for the last four.  A span of 2^20 (one wave)
@@ -1678,8 +1678,8 @@ __global__ __launch_bounds__(256) void k_big_keys(const int32_t *rowptr, const i
 //                  columns;
 //   k_run_out      a run of 256 TC blocks: the blocks' occupancies in LDS,
 //                  the entries' places in TC-block order, the outputs.
-// 6.1 M entries in 137 windows of an R-MAT matrix of 2^20 rows: 42 + 80 + 115 us
-// beside the LDS path's kernels, where keys, three passes of the segmented sort,
+// 6.1 M entries in 137 windows of an R-MAT matrix of 2^20 rows: 44 + 79 + 86 us
+// alone, where keys, three passes of the segmented sort,
 // its scan and the passes after it took 760 us.  Bound by the latency of short
 // pieces (a slice of 2^16 columns holds 2,800 of these entries, a run 2,600) and
 // by the longest one (85,000 entries): 1,024 threads a slice and four loads in

@@ -65,8 +65,11 @@ VARIANTS = [
 
 
 def default_chunk_blocks(num_blocks: int) -> int:
-    """The library's balanced chunk when options leave it at 0: the largest
-    power of two in [32, 512] at most num_blocks / 8192 (csrc/spmm.hip)."""
+    """The longest chunk the library takes by default: the largest power of two
+    in [32, 512] at most num_blocks / 8192.  Options that leave the chunk at 0
+    give it with a cut span, and a shorter one otherwise that depends on N too
+    (csrc/spmm.hip); this one is stated wherever a chunk has to depend on the
+    block count alone (the selector's variants, the GCN layer's backward)."""
     c = 32
     while c < 512 and c * 2 * 8192 <= num_blocks:
         c *= 2
@@ -87,10 +90,10 @@ def default_schedule(max_window_blocks: int) -> str:
 
 
 def default_variant(num_blocks: int, max_window_blocks: int) -> int:
-    """Index in VARIANTS of what the library runs with default options (the
-    method without the selector): FP32, unbalanced with 64-column tiles when
-    no window is longer than AUTO_WINDOW_BLOCKS, else balanced with 32-column
-    tiles and the default chunk."""
+    """Index in VARIANTS of the fixed rule without the selector: FP32,
+    unbalanced with 64-column tiles when no window is longer than
+    AUTO_WINDOW_BLOCKS, else balanced with 32-column tiles and the chunk of
+    default_chunk_blocks."""
     if default_schedule(max_window_blocks) == "windows":
         return VARIANTS.index(("windows", "fp32", 0, 4, 1, False, 0))
     return VARIANTS.index(("balanced", "fp32", default_chunk_blocks(int(num_blocks)), 2, 1, False, 0))
