@@ -840,14 +840,15 @@ __global__ __launch_bounds__(64 * WAVES, ITEMS == 16 ? 4 : 6) void k_window_bits
   {
     int row = 0;                                     // rows started at or before the slot, less one
     int next = __builtin_amdgcn_readlane(rp, 1);     // start of row + 1
+    uint32_t last = prev_wave;                       // column of the entry before the slot's first
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const int q = vbase + k * 64 + lane;
       ix[k] = 0;
       if (vbase + k * 64 < E) {  // wave-uniform
         uint32_t before = __shfl_up(key[k], 1, 64);
-        if (lane == 0)
-          before = k > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)key[k > 0 ? k - 1 : 0], 63) : prev_wave;
+        if (lane == 0) before = last;
+        last = (uint32_t)__builtin_amdgcn_readlane((int)key[k], 63);  // (key[k] is made relative below)
         bool starts = q == 0;
         int r = row;
         while (row < kWinH - 1 && next < vbase + k * 64 + 64) {  // wave-uniform

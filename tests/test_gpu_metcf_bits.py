@@ -105,6 +105,31 @@ def test_left_to_the_sort(ext, monkeypatch, kind):
     check(ext, rows, kind)
 
 
+@pytest.mark.parametrize("kind", ["duplicate", "swap"])
+@pytest.mark.parametrize("first", [0, 1, 1000])
+@pytest.mark.parametrize("cls", [1, 2, 3, 4, 5])
+def test_defect_between_slots(ext, monkeypatch, cls, first, kind):
+    """Windows whose only duplicate, or only descent, lies between local entries
+    64 j - 1 and 64 j of one row, the two held by different slots of a lane or
+    by different waves, with a first column of 0 and above; among sorted ones."""
+    monkeypatch.setenv("DTC_METCF_PATH", "auto")
+    rng = np.random.default_rng(500 + cls)
+    cap = CAPS[cls]
+    per_wave = 64 * (16 if cls >= 4 else 8)  # entries of a wave
+    rows = []
+    # a wave's first and last boundary, the window's last, and (larger classes) waves' ends
+    for at in sorted({64, per_wave - 64, cap - 64} | ({per_wave, cap - per_wave} if cap > per_wave else set())):
+        # short rows around one that holds entries at - 40 .. at + 39
+        sizes = [(at - 40) // 8] * 7 + [(at - 40) // 8 + (at - 40) % 8] + [80] + [(cap - at - 40) // 7] * 7
+        w = [first + np.sort(rng.choice(1 << 14, n, replace=False)) for n in sizes]
+        if kind == "duplicate":
+            w[8][40] = w[8][39]
+        else:
+            w[8][[39, 40]] = w[8][[40, 39]]
+        rows += w + window(rng, cap - 3, 1 << 14, first=first)
+    check(ext, rows, f"class {cls} {kind} between slots, first {first}")
+
+
 @pytest.mark.parametrize("span", [16384, (1 << 16) - 1, 1 << 16, (1 << 16) + 1, 300000])
 def test_large_windows(ext, monkeypatch, span):
     """Windows beyond the LDS kernels: spans at the edges of a slice, full rows
