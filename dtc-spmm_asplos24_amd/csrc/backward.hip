@@ -308,6 +308,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAIL && NC 
   for (int e0 = first; e0 < last;) {
     int my_col, my_row;
     load_ids(e0, my_col, my_row);
+    // Edges (bit e - e0) with both rows: the others read zeros, which an
+    // infinity or a NaN on the other side turns into NaN, and get 0 at the store.
+    const uint64_t valid = __ballot((unsigned)my_col < (unsigned)y_rows && (unsigned)my_row < (unsigned)M);
     // Edges of this block: up to 64, fewer when their rows do not fit in LDS
     // (a multiple of a step's 4 U; with fewer than one step's, X is read per
     // edge).  Rows never decrease in a valid CSR; a block ends where they do.
@@ -397,8 +400,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TAIL && NC 
       if constexpr (U == 8) p[0] = (b1 ? p[1] : p[0]) + dpp_f32<kDppXor2>(b1 ? p[0] : p[1]);
       else p[0] += dpp_f32<kDppXor2>(p[0]);
       const float v = p[0] + dpp_f32<kDppXor1>(p[0]);
-      const int eo = e0 + (lane >> 4) * per + U * s + c / (16 / U);
-      if (c % (16 / U) == 0 && eo < e0 + count) out[eo] = v;
+      const int eo = (lane >> 4) * per + U * s + c / (16 / U);
+      if (c % (16 / U) == 0 && eo < count) out[e0 + eo] = (valid >> eo) & 1 ? v : 0.f;
     }
     e0 += count;
   }

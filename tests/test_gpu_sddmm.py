@@ -60,3 +60,37 @@ def test_bfloat16(shape, n):
 def test_rows_searched_and_short_y(n, dtype):
     run("mixed", n, dtype, False)
     run("mixed", n, dtype, True, y_rows=500)
+
+
+@pytest.mark.parametrize("shape", ["mixed", "single"])
+@pytest.mark.parametrize("n,dtype", [(4, torch.float32), (64, torch.float32), (65, torch.float32),
+                                     (128, torch.float32), (192, torch.float32), (193, torch.float32),
+                                     (8, torch.bfloat16), (128, torch.bfloat16), (256, torch.bfloat16),
+                                     (264, torch.bfloat16)])
+def test_columns_past_y_of_nonfinite_rows(shape, n, dtype):
+    """An edge whose column Y does not have gives 0 at every width, also where
+    its row of X holds infinities or NaN."""
+    from dtc import load_extension
+    ext = load_extension()
+    lengths = np.array(SHAPES[shape])
+    rng = np.random.default_rng(n)
+    M, y_rows = len(lengths), 300
+    rowptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(800, k, replace=False)) for k in lengths]).astype(np.int32)
+    row = np.repeat(np.arange(M), lengths).astype(np.int32)
+    Xn = rng.standard_normal((M, n)).astype(np.float32)
+    # rows whose edges are all past Y become non-finite
+    past = np.array([len(c) > 0 and (c >= y_rows).all() for c in np.split(col, rowptr[1:-1])])
+    Xn[past] = np.inf
+    Xn[np.flatnonzero(past)[::2], 0] = np.nan
+    X = torch.from_numpy(Xn).cuda()
+    Y = torch.from_numpy(rng.standard_normal((y_rows, n)).astype(np.float32)).to(dtype).cuda()
+    say("sddmm short y, non-finite x", shape, n, dtype, int(past.sum()))
+    assert past.any()
+    out = ext.sddmm_csr(torch.from_numpy(rowptr).cuda(), torch.from_numpy(col).cuda(), X, Y,
+                        torch.from_numpy(row).cuda()).cpu().numpy()
+    inside = col < y_rows
+    assert np.array_equal(out[~inside], np.zeros((~inside).sum(), np.float32))
+    a, b = Xn.astype(np.float64)[row], Y.double().cpu().numpy()[np.minimum(col, y_rows - 1)]
+    a[~inside] = b[~inside] = 0.0
+    assert np.all(np.abs(out - (a * b).sum(1)) <= (n + 4) * 2.0 ** -24 * np.abs(a * b).sum(1))
