@@ -98,6 +98,8 @@ struct SpmmParams {
   int32_t span;        // balanced cut span in TC blocks (a multiple of chunk)
   int32_t ct_blocks;   // workgroups per column tile when column tiles go one after another, 0: side by side
   int32_t long_blocks; // unbalanced: windows of more blocks are shared out to the workgroup
+  int32_t groups;      // unbalanced: workgroups per column tile
+  int32_t long_groups; // ... and of the launch's first part, which takes only long windows (0: no such part)
 };
 
 // Kernels take the arrays as restrict-qualified arguments: the compiler may
@@ -113,7 +115,7 @@ struct SpmmParams {
     a_rwo, a_rowid, a_tile, a_off, a_atox, a_vals, a_B, a_C, a_p.num_windows,              \
         a_p.num_blocks, a_p.M, a_p.b_rows, a_p.N, a_p.nnz, a_p.n_ct, a_p.num_items,        \
         a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span, a_p.ct_blocks, \
-        a_p.long_blocks                                                                    \
+        a_p.long_blocks, a_p.groups, a_p.long_groups                                       \
   }
 
 template <int VEC>
@@ -950,49 +952,92 @@ __device__ __forceinline__ void split_window(const SpmmParams &p, int w, int ct,
 // those of more than p.long_blocks blocks, which the workgroup's four waves
 // then take together: one hub window is otherwise the whole launch (R-MAT of
 // 761,088 rows, N = 48: a window of 5,585 blocks at 0.29 us each).
+//
+// With the column tiles one after another a hub window of the last tile would
+// start late and outlast the launch, so a first part of the launch
+// (p.long_groups workgroups a tile, the tiles side by side) takes the long
+// windows of all tiles, and the second the others (R-MAT of 2^20 rows and 31.4 M
+// entries, N = 128 4.54 -> 3.93 ms, 256 7.35 -> 5.74).  A workgroup of the first
+// part looks at kLongGroups groups (one each took 60 us of a 2.56 ms launch
+// without long windows, only to find none), one of each quarter: with group i of
+// the first quarter the i-th from the end of the others, which in a power-law
+// graph are light where it is heavy.
+constexpr int kLongGroups = 4;
 template <int PREC, int VEC, int NSUB, int MODE>
-__device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int ct,
+__device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int ct, bool long_part,
                                             float (*s_tile)[wave_lds_words<VEC, NSUB>()], uint32_t *s_long) {
   const int wave = wave_uniform(threadIdx.x >> 6);
   const int lane = lane_id();
-  const int g0 = group * kWavesPerBlock * p.chunk;  // the workgroup's windows (g0 < num_windows)
-  const int g1 = min(g0 + kWavesPerBlock * p.chunk, p.num_windows);
-  const int w0 = min(g0 + wave * p.chunk, g1);
-  const int w1 = min(w0 + p.chunk, g1);
-  // Lane l (at most 32): start of window w0 + l; lanes 62 and 63: the
-  // workgroup's first block and end.  Offsets are clamped to the blocks
-  // actually passed in.
-  int rwo = max(0, min(p.rwo[lane == 62 ? g0 : lane == 63 ? g1 : min(w0 + lane, w1)], p.num_blocks));
-  // (Not for dense blocks: their windows are near their average -- a hub row
-  // has one entry a column -- and the second walk's registers cost a band of
-  // 45,312 rows, bf16x6, N = 240 2%: 27.9 against 28.5 us.)
-  const bool any_long = MODE != kDense && __builtin_amdgcn_readlane(rwo, 63) -
-                                                  __builtin_amdgcn_readlane(rwo, 62) > p.long_blocks;
-  uint32_t longs = 0;  // this wave's long windows, a bit each
-  if (any_long) {
-    const int blocks = __shfl_down(rwo, 1, 64) - rwo;
-    longs = (uint32_t)__ballot(w0 + lane < w1 && blocks > p.long_blocks);
+  // first window of the workgroup's share v & 3 (a wave's chunk) of its group v / 4
+  auto first_window = [&](int v) {
+    const int g = v < kWavesPerBlock ? group : (v / kWavesPerBlock + 1) * p.long_groups - 1 - group;
+    return (g * kWavesPerBlock + v % kWavesPerBlock) * p.chunk;
+  };
+  auto blocks_before = [&](int w) { return max(0, min(p.rwo[min(w, p.num_windows)], p.num_blocks)); };
+  if (MODE == kDense || !long_part) {
+    const int g0 = group * kWavesPerBlock * p.chunk;  // the workgroup's windows (g0 < num_windows)
+    const int g1 = min(g0 + kWavesPerBlock * p.chunk, p.num_windows);
+    const int w0 = min(g0 + wave * p.chunk, g1);
+    const int w1 = min(w0 + p.chunk, g1);
+    // Lane l (at most 32): start of window w0 + l; lanes 62 and 63: the
+    // workgroup's first block and end.  Offsets are clamped to the blocks
+    // actually passed in.
+    int rwo = blocks_before(lane == 62 ? g0 : lane == 63 ? g1 : min(w0 + lane, w1));
+    // (Not for dense blocks: their windows are near their average -- a hub row
+    // has one entry a column -- and the second walk's registers cost a band of
+    // 45,312 rows, bf16x6, N = 240 2%: 27.9 against 28.5 us.)
+    const bool any_long = MODE != kDense && __builtin_amdgcn_readlane(rwo, 63) -
+                                                    __builtin_amdgcn_readlane(rwo, 62) > p.long_blocks;
+    uint32_t longs = 0;  // this wave's long windows, a bit each
+    if (any_long) {
+      const int blocks = __shfl_down(rwo, 1, 64) - rwo;
+      longs = (uint32_t)__ballot(w0 + lane < w1 && blocks > p.long_blocks);
+    }
+    if (any_long && lane == 0) s_long[wave] = longs;
+    floatx4 acc[NSUB][VEC];
+    for (int a = w0; a < w1;) {
+      const int n = min(w1 - a, longs ? (int)__builtin_ctz(longs) : 32);  // windows up to the next long one
+      if (n > 0)
+        walk_blocks<PREC, VEC, NSUB, kWindows, MODE>(p, 0, __builtin_amdgcn_readlane(rwo, n), a, a + n, rwo, ct,
+                                                     s_tile[wave], -1, -1, acc);
+      if (!longs) break;
+      a += n + 1;
+      longs = n + 1 < 32 ? longs >> (n + 1) : 0;
+      rwo = __shfl(rwo, lane + n + 1, 64);
+    }
+    if (!any_long || p.long_groups) return;  // workgroup-uniform
+  } else {
+#pragma unroll 1
+    for (int k = 0; k < kLongGroups; ++k) {
+      const int w = first_window(k * kWavesPerBlock + wave) + lane;
+      const uint64_t longs = __ballot(lane < p.chunk && blocks_before(w + 1) - blocks_before(w) > p.long_blocks);
+      if (lane == 0) s_long[k * kWavesPerBlock + wave] = (uint32_t)longs;
+    }
   }
-  if (any_long && lane == 0) s_long[wave] = longs;
-  floatx4 acc[NSUB][VEC];
-  for (int a = w0; a < w1;) {
-    const int n = min(w1 - a, longs ? (int)__builtin_ctz(longs) : 32);  // windows up to the next long one
-    if (n > 0)
-      walk_blocks<PREC, VEC, NSUB, kWindows, MODE>(p, 0, __builtin_amdgcn_readlane(rwo, n), a, a + n, rwo, ct,
-                                                   s_tile[wave], -1, -1, acc);
-    if (!longs) break;
-    a += n + 1;
-    longs = n + 1 < 32 ? longs >> (n + 1) : 0;
-    rwo = __shfl(rwo, lane + n + 1, 64);
-  }
-  if (!any_long) return;  // workgroup-uniform
   __syncthreads();
-  for (int v = 0; v < kWavesPerBlock; ++v) {
-    for (uint32_t m = wave_uniform((int)s_long[v]); m; m &= m - 1) {
-      split_window<PREC, VEC, NSUB, MODE>(p, g0 + v * p.chunk + (int)__builtin_ctz(m), ct, s_tile);
+  const int shares = long_part ? kLongGroups * kWavesPerBlock : kWavesPerBlock;
+  const int longs = (int)s_long[min(lane, shares - 1)];  // lane v: share v's
+  for (int v = 0; v < shares; ++v) {
+    for (uint32_t m = (uint32_t)__builtin_amdgcn_readlane(longs, v); m; m &= m - 1) {
+      split_window<PREC, VEC, NSUB, MODE>(p, first_window(v) + (int)__builtin_ctz(m), ct, s_tile);
       __syncthreads();  // its tiles are read
     }
   }
+}
+
+// Group g of `groups` for a workgroup that would take group g in turn, the
+// runs of 8 groups permuted: by the sum of the octal digits above the lowest.
+// Workgroups go to the 8 XCDs round robin, and in a power-law graph the work
+// falls with every bit set in a row's number, so groups in turn give one XCD
+// the heavy ones of all runs: of an R-MAT matrix of 2^20 rows and 31.4 M
+// entries 40% of the TC blocks go to one XCD and 1.7% to another in turn (18%
+// and 6% with four tiles side by side), 12.9% and 12.0% so.  N = 48 4.71 -> 3.51
+// ms, 128 8.45 -> 4.54, 256 16.4 -> 7.35.
+__device__ __forceinline__ int spread_group(int g, int groups) {
+  int turn = 0;
+#pragma unroll
+  for (int k = 3; k < 30; k += 3) turn += g >> k;  // (of which the low three bits count)
+  return (g | 7) < groups ? (g & ~7) | ((g + turn) & 7) : g;
 }
 
 // Workgroup i serves column tile i % n_ct: workgroups are dispatched to the
@@ -1006,15 +1051,22 @@ __global__ __launch_bounds__(256) __attribute__((
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
   __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   const int wave = wave_uniform(threadIdx.x >> 6);
-  const int ct = p.ct_blocks ? blockIdx.x / p.ct_blocks : blockIdx.x % p.n_ct;
-  const int group = p.ct_blocks ? blockIdx.x % p.ct_blocks : blockIdx.x / p.n_ct;
   if constexpr (BALANCED) {
+    const int ct = p.ct_blocks ? blockIdx.x / p.ct_blocks : blockIdx.x % p.n_ct;
+    const int group = p.ct_blocks ? blockIdx.x % p.ct_blocks : blockIdx.x / p.n_ct;
     const int item = group * kWavesPerBlock + wave;
     if (item >= p.num_items) return;
     run_unit<PREC, VEC, NSUB, MODE>(p, item, ct, s_tile[wave]);
   } else {
-    __shared__ uint32_t s_long[kWavesPerBlock];
-    run_windows<PREC, VEC, NSUB, MODE>(p, group, ct, s_tile, s_long);
+    __shared__ uint32_t s_long[kLongGroups * kWavesPerBlock];
+    const int long_wgs = MODE != kDense ? p.long_groups * p.n_ct : 0;
+    const bool long_part = (int)blockIdx.x < long_wgs;
+    const bool in_turn = p.ct_blocks && !long_part;
+    const unsigned at = blockIdx.x - (long_part ? 0 : long_wgs), per = in_turn ? p.ct_blocks : p.n_ct;
+    const int q = at / per, r = at % per;
+    const int ct = in_turn ? q : r;
+    const int group = spread_group(in_turn ? r : q, long_part ? p.long_groups : p.groups);
+    run_windows<PREC, VEC, NSUB, MODE>(p, group, ct, long_part, s_tile, s_long);
   }
 }
 
@@ -1758,7 +1810,9 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   p.ct_blocks = split ? 0 : column_order(p, esz);
   p.long_blocks = long_window(W, num_blocks);
   KernelFn fn = pick_kernel(var, split ? kRunSplit : kRunWindows);
-  const int64_t grid = (int64_t)p.n_ct * (split ? W : ceil_div(p.num_items, kWavesPerBlock));
+  p.groups = split ? W : (int32_t)ceil_div(p.num_items, kWavesPerBlock);
+  p.long_groups = p.ct_blocks && mode != kDense ? (int32_t)ceil_div(p.groups, kLongGroups) : 0;
+  const int64_t grid = (int64_t)p.n_ct * ((int64_t)p.groups + p.long_groups);
   if (grid > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "grid too large");
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, stream, p.rwo, p.rowid, p.tile, p.off,
                      p.atox, p.vals, p.B, p.C, p);

@@ -98,6 +98,28 @@ def test_long_windows(n, windows):
     check(*random_csr(rng, rows, cols, lengths), cols, n, "windows")
 
 
+@pytest.mark.parametrize("n,options", [(128, {}), (130, {}), (64, {"vec": 1}), (192, {"vec": 2})])
+@pytest.mark.parametrize("rows", [16 * 2301 - 3, 16 * 2304])
+def test_long_windows_wide_b(rows, n, options):
+    """B beyond 256 MB: the column tiles go one after another, the hub windows of
+    all tiles before the others; group counts that are and are not a multiple of
+    8 and of 4, hub windows in every quarter, next to each other and at both
+    ends."""
+    rng = np.random.default_rng(rows + n)
+    cols = (1 << 28) // (4 * n) + 1000
+    windows = -(-rows // 16)
+    lengths = rng.integers(0, 3, rows)
+    lengths[16 * 800:16 * 808] = 0
+    for w in (0, 1, 2, 3, 4, 575, 576, 1150, 1151, 1152, 1727, windows - 2, windows - 1):
+        lengths[min(16 * w + 7, rows - 1)] = 8 * 129 + w % 64
+    # rows with a hub's length pick from all of B's rows: distinct by construction
+    rowptr = np.zeros(rows + 1, np.int64)
+    rowptr[1:] = np.cumsum(lengths)
+    col = np.concatenate([np.sort((rng.integers(0, cols) + np.arange(k) * (cols // 1200)) % cols) for k in lengths])
+    values = rng.uniform(-1, 1, col.shape[0]).astype(np.float32)
+    check(rowptr.astype(np.int32), col.astype(np.int32), values, cols, n, "windows", **options)
+
+
 @pytest.mark.parametrize("n", [48, 64, 65, 96, 97, 224])
 @pytest.mark.parametrize("blocks", [8800, 8801, 17600, 17601, 35200, 35201])
 def test_default_chunks(n, blocks):
