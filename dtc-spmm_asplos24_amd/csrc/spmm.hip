@@ -1479,12 +1479,14 @@ int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks) {
 
 // Blocks from which the unbalanced schedule shares a window out to a workgroup:
 // windows far longer than the others, whose chains would outlast the launch.
-// (R-MAT, us before and after: 761,088 rows, N = 48, longest window 5,585
-// blocks 1,840 -> 1,320; 262,144, N = 128 1,470 -> 910; 100,000, N = 32 621 ->
-// 288; 20,000, N = 64 196 -> 93.  Block model and band, whose windows are near
-// their average, are unchanged.)
+// (us, none shared / from 16 / 8 / 4 times the average on: R-MAT of 16 a row,
+// 761,088 rows, N = 48 2,700 / 1,334 / 1,332 / 1,333; 262,144 of 32, N = 128
+// 2,018 / 1,199 / 1,179 / 1,188; 20,000 of 40, N = 64 264 / 215 / 152 / 142;
+// 25,568 of 40, N = 85 511 / 434 / 355 / 255; block model of 60,000 rows and hubs,
+// N = 128 714 / 715 / 683 / 446.  From 64 or 256 blocks on instead of 128: within
+// 1%.  Uniform matrices, whose windows are near their average, have none.)
 int32_t long_window(int64_t windows, int64_t num_blocks) {
-  return (int32_t)std::min<int64_t>(std::max<int64_t>(128, 8 * num_blocks / windows), INT32_MAX);
+  return (int32_t)std::min<int64_t>(std::max<int64_t>(128, 4 * num_blocks / windows), INT32_MAX);
 }
 
 // Workgroups per column tile when the column tiles go one after another, 0
