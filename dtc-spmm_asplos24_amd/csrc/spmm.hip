@@ -898,10 +898,15 @@ __device__ __forceinline__ void run_unit(const SpmmParams &p, int item, int ct, 
 // Waves per SIMD the compiler must leave room for (its register budget), per
 // instance: asked for these it keeps the accumulators out of the AGPRs and
 // spills nothing in the loop; left to itself it stops one or two waves short.
-// The bf16x3 and bf16x6 splits would spill and keep the default.
-template <int PREC, int VEC, int NSUB, bool BALANCED>
+// The unbalanced bf16x6 fits four (at three a band of 100,000 rows, N = 224, took
+// 50 us against 43, R-MAT of 262,144, N = 128, 902 against 832); the other bf16x3
+// and bf16x6 splits would spill and keep the default.  The balanced schedule over
+// dense blocks spills at five (the same band, N = 512, 107 us against 94 at four).
+template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
 constexpr int spmm_waves_per_eu() {
+  if (PREC == DTC_PRECISION_BF16X6 && !BALANCED && VEC * NSUB == 4) return 4;
   if (PREC == DTC_PRECISION_BF16X3 || PREC == DTC_PRECISION_BF16X6) return 1;
+  if (PREC == DTC_PRECISION_FP32 && BALANCED && MODE == kDense && VEC * NSUB == 4) return 4;
   if (is_bf16b<PREC>()) return VEC == 8 ? 4 : 5;
   return VEC * NSUB <= 2 ? 6 : VEC * NSUB == 4 ? 5 : 1;
 }
@@ -1047,7 +1052,7 @@ __device__ __forceinline__ int spread_group(int g, int groups) {
 // then gather from the same column slice of B at a time.
 template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
 __global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED>()))) void spmm_kernel(SPMM_KERNEL_ARGS) {
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED, MODE>()))) void spmm_kernel(SPMM_KERNEL_ARGS) {
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
   __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   const int wave = wave_uniform(threadIdx.x >> 6);
@@ -1074,7 +1079,7 @@ __global__ __launch_bounds__(256) __attribute__((
 // per (window, column tile).
 template <int PREC, int VEC, int NSUB, int MODE>
 __global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, false>()))) void spmm_kernel_split(SPMM_KERNEL_ARGS) {
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, false, MODE>()))) void spmm_kernel_split(SPMM_KERNEL_ARGS) {
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
   __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   split_window<PREC, VEC, NSUB, MODE>(p, blockIdx.x / p.n_ct, blockIdx.x % p.n_ct, s_tile);  // grid: n_ct * num_windows
@@ -1084,7 +1089,7 @@ __global__ __launch_bounds__(256) __attribute__((
 // global counter until the list is exhausted.
 template <int PREC, int VEC, int NSUB, int MODE>
 __global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, true>()))) void spmm_kernel_persistent(SPMM_KERNEL_ARGS) {
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, true, MODE>()))) void spmm_kernel_persistent(SPMM_KERNEL_ARGS) {
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
   __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   const int wave = wave_uniform(threadIdx.x >> 6);
