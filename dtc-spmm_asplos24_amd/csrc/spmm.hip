@@ -1475,9 +1475,16 @@ bool split_windows(int64_t windows, int64_t n_ct, int64_t num_blocks) {
 }
 
 // Consecutive windows per unit of the unbalanced schedule: short windows are
-// walked several to a wave, as one pipeline, while enough units remain.
-int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks) {
+// walked several to a wave, as one pipeline, while enough units remain.  For
+// tiles of up to 32 columns only, where a window is little work: wider ones lose
+// more by the longer chains, and in a band by rows of B that the workgroup's
+// waves no longer read at the same time.  us, one window and several: uniform
+// 2^20 rows of 4, N = 16 111 and 103, of 8, N = 32 194 and 188, of 4, N = 64 186
+// and 197; band of 19 columns half filled, 500,001 rows, N = 100 105 and 117, of
+// 25, 10^6 rows, N = 128 262 and 277; R-MAT of 2^20 rows of 4, N = 64 618 and 843.
+int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks, int32_t tile) {
   int32_t k = 1;
+  if (tile > 32) return k;
   while (k < 32 && 2 * k * num_blocks <= 32 * windows && windows * n_ct >= 2 * k * 16384) k *= 2;
   return k;
 }
@@ -1812,7 +1819,7 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   p.num_blocks = num_blocks;
   p.nnz = nnz;
   const bool split = split_windows(W, p.n_ct, num_blocks);
-  p.chunk = split ? 1 : windows_per_unit(W, p.n_ct, num_blocks);
+  p.chunk = split ? 1 : windows_per_unit(W, p.n_ct, num_blocks, 16 * var.vec * var.nsub);
   p.num_items = (int32_t)ceil_div(W, p.chunk);
   p.ct_blocks = split ? 0 : column_order(p, esz);
   p.long_blocks = long_window(W, num_blocks);
