@@ -96,10 +96,9 @@ struct SpmmParams {
   const int2 *runs;    // balanced: run [b, e) of every chunk, cut flags in the sign bits
   float *parts;        // balanced, deterministic merge: partial-tile slots (NULL: atomics)
   int32_t span;        // balanced cut span in TC blocks (a multiple of chunk)
-  int32_t ct_blocks;   // workgroups per column tile when column tiles go one after another, 0: side by side
   int32_t long_blocks; // unbalanced: windows of more blocks are shared out to the workgroup
-  int32_t groups;      // unbalanced: workgroups per column tile
-  int32_t long_groups; // ... and of the launch's first part, which takes only long windows (0: no such part)
+  int32_t groups;      // workgroups per column tile
+  int32_t long_groups; // unbalanced, tiles in turn: those of the part that takes the long windows
 };
 
 // Kernels take the arrays as restrict-qualified arguments: the compiler may
@@ -114,7 +113,7 @@ struct SpmmParams {
   SpmmParams {                                                                             \
     a_rwo, a_rowid, a_tile, a_off, a_atox, a_vals, a_B, a_C, a_p.num_windows,              \
         a_p.num_blocks, a_p.M, a_p.b_rows, a_p.N, a_p.nnz, a_p.n_ct, a_p.num_items,        \
-        a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span, a_p.ct_blocks, \
+        a_p.chunk, a_p.queue, a_p.runs, a_p.parts, a_p.span,                               \
         a_p.long_blocks, a_p.groups, a_p.long_groups                                       \
   }
 
@@ -968,7 +967,7 @@ __device__ __forceinline__ void split_window(const SpmmParams &p, int w, int ct,
 // the first quarter the i-th from the end of the others, which in a power-law
 // graph are light where it is heavy.
 constexpr int kLongGroups = 4;
-template <int PREC, int VEC, int NSUB, int MODE>
+template <int PREC, int VEC, int NSUB, int MODE, bool IN_TURN>
 __device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int ct, bool long_part,
                                             float (*s_tile)[wave_lds_words<VEC, NSUB>()], uint32_t *s_long) {
   const int wave = wave_uniform(threadIdx.x >> 6);
@@ -979,7 +978,7 @@ __device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int 
     return (g * kWavesPerBlock + v % kWavesPerBlock) * p.chunk;
   };
   auto blocks_before = [&](int w) { return max(0, min(p.rwo[min(w, p.num_windows)], p.num_blocks)); };
-  if (MODE == kDense || !long_part) {
+  if (!IN_TURN || !long_part) {
     const int g0 = group * kWavesPerBlock * p.chunk;  // the workgroup's windows (g0 < num_windows)
     const int g1 = min(g0 + kWavesPerBlock * p.chunk, p.num_windows);
     const int w0 = min(g0 + wave * p.chunk, g1);
@@ -1010,7 +1009,7 @@ __device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int 
       longs = n + 1 < 32 ? longs >> (n + 1) : 0;
       rwo = __shfl(rwo, lane + n + 1, 64);
     }
-    if (!any_long || p.long_groups) return;  // workgroup-uniform
+    if (!any_long || IN_TURN) return;  // workgroup-uniform
   } else {
 #pragma unroll 1
     for (int k = 0; k < kLongGroups; ++k) {
@@ -1020,7 +1019,7 @@ __device__ __forceinline__ void run_windows(const SpmmParams &p, int group, int 
     }
   }
   __syncthreads();
-  const int shares = long_part ? kLongGroups * kWavesPerBlock : kWavesPerBlock;
+  const int shares = IN_TURN ? kLongGroups * kWavesPerBlock : kWavesPerBlock;
   const int longs = (int)s_long[min(lane, shares - 1)];  // lane v: share v's
   for (int v = 0; v < shares; ++v) {
     for (uint32_t m = (uint32_t)__builtin_amdgcn_readlane(longs, v); m; m &= m - 1) {
@@ -1047,31 +1046,54 @@ __device__ __forceinline__ int spread_group(int g, int groups) {
 
 // Workgroup i serves column tile i % n_ct: workgroups are dispatched to the
 // 8 XCDs round robin, so when n_ct divides 8 every XCD (and its L2) only
-// sees one column tile of B.  With ct_blocks set, the column tiles go one
-// after another instead (workgroup i serves tile i / ct_blocks): all XCDs
-// then gather from the same column slice of B at a time.
+// sees one column tile of B.
 template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
 __global__ __launch_bounds__(256) __attribute__((
     amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED, MODE>()))) void spmm_kernel(SPMM_KERNEL_ARGS) {
   const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
   __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
   const int wave = wave_uniform(threadIdx.x >> 6);
+  const int ct = blockIdx.x % p.n_ct;
+  const int group = blockIdx.x / p.n_ct;
   if constexpr (BALANCED) {
-    const int ct = p.ct_blocks ? blockIdx.x / p.ct_blocks : blockIdx.x % p.n_ct;
-    const int group = p.ct_blocks ? blockIdx.x % p.ct_blocks : blockIdx.x / p.n_ct;
+    const int item = group * kWavesPerBlock + wave;
+    if (item >= p.num_items) return;
+    run_unit<PREC, VEC, NSUB, MODE>(p, item, ct, s_tile[wave]);
+  } else {
+    __shared__ uint32_t s_long[kWavesPerBlock];
+    run_windows<PREC, VEC, NSUB, MODE, false>(p, spread_group(group, p.groups), ct, false, s_tile, s_long);
+  }
+}
+
+// The same with the column tiles one after another: workgroup i serves tile
+// i / groups.  All XCDs then gather from the same column slice of B at a time; in
+// the balanced schedule from two, half of B's columns apart: with one alone, where
+// many gathers go to rows whose numbers are multiples of 16 (R-MAT as its
+// generator labels it), few memory channels serve them.  2^20 rows, N = 256, ms,
+// side by side, one and two slices at a time: 3.98, 4.50 and 4.22; with the
+// numbers shuffled inside groups of 16 3.45, 3.20 and 3.16.  The unbalanced launch
+// begins with the part that takes the long windows.
+template <int PREC, int VEC, int NSUB, bool BALANCED, int MODE>
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(spmm_waves_per_eu<PREC, VEC, NSUB, BALANCED, MODE>()))) void spmm_kernel_turn(SPMM_KERNEL_ARGS) {
+  const SpmmParams p = SPMM_PARAMS_FROM_ARGS;
+  __shared__ __attribute__((aligned(16))) float s_tile[kWavesPerBlock][wave_lds_words<VEC, NSUB>()];
+  if constexpr (BALANCED) {
+    const int wave = wave_uniform(threadIdx.x >> 6);
+    const int pass = blockIdx.x / p.groups;
+    const int group = blockIdx.x % p.groups;
+    const int ct = !(group & 1) ? pass : pass < p.n_ct / 2 ? pass + (p.n_ct + 1) / 2 : pass - p.n_ct / 2;
     const int item = group * kWavesPerBlock + wave;
     if (item >= p.num_items) return;
     run_unit<PREC, VEC, NSUB, MODE>(p, item, ct, s_tile[wave]);
   } else {
     __shared__ uint32_t s_long[kLongGroups * kWavesPerBlock];
-    const int long_wgs = MODE != kDense ? p.long_groups * p.n_ct : 0;
+    const int long_wgs = p.long_groups * p.n_ct;
     const bool long_part = (int)blockIdx.x < long_wgs;
-    const bool in_turn = p.ct_blocks && !long_part;
-    const unsigned at = blockIdx.x - (long_part ? 0 : long_wgs), per = in_turn ? p.ct_blocks : p.n_ct;
+    const unsigned at = blockIdx.x - (long_part ? 0 : long_wgs), per = long_part ? p.n_ct : p.groups;
     const int q = at / per, r = at % per;
-    const int ct = in_turn ? q : r;
-    const int group = spread_group(in_turn ? r : q, long_part ? p.long_groups : p.groups);
-    run_windows<PREC, VEC, NSUB, MODE>(p, group, ct, long_part, s_tile, s_long);
+    const int group = spread_group(long_part ? q : r, long_part ? p.long_groups : p.groups);
+    run_windows<PREC, VEC, NSUB, MODE, true>(p, group, long_part ? r : q, long_part, s_tile, s_long);
   }
 }
 
@@ -1336,6 +1358,7 @@ struct Variant {
 
 // Launch schedules of a kernel instance.
 constexpr int kRunWindows = 0, kRunBalanced = 1, kRunPersistent = 2, kRunSplit = 3;
+constexpr int kRunWindowsTurn = 4, kRunBalancedTurn = 5;
 
 template <int PREC, int VEC, int NSUB, int MODE>
 KernelFn pick_schedule(int schedule) {
@@ -1343,6 +1366,8 @@ KernelFn pick_schedule(int schedule) {
     case kRunWindows: return spmm_kernel<PREC, VEC, NSUB, false, MODE>;
     case kRunBalanced: return spmm_kernel<PREC, VEC, NSUB, true, MODE>;
     case kRunPersistent: return spmm_kernel_persistent<PREC, VEC, NSUB, MODE == kDense ? kBuf : MODE>;
+    case kRunWindowsTurn: return spmm_kernel_turn<PREC, VEC, NSUB, false, MODE == kDense ? kBuf : MODE>;
+    case kRunBalancedTurn: return spmm_kernel_turn<PREC, VEC, NSUB, true, MODE>;
     default: return spmm_kernel_split<PREC, VEC, NSUB, MODE>;
   }
 }
@@ -1476,15 +1501,15 @@ bool split_windows(int64_t windows, int64_t n_ct, int64_t num_blocks) {
 
 // Consecutive windows per unit of the unbalanced schedule: short windows are
 // walked several to a wave, as one pipeline, while enough units remain.  For
-// tiles of up to 32 columns only, where a window is little work: wider ones lose
+// units of up to 32 columns only, where a window is little work: wider ones lose
 // more by the longer chains, and in a band by rows of B that the workgroup's
 // waves no longer read at the same time.  us, one window and several: uniform
 // 2^20 rows of 4, N = 16 111 and 103, of 8, N = 32 194 and 188, of 4, N = 64 186
 // and 197; band of 19 columns half filled, 500,001 rows, N = 100 105 and 117, of
 // 25, 10^6 rows, N = 128 262 and 277; R-MAT of 2^20 rows of 4, N = 64 618 and 843.
-int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks, int32_t tile) {
+int32_t windows_per_unit(int64_t windows, int64_t n_ct, int64_t num_blocks, int32_t columns) {
   int32_t k = 1;
-  if (tile > 32) return k;
+  if (columns > 32) return k;
   while (k < 32 && 2 * k * num_blocks <= 32 * windows && windows * n_ct >= 2 * k * 16384) k *= 2;
   return k;
 }
@@ -1501,12 +1526,19 @@ int32_t long_window(int64_t windows, int64_t num_blocks) {
   return (int32_t)std::min<int64_t>(std::max<int64_t>(128, 4 * num_blocks / windows), INT32_MAX);
 }
 
-// Workgroups per column tile when the column tiles go one after another, 0
-// when they go side by side.  B beyond the 256 MB memory-side cache: one
-// slice at a time, so that most of its gathers hit there.
-int32_t column_order(const SpmmParams &p, int64_t esz) {
+// Whether hardly any column has two entries in a window (of the least 8 entries
+// a block, at most 8.25): uniform matrices; in power-law ones rows share the
+// hubs' columns (8.3 to 13 entries a block).
+bool unshared_columns(int64_t nnz, int64_t num_blocks) { return 4 * nnz <= 33 * num_blocks; }
+
+// Whether the column tiles go one after another instead of side by side.  B
+// beyond the 256 MB memory-side cache: one slice (or two) at a time, so that most
+// of its gathers hit there.  (Two tiles of 256 MB each are no faster in turn,
+// uniform 2^20 rows of 16, N = 128 1.24 and 1.29 ms; two of 512 are, N = 256 2.93
+// and 2.53.)
+bool tiles_in_turn(const SpmmParams &p, int64_t esz) {
   const int64_t b_bytes = (int64_t)p.b_rows * p.N * esz;
-  return p.n_ct > 1 && b_bytes > ((int64_t)256 << 20) ? (int32_t)ceil_div(p.num_items, kWavesPerBlock) : 0;
+  return p.n_ct > 1 && b_bytes > (int64_t)(p.n_ct > 2 ? 256 : 512) << 20;
 }
 
 dtc_status_t check_common(const uint8_t *tile, const int32_t *off, const int32_t *atox,
@@ -1797,6 +1829,7 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   Variant var;
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
+  const bool unshared = unshared_columns(nnz, num_blocks);
   st = resolve_shape(options, n, b, c, false, false, mode, &var);
   if (st != DTC_SUCCESS) return st;
   // Only windows that hold output rows are processed.
@@ -1819,13 +1852,16 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   p.num_blocks = num_blocks;
   p.nnz = nnz;
   const bool split = split_windows(W, p.n_ct, num_blocks);
-  p.chunk = split ? 1 : windows_per_unit(W, p.n_ct, num_blocks, 16 * var.vec * var.nsub);
+  p.chunk = split ? 1 : windows_per_unit(W, p.n_ct, num_blocks, std::min(n, 16 * var.vec * var.nsub));
   p.num_items = (int32_t)ceil_div(W, p.chunk);
-  p.ct_blocks = split ? 0 : column_order(p, esz);
+  // (Uniform 2^20 rows of 16, N = 256, ms, side by side and one after another: 3.10
+  // and 2.56; R-MAT of 31.4 M entries 4.94 and 5.74, of 8 M, N = 128 1.29 and 2.02;
+  // band of 400,000 rows, N = 260 0.304 and 0.337.)
+  const bool turn = !split && unshared && tiles_in_turn(p, esz);
   p.long_blocks = long_window(W, num_blocks);
-  KernelFn fn = pick_kernel(var, split ? kRunSplit : kRunWindows);
+  KernelFn fn = pick_kernel(var, split ? kRunSplit : turn ? kRunWindowsTurn : kRunWindows);
   p.groups = split ? W : (int32_t)ceil_div(p.num_items, kWavesPerBlock);
-  p.long_groups = p.ct_blocks && mode != kDense ? (int32_t)ceil_div(p.groups, kLongGroups) : 0;
+  p.long_groups = turn ? (int32_t)ceil_div(p.groups, kLongGroups) : 0;
   const int64_t grid = (int64_t)p.n_ct * ((int64_t)p.groups + p.long_groups);
   if (grid > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "grid too large");
   hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, stream, p.rwo, p.rowid, p.tile, p.off,
@@ -1908,7 +1944,10 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   p.num_items = (int32_t)ceil_div(num_blocks, chunk);
   p.chunk = chunk;
   p.span = span;
-  p.ct_blocks = column_order(p, esz);
+  // (Chunks that keep windows up to a span whole run longer, and side by side they
+  // lose nothing as labelled by the generator: spans of 256, ms, 3.93 against 4.04.)
+  const bool turn = span == chunk && tiles_in_turn(p, esz);
+  p.groups = (int32_t)ceil_div(p.num_items, kWavesPerBlock);
   p.queue = persistent ? static_cast<int32_t *>(workspace) : nullptr;
   int2 *runs = reinterpret_cast<int2 *>(static_cast<char *>(workspace) + kQueueBytes);
   p.runs = runs;
@@ -1920,8 +1959,8 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
       tcblock_rowid, num_blocks, num_nodes, n, chunk, span, p.num_items, c, p.queue, runs, det ? 0 : 1);
   DTC_LAUNCH_CHECK("balance_prep");
   if (!persistent) {
-    KernelFn fn = pick_kernel(var, kRunBalanced);
-    const int64_t grid = (int64_t)p.n_ct * ceil_div(p.num_items, kWavesPerBlock);
+    KernelFn fn = pick_kernel(var, turn ? kRunBalancedTurn : kRunBalanced);
+    const int64_t grid = (int64_t)p.n_ct * p.groups;
     if (grid > INT32_MAX) return fail(DTC_ERROR_UNSUPPORTED, "grid too large");
     hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(256), 0, stream, p.rwo, p.rowid, p.tile, p.off,
                      p.atox, p.vals, p.B, p.C, p);

@@ -120,6 +120,24 @@ def test_long_windows_wide_b(rows, n, options):
     check(rowptr.astype(np.int32), col.astype(np.int32), values, cols, n, "windows", **options)
 
 
+@pytest.mark.parametrize("n,options", [(130, {}), (256, {}), (64, {"vec": 1, "deterministic": True}), (160, {"vec": 2}),
+                                       (130, {"chunk_blocks": 8, "cut_span_blocks": 64})])
+def test_balanced_wide_b(n, options):
+    """B beyond 256 MB in three, four and five column tiles, two of them at a
+    time; with a cut span side by side."""
+    rng = np.random.default_rng(n)
+    cols = (1 << 28) // (4 * n) + 1000
+    rows = 16 * 90 - 5
+    lengths = rng.integers(0, 20, rows)
+    lengths[160:192] = 0
+    lengths[400] = 1100
+    rowptr = np.zeros(rows + 1, np.int64)
+    rowptr[1:] = np.cumsum(lengths)
+    col = np.concatenate([np.sort((rng.integers(0, cols) + np.arange(k) * (cols // 1200)) % cols) for k in lengths])
+    values = rng.uniform(-1, 1, col.shape[0]).astype(np.float32)
+    check(rowptr.astype(np.int32), col.astype(np.int32), values, cols, n, "balanced", **options)
+
+
 @pytest.mark.parametrize("n", [48, 64, 65, 96, 97, 224])
 @pytest.mark.parametrize("blocks", [8800, 8801, 17600, 17601, 35200, 35201])
 def test_default_chunks(n, blocks):
