@@ -1428,7 +1428,8 @@ int operand_mode(int64_t b_rows, int64_t n, int64_t esz, int64_t nnz, int64_t nu
 // vec 0 for float32 B: 4 floats per lane (64-column tiles), less where N is
 // narrower.
 dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void *b, const float *c,
-                           bool balanced, bool dense, int mode, Variant *out) {
+                           bool balanced, bool dense, bool unshared, bool short_windows, int mode,
+                           Variant *out) {
   const bool wide = mode == kPtr;
   const int prec = opt ? opt->precision : DTC_PRECISION_FP32;
   const int bdt = opt ? opt->b_dtype : DTC_B_FLOAT32;
@@ -1474,11 +1475,23 @@ dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void 
     // builds its A again), else three of 32 in the balanced one (N = 96, us: 46,000
     // blocks 40 against 47 and 55, 157,000 96 / 108 / 121, 1.08 M 476 / 526 / 539;
     // block model of 958,000 blocks of 13 382 / 397 / 372, band of 55 a block 66 and
-    // 60).  128-column tiles also
-    // for wide B in the unbalanced schedule.
+    // 60).  128-column tiles also for wide B in the unbalanced schedule.  There not
+    // where rows share columns without being dense, as hubs do, whose windows then
+    // take longer (us with one and two subtiles: R-MAT of 25,568 rows, N = 84 220 and
+    // 313, of 262,144 631 and 881, block model of 60,000, N = 320 1,218 and 1,465;
+    // uniform 65,536 rows of 32, N = 84 111 and 84, 200,000 of 16, N = 260 755 and
+    // 627), and for dense blocks not with the limb splits, whose registers cost waves
+    // in windows of a group or two (band of 5 blocks a window, N = 224, bf16x3 37 and
+    // 40, bf16x6 43 and 47; of 10, N = 512 72 and 63, 77 and 75), nor where wide B
+    // leaves half of the last tile empty (N = 320 51 and 55, 384 62 and 58).
     const bool half = n % 128 > 64 && n % 128 <= 96;
     if (nsub == 0 && balanced && half && n < 128 && !dense) vec = 2;
-    if (nsub == 0) nsub = (half && (!balanced || dense)) || (!balanced && n > 256) ? 2 : 1;
+    if (nsub == 0 && balanced) nsub = half && dense ? 2 : 1;
+    if (nsub == 0) {
+      const bool limbs = prec == DTC_PRECISION_BF16X3 || prec == DTC_PRECISION_BF16X6;
+      const bool two = mode == kDense ? !(limbs && short_windows) && (half || (n > 256 && (n - 1) % 128 >= 64)) : half || n > 256;
+      nsub = two && (mode == kDense || unshared) ? 2 : 1;
+    }
   }
   if (wide) vec = n >= 4 ? 4 : 1;
   if (nsub == 0 || wide || vec != 4) nsub = 1;
@@ -1776,7 +1789,7 @@ dtc_status_t dtc_spmm_tcgnn(const int32_t *node_pointer, const int32_t *edge_lis
   o.vec = options ? options->vec : 0;
   o.subtiles = 1;
   Variant var;
-  dtc_status_t st = resolve_shape(&o, n, b, c, false, false, kBuf, &var);
+  dtc_status_t st = resolve_shape(&o, n, b, c, false, false, false, false, kBuf, &var);
   if (st != DTC_SUCCESS) return st;
   const int32_t W = (int32_t)ceil_div(num_nodes, kBlkH);
   if (b_rows == 0) return zero_output(c, num_nodes, n, stream);
@@ -1830,7 +1843,7 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
   const bool unshared = unshared_columns(nnz, num_blocks);
-  st = resolve_shape(options, n, b, c, false, false, mode, &var);
+  st = resolve_shape(options, n, b, c, false, false, unshared, num_blocks <= 6 * (int64_t)num_windows, mode, &var);
   if (st != DTC_SUCCESS) return st;
   // Only windows that hold output rows are processed.
   const int32_t W = (int32_t)std::min<int64_t>(num_windows, ceil_div(num_nodes, kBlkH));
@@ -1908,7 +1921,8 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   Variant var;
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
-  st = resolve_shape(options, n, b, c, true, nnz > (num_blocks >= (1 << 19) ? 11 : 24) * (int64_t)num_blocks, mode, &var);
+  st = resolve_shape(options, n, b, c, true, nnz > (num_blocks >= (1 << 19) ? 11 : 24) * (int64_t)num_blocks, false, false,
+                     mode, &var);
   if (st != DTC_SUCCESS) return st;
   const int chunk = resolve_chunk(options, num_blocks, nnz, n);
   int span = chunk;
