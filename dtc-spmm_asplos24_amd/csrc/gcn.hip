@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64 * kDwWaves, 3) void k_gcn_dw(const void *__restr
   xvec xv[8];
   gfloatx4 yv[8];
   // Rows m0 + 8 h + j: a wave-uniform row base and one 32-bit lane offset
-  // (8 h K + kx is below 2^31 elements for any K the shape check lets in).
+  // (25 K and 25 F are below 2^31: check_gradient_shape).
   const uint32_t xo = (uint32_t)(8 * h * K + kx), yo = (uint32_t)(8 * h * F + f0 + 4 * c);
   auto load = [&](int64_t m0) {
 #pragma unroll
@@ -412,6 +412,15 @@ dtc_status_t check_gcn_shape(int32_t m, int32_t k, int32_t f) {
   return DTC_SUCCESS;
 }
 
+// The gradients' kernels hold row offsets and tile counts in 32 bits and launch
+// a thread per two of dW's elements, of which a launch takes fewer than 2^32.
+dtc_status_t check_gradient_shape(int32_t m, int32_t k, int32_t f) {
+  const dtc_status_t st = check_gcn_shape(m, k, f);
+  if (st == DTC_SUCCESS && (int64_t)k * f >= (int64_t)1 << 31)
+    return fail(DTC_ERROR_UNSUPPORTED, "K * F must be below 2^31 for the gradients");
+  return st;
+}
+
 }  // namespace
 }  // namespace dtc
 
@@ -463,7 +472,7 @@ dtc_status_t dtc_gcn_input_grad(const float *dy, const void *w, const void *x, i
                                 int32_t m, int32_t k, int32_t f, void *dx, void *workspace,
                                 size_t workspace_bytes, dtc_stream_t stream_) {
   clear_error();
-  dtc_status_t st = check_gcn_shape(m, k, f);
+  dtc_status_t st = check_gradient_shape(m, k, f);
   if (st != DTC_SUCCESS) return st;
   if (x_dtype != DTC_GCN_X_FLOAT32 && x_dtype != DTC_GCN_X_BFLOAT16)
     return fail(DTC_ERROR_INVALID_VALUE, "x_dtype must be DTC_GCN_X_FLOAT32 or DTC_GCN_X_BFLOAT16");
@@ -493,7 +502,7 @@ dtc_status_t dtc_gcn_input_grad(const float *dy, const void *w, const void *x, i
 dtc_status_t dtc_gcn_weight_grad_workspace_size(int32_t m, int32_t k, int32_t f, size_t *bytes) {
   clear_error();
   if (!bytes) return fail(DTC_ERROR_INVALID_VALUE, "bytes is NULL");
-  dtc_status_t st = check_gcn_shape(m, k, f);
+  dtc_status_t st = check_gradient_shape(m, k, f);
   if (st != DTC_SUCCESS) return st;
   *bytes = (size_t)dw_plan(m, k, f).splits * k * f * sizeof(float);
   return DTC_SUCCESS;
@@ -503,7 +512,7 @@ dtc_status_t dtc_gcn_weight_grad(const void *x, int32_t x_dtype, int32_t relu, c
                                  int32_t k, int32_t f, void *dw, void *workspace, size_t workspace_bytes,
                                  dtc_stream_t stream_) {
   clear_error();
-  dtc_status_t st = check_gcn_shape(m, k, f);
+  dtc_status_t st = check_gradient_shape(m, k, f);
   if (st != DTC_SUCCESS) return st;
   if (x_dtype != DTC_GCN_X_FLOAT32 && x_dtype != DTC_GCN_X_BFLOAT16)
     return fail(DTC_ERROR_INVALID_VALUE, "x_dtype must be DTC_GCN_X_FLOAT32 or DTC_GCN_X_BFLOAT16");

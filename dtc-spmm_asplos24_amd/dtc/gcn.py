@@ -52,12 +52,13 @@ def fused_transform_applies(X: torch.Tensor, W: torch.Tensor, relu: bool = True)
 def fused_gradients_apply(X: torch.Tensor, W: torch.Tensor, dY: torch.Tensor) -> bool:
     """Whether act(X) W's gradients run on libdtc's kernels, which read the
     float32 dY and X once each and fuse the ReLU, its mask and the casts: bf16
-    W of a shape they take, 16-byte aligned X.  (On X 262,144 x 256 float32 and
+    W of a shape they take, fewer than 2^31 weights (their row offsets are 32-bit),
+    16-byte aligned X.  (On X 262,144 x 256 float32 and
     F = 256: 345 us; torch's cast, GEMM, compare, product and cast for dX and
     ReLU, cast, transposing copy and batched GEMM for dW took 860.)"""
     return (W.dtype == torch.bfloat16 and X.dtype in (torch.float32, torch.bfloat16)
             and W.shape[0] % 32 == 0 and W.shape[1] % 64 == 0 and X.shape[0] == dY.shape[0]
-            and X.data_ptr() % 16 == 0)
+            and X.data_ptr() % 16 == 0 and W.numel() < 1 << 31)
 
 
 def _act(X: torch.Tensor, relu: bool, dtype) -> torch.Tensor:

@@ -394,7 +394,8 @@ dtc_status_t dtc_gcn_transform(const void *x, int32_t x_dtype, int32_t relu, con
 
 /* Gradients of Y = act(X) W from dY [M x F] float32 (dY, and act(X) for dW,
  * rounded to bf16 as they are loaded; float32 accumulation).  X and W as
- * above, W unpacked; 16-byte aligned operands.
+ * above, W unpacked, K * F below 2^31 (else DTC_ERROR_UNSUPPORTED); 16-byte
+ * aligned operands.
  * dx[i][k] = bf16(sum_j dY[i][j] W[k][j]) * (relu ? X[i][k] > 0 : 1), [M x K]
  * in x_dtype; workspace: K * F * 2 bytes. */
 dtc_status_t dtc_gcn_input_grad(const float *dy, const void *w, const void *x, int32_t x_dtype,

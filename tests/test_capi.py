@@ -173,6 +173,22 @@ def test_host_side_argument_errors(lib):
         assert st == 1 and b"cut_span_blocks" in lib.dtc_last_error()
 
 
+def test_gcn_gradient_shapes(lib):
+    """K * F of 2^31 and more exceeds the gradients' 32-bit row offsets: refused
+    before any launch, and left to the plain products by the layer."""
+    from dtc.gcn import fused_gradients_apply
+    size, dummy, room = ctypes.c_size_t(), ctypes.c_void_p(4096), ctypes.c_size_t(1 << 50)
+    for k, f in ((1 << 25, 64), (32, 1 << 26), (1 << 27, 64), (64, 1 << 30)):
+        assert lib.dtc_gcn_weight_grad_workspace_size(32, k, f, ctypes.byref(size)) == 2, (k, f)
+        assert lib.dtc_gcn_weight_grad(dummy, 0, 0, dummy, 32, k, f, dummy, dummy, room, None) == 2
+        assert lib.dtc_gcn_input_grad(dummy, dummy, dummy, 0, 0, 32, k, f, dummy, dummy, room, None) == 2
+    assert lib.dtc_gcn_weight_grad_workspace_size(32, (1 << 25) - 32, 64, ctypes.byref(size)) == 0
+    assert size.value == ((1 << 25) - 32) * 64 * 4
+    for k, fits in ((1 << 25, False), ((1 << 25) - 32, True)):
+        X, W = (torch.empty(n, dtype=torch.bfloat16, device="meta") for n in ((32, k), (k, 64)))
+        assert fused_gradients_apply(X, W, torch.empty((32, 64), device="meta")) is fits
+
+
 @pytest.fixture(scope="module")
 def ext():
     from dtc import load_extension
