@@ -115,13 +115,18 @@ class DTCMatrix:
     # ------------------------------------------------------------- transpose
     def transpose(self) -> "DTCMatrix":
         """ME-TCF of A^T (built on the GPU once and cached).  Its values are
-        set per call from A's CSR values through ``perm_t``."""
+        set per call from A's CSR values through ``tc_edge_t``, which is made
+        here too: made by the first gradient instead, it would belong to that
+        one's stream, or to the graph that records it."""
         if self._transpose is None:
             ext = load_extension()
             rpt, ct, perm = ext.csr_transpose(self.rowptr, self.col, self.num_rows, self.num_cols)
-            self._perm_t = perm
-            self._transpose = DTCMatrix(rpt, ct, None, num_rows=self.num_cols,
-                                        num_cols=self.num_rows, device=self.device)
+            # perm goes through the build as values (32-bit words, moved and not looked at)
+            At = DTCMatrix(rpt, ct, perm.view(torch.float32), num_rows=self.num_cols,
+                           num_cols=self.num_rows, device=self.device)
+            self._perm_t, self._tc_edge_t = perm, At.values_tc.view(torch.int32)
+            At.values = At.values_tc = None
+            self._transpose = At
         return self._transpose
 
     @property
@@ -132,12 +137,8 @@ class DTCMatrix:
     @property
     def tc_edge_t(self) -> torch.Tensor:
         """CSR edge of A behind every TC position of A^T (perm_t after A^T's
-        tc_edge, composed once): A's CSR values reach A^T's TC order in one
-        gather."""
-        if self._tc_edge_t is None:
-            At = self.transpose()
-            # the gather moves 32-bit words whatever they hold
-            self._tc_edge_t = load_extension().gather(self._perm_t.view(torch.float32), At.tc_edge).view(torch.int32)
+        tc_edge): A's CSR values reach A^T's TC order in one gather."""
+        self.transpose()
         return self._tc_edge_t
 
     def transposed_operands(self, schedule: str = "windows", values: torch.Tensor | None = None) -> tuple:

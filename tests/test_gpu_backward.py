@@ -242,3 +242,49 @@ def test_reference_backward_names(ext):
     assert comp(fwd) > 1e-2
     with pytest.raises(ValueError, match="transposed"):
         ext.backward_ptx_uint8_improved(dY, *w_args, "float4_split", transposed=(tw[0],))
+
+
+def test_first_gradient_recorded():
+    """Everything that gradients keep is made with the transpose: a graph that
+    records the first gradient leaves eager ones before its first replay right,
+    and both agree bit for bit from then on."""
+    from dtc.matrix import DTCMatrix, spmm_autograd
+    rng = np.random.default_rng(61)
+    M, K, n = 900, 700, 48
+
+    def matrix():
+        rowptr, col = random_csr(rng, M, K, 7.0, sorted_rows=True, empty_frac=0.1)
+        return rowptr, col, DTCMatrix(rowptr, col, None, num_rows=M, num_cols=K)
+
+    rowptr, col, A = matrix()
+    At = A.transpose()
+    assert A._tc_edge_t is not None and At.values is None and At.values_tc is None
+    assert torch.equal(A.tc_edge_t, A.perm_t[At.tc_edge.long()])
+    values = torch.from_numpy(rng.uniform(-1, 1, col.shape[0]).astype(np.float32)).cuda().requires_grad_(True)
+    B = torch.from_numpy(rng.standard_normal((K, n)).astype(np.float32)).cuda().requires_grad_(True)
+    dC = torch.from_numpy(rng.standard_normal((M, n)).astype(np.float32)).cuda()
+
+    def step(values, B, A):
+        return torch.autograd.grad(spmm_autograd(values, B, A, schedule="windows"), (values, B), dC)
+
+    _, col2, A2 = matrix()  # warm-up with a matrix of its own
+    step(torch.ones(col2.shape[0], device="cuda", requires_grad=True), B, A2)
+    torch.cuda.synchronize()
+    say("record the first gradient")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recorded = step(values, B, A)
+    say("eager before the first replay")
+    eager = step(values, B, A)
+    v = values.detach().cpu().numpy().astype(np.float64)
+    rows = np.repeat(np.arange(M), np.diff(rowptr))
+    dB = np.zeros((K, n))
+    np.add.at(dB, col, v[:, None] * dC.cpu().numpy().astype(np.float64)[rows])
+    assert np.allclose(eager[1].cpu().numpy(), dB, rtol=1e-5, atol=1e-5)
+    for i in range(3):
+        say("replay", i)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(recorded, eager))
+        assert all(torch.equal(a, b) for a, b in zip(step(values, B, A), eager))
+        torch.cuda.synchronize()
