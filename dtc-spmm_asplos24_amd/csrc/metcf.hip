@@ -447,7 +447,10 @@ __global__ __launch_bounds__(1024) void k_big_offsets(const int32_t *rowptr, int
 // from 106 to 57 us.  Whole builds with this kernel and with the launches it
 // replaces, 8 entries a row: 256 windows 56 and 64 us, 1,024 60 and 64, 2,048
 // 68 and 67, 4,096 86 and 72.)
-constexpr int kOnePlanWindows = 1024;
+// The rows are bounded too, to what those windows have at 16 rows: one workgroup
+// checks their pointers 1,024 at a time (1,024 windows of 1,024 rows 596 us with the
+// other launches and 1,050 with this one, 1,024 of 4,096 1.21 and 3.00 ms).
+constexpr int kOnePlanWindows = 1024, kOnePlanRows = kOnePlanWindows * kWinH;
 __global__ __launch_bounds__(1024) void k_plan(const int32_t *rowptr, int32_t M, int32_t nnz,
                                                int32_t W, int32_t blk_h, int mode,
                                                const int32_t *bp, const int32_t *col,
@@ -2294,7 +2297,7 @@ dtc_status_t dtc_metcf_build_windows(const int32_t *edge_list, const int32_t *no
       std::memcpy(&host, dev_state->pinned, kHeaderRead);
       return DTC_SUCCESS;
     };
-    if (W <= kOnePlanWindows) {
+    if (W <= kOnePlanWindows && num_nodes <= kOnePlanRows) {
       k_plan<<<1, 1024, 0, stream>>>(node_pointer, num_nodes, nnz, (int32_t)W, blk_h, mode,
                                      block_partition, edge_list, ws.lists, row_window_offset,
                                      sort_tile, ws.csb, ws.tb, ws.tw, ws.hdr, report);

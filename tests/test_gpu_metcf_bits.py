@@ -57,6 +57,16 @@ def window(rng, entries, span, first=0):
     return [first + r for r in rows]
 
 
+@pytest.mark.parametrize("blk_h", [24, 32])
+@pytest.mark.parametrize("M", [1024 * 16, 1024 * 16 + 1])
+def test_tall_windows(ext, M, blk_h):
+    """Few windows of many rows: one workgroup plans the build up to 16,384 rows."""
+    rng = np.random.default_rng(M + blk_h)
+    rowptr, col = csr([np.sort(rng.choice(300, n, replace=False)) for n in rng.integers(0, 5, M)])
+    say("metcf", "tall", M, blk_h)
+    assert_metcf_equal(gpu_metcf(ext, rowptr, col, M, blk_h, 8), oracle.metcf(rowptr, col, M, blk_h, 8), ctx=(M, blk_h))
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("cls", [1, 2, 3, 4, 5])
 def test_spans_and_sizes(ext, monkeypatch, cls, wide):
