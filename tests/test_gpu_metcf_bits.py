@@ -213,3 +213,22 @@ def test_row_pointer_beyond_the_edges(ext, windows):
     rowptr[100] = 2_000_000_000
     with pytest.raises(RuntimeError, match="nodePointer decreases"):
         gpu_metcf(ext, rowptr, np.zeros(windows * 16, np.int32), windows * 16, 16, 8)
+
+
+@pytest.mark.parametrize("repeat", [False, True])
+@pytest.mark.parametrize("every", [1, 7, 400])
+def test_unsorted_rows_among_many(ext, monkeypatch, every, repeat):
+    """A repeated entry or a descent in one row of every window, of some and of
+    one or two, in any of the 16 rows: found by the look at each window or by its
+    own kernel."""
+    monkeypatch.setenv("DTC_METCF_PATH", "auto")
+    rng = np.random.default_rng(every + repeat)
+    rows = []
+    for w in range(700):
+        rows += window(rng, int(rng.choice([90, 300, 700, 2500])) if w % 50 else 5000, 9000, first=w % 3)
+        if w % every == every // 2:
+            r = max(range(len(rows) - 16, len(rows)), key=lambda i: (len(rows[i]) >= 3) * rng.random())
+            if len(rows[r]) >= 2:
+                i = int(rng.integers(0, len(rows[r]) - 1))
+                rows[r][i:i + 2] = rows[r][i:i + 1] if repeat else rows[r][i:i + 2][::-1].copy()
+    check(ext, rows, ("unsorted rows", every, repeat))
