@@ -1578,8 +1578,9 @@ dtc_status_t check_common(const uint8_t *tile, const int32_t *off, const int32_t
   return DTC_SUCCESS;
 }
 
-// Longest default of a balanced chunk, in TC blocks: the one that a cut span is
-// measured against, and the one for a fixed workspace that short chunks exceed.
+// The default chunk by the block count alone, in TC blocks: the one that a cut
+// span is measured against, and the one for a workspace that the chunks of
+// resolve_chunk exceed (it is mostly longer than those, not always).
 int long_chunk_blocks(int32_t num_blocks) {
   int c = 32;
   while (c < 512 && (int64_t)c * 2 * 8192 <= (int64_t)num_blocks) c *= 2;
@@ -1602,11 +1603,12 @@ int long_chunk_blocks(int32_t num_blocks) {
 // block, 53,000 blocks, N = 64 (32) 37 (16) 44, 106,000, N = 256 (32) 164 (64)
 // 187, 8,750, N = 128 (8) 19.6 (16) 21.3.
 // nnz 0: not known, the shortest chunk it could be.
+constexpr int64_t kChunkUnits = 550;
 int resolve_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n) {
   if (opt && opt->chunk_blocks > 0) return opt->chunk_blocks;
   if (opt && opt->cut_span_blocks != 0) return long_chunk_blocks(num_blocks);
   const bool dense = nnz > 24 * (int64_t)num_blocks;
-  const int64_t k = !dense && nnz > 11 * (int64_t)num_blocks ? 275 : 550;
+  const int64_t k = !dense && nnz > 11 * (int64_t)num_blocks ? kChunkUnits / 2 : kChunkUnits;
   int c = dense && num_blocks >= 1 << 15 ? 32 : 8;
   while (c < 256 && (int64_t)num_blocks * ceil_div(std::max(n, 1), 64) > k * c * c) c *= 2;
   return c;
@@ -1644,6 +1646,17 @@ size_t balanced_workspace_bytes_for(int32_t num_blocks, int32_t n, int32_t chunk
   const int64_t npad = ceil_div(std::max<int32_t>(n, 1), 128) * 128;
   return balanced_parts_offset(num_blocks, chunk) +
          (size_t)(2 * num_chunks(num_blocks, chunk)) * kBlkH * (size_t)npad * sizeof(float);
+}
+
+// The chunk for a workspace of this size: resolve_chunk's, or with the default
+// the one by the block count alone where only that one fits.
+int fit_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, size_t workspace_bytes) {
+  const int chunk = resolve_chunk(opt, num_blocks, nnz, n);
+  const bool det = opt && opt->deterministic;
+  if ((opt && (opt->chunk_blocks > 0 || opt->cut_span_blocks != 0)) ||
+      balanced_workspace_bytes_for(num_blocks, n, chunk, det) <= workspace_bytes)
+    return chunk;
+  return std::max(chunk, long_chunk_blocks(num_blocks));
 }
 
 __global__ __launch_bounds__(256) void k_zero(float *c, int64_t count) {
@@ -1900,8 +1913,15 @@ dtc_status_t dtc_spmm_balanced_workspace_size_ex(int32_t num_blocks, int32_t n,
   if (options && options->chunk_blocks < 0)
     return fail(DTC_ERROR_INVALID_VALUE, "chunk_blocks must be >= 0");
   const bool det = options && options->deterministic;
-  const int chunk = resolve_chunk(options, num_blocks, 0, n);
-  *bytes = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
+  // For every N up to this one: a narrower N can have shorter, i.e. more chunks.
+  *bytes = 0;
+  for (int64_t m = n;;) {
+    const int64_t chunk = resolve_chunk(options, num_blocks, 0, (int32_t)m);
+    *bytes = std::max(*bytes, balanced_workspace_bytes_for(num_blocks, (int32_t)m, (int32_t)chunk, det));
+    if ((options && (options->chunk_blocks > 0 || options->cut_span_blocks != 0)) || chunk <= 8) break;
+    m = kChunkUnits * (chunk / 2) * (chunk / 2) / num_blocks * 64;  // the widest with half the chunk
+    if (m == 0) break;
+  }
   return DTC_SUCCESS;
 }
 
@@ -1924,14 +1944,14 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   st = resolve_shape(options, n, b, c, true, nnz > (num_blocks >= (1 << 19) ? 11 : 24) * (int64_t)num_blocks, false, false,
                      mode, &var);
   if (st != DTC_SUCCESS) return st;
-  const int chunk = resolve_chunk(options, num_blocks, nnz, n);
+  const bool det = options && options->deterministic;
+  const int chunk = fit_chunk(options, num_blocks, nnz, n, workspace_bytes);
   int span = chunk;
   st = resolve_cut_span(options, chunk, &span);
   if (st != DTC_SUCCESS) return st;
   const bool persistent = options && options->persistent;
   if (options && (options->deterministic < 0 || options->deterministic > 1))
     return fail(DTC_ERROR_INVALID_VALUE, "deterministic must be 0 or 1");
-  const bool det = options && options->deterministic;
   const int32_t W = (int32_t)ceil_div(num_nodes, kBlkH);
   if (W == 0) return DTC_SUCCESS;
   const size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
@@ -2016,12 +2036,8 @@ dtc_status_t dtc_spmm_balanced_noalloc(const int32_t *tcblock_rowid, const uint8
   const bool det = options && options->deterministic;
   dtc_spmm_options_t o{};
   if (options) o = *options;
-  int chunk = resolve_chunk(options, num_blocks, nnz, n);
-  size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
-  if (need > kNoAllocScratchBytes && o.chunk_blocks == 0) {
-    chunk = std::max(chunk, long_chunk_blocks(num_blocks));
-    need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
-  }
+  const int chunk = fit_chunk(options, num_blocks, nnz, n, kNoAllocScratchBytes);
+  const size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
   o.chunk_blocks = chunk;
   if (need > kNoAllocScratchBytes)
     return fail(DTC_ERROR_UNSUPPORTED,

@@ -65,11 +65,11 @@ VARIANTS = [
 
 
 def default_chunk_blocks(num_blocks: int) -> int:
-    """The longest chunk the library takes by default: the largest power of two
+    """The chunk that depends on the block count alone: the largest power of two
     in [32, 512] at most num_blocks / 8192.  Options that leave the chunk at 0
-    give it with a cut span, and a shorter one otherwise that depends on N too
-    (csrc/spmm.hip); this one is stated wherever a chunk has to depend on the
-    block count alone (the selector's variants, the GCN layer's backward)."""
+    give it with a cut span, and otherwise one that depends on N too, mostly
+    shorter (csrc/spmm.hip); the selector's variants and the GCN layer's backward
+    state this one."""
     c = 32
     while c < 512 and c * 2 * 8192 <= num_blocks:
         c *= 2

@@ -188,13 +188,15 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
  * variant and, with options->deterministic, the partial tiles; its size is
  * dtc_spmm_balanced_workspace_size_ex for these options and N
  * (256 + 8 * ceil(num_blocks / chunk) bytes without the deterministic merge;
- * for the default chunk, the shortest that num_blocks and N can have),
+ * for the default chunk, enough for every N up to this one; a smaller one is
+ * accepted down to what chunks of the size that cut_span_blocks implies need,
+ * which are then used),
  * or dtc_spmm_balanced_workspace_size (256 + 8 * num_blocks bytes, enough for
  * any chunk size without the deterministic merge).
  */
 dtc_status_t dtc_spmm_balanced_workspace_size(int32_t num_blocks, size_t *bytes);
-/* Workspace bytes for the given options and N (NULL options: the defaults):
- * 256 + 8 * ceil(num_blocks / chunk), plus with options->deterministic two
+/* Workspace bytes for the given options and every N up to this one (NULL options:
+ * the defaults): 256 + 8 * ceil(num_blocks / chunk), plus with options->deterministic two
  * partial-tile slots of 16 x N float32 (N rounded up to 128) per chunk. */
 dtc_status_t dtc_spmm_balanced_workspace_size_ex(int32_t num_blocks, int32_t n,
                                                  const dtc_spmm_options_t *options, size_t *bytes);

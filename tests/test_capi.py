@@ -173,6 +173,32 @@ def test_host_side_argument_errors(lib):
         assert st == 1 and b"cut_span_blocks" in lib.dtc_last_error()
 
 
+@pytest.mark.parametrize("deterministic", [0, 1])
+@pytest.mark.parametrize("blocks", [4, 1000, 40000, 157000, 3428580])
+def test_balanced_workspace_covers_narrower(lib, blocks, deterministic):
+    """The size for one N is enough for every narrower one (the default chunk
+    depends on N); workspaces below the formula of the chunk by the block count
+    alone stay refused."""
+    o = Opts(0, 0, 0, 0, 0, 0, deterministic)
+
+    def size(n):
+        b = ctypes.c_size_t()
+        assert lib.dtc_spmm_balanced_workspace_size_ex(blocks, n, ctypes.byref(o), ctypes.byref(b)) == 0
+        return b.value
+
+    widths = [1, 8, 64, 65, 128, 129, 192, 256, 300, 512, 1024, 4096]
+    sizes = [size(n) for n in widths]
+    assert sizes == sorted(sizes)
+    chunk = 32
+    while chunk < 512 and chunk * 2 * 8192 <= blocks:
+        chunk *= 2
+    if not deterministic:
+        dummy = ctypes.c_void_p(4096)
+        small = 256 + 8 * -(-blocks // chunk) - 1
+        assert lib.dtc_spmm_balanced(dummy, dummy, dummy, dummy, None, blocks, 8 * blocks, 16, dummy, 16, 8, dummy,
+                                     ctypes.byref(o), dummy, ctypes.c_size_t(small), None) == 3
+
+
 def test_gcn_gradient_shapes(lib):
     """K * F of 2^31 and more exceeds the gradients' 32-bit row offsets: refused
     before any launch, and left to the plain products by the layer."""

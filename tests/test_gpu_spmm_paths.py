@@ -151,6 +151,38 @@ def test_default_chunks(n, blocks):
     check(*random_csr(rng, rows, 400, lengths), 400, n, "balanced")
 
 
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_balanced_workspace_by_block_count(deterministic):
+    """A workspace sized by the chunk of the block count alone, or for a wider N:
+    accepted for a narrow N, whose default chunks are shorter."""
+    from dtc.capi import Library
+    from dtc.matrix import DTCMatrix
+    lib = Library()
+    rng = np.random.default_rng(9)
+    rows, n = 16 * 3000, 64
+    lengths = np.zeros(rows, np.int64)
+    lengths[::16] = 32
+    rowptr, col, values = random_csr(rng, rows, 400, lengths)
+    A = DTCMatrix(rowptr, col, values, num_rows=rows, num_cols=400)
+    B = rng.standard_normal((400, n)).astype(np.float32)
+    Bd = torch.from_numpy(B).cuda()
+    exact, mag = oracle.spmm_csr_f64(rowptr, col, values, B, rows, with_abs=True)
+    opt = lib.options(deterministic=deterministic)
+    chunks = -(-A.block_count // 32)
+    formula = 256 + 8 * chunks
+    if deterministic:
+        formula = -(-formula // 256) * 256 + 2 * chunks * 16 * 128 * 4
+    for bytes_ in (formula, lib.spmm_balanced_workspace_size(A.block_count, 4096, opt)):
+        C = torch.full((rows, n), float("nan"), device="cuda")
+        ws = torch.empty(bytes_, dtype=torch.uint8, device="cuda")
+        say("balanced workspace", bytes_)
+        lib.spmm_balanced(A.tcblock_rowid.data_ptr(), A.tcblocktile_id.data_ptr(), A.tcblock_offset.data_ptr(),
+                          A.sparse_atox.data_ptr(), A.values_tc.data_ptr(), A.block_count, A.nnz, rows, Bd.data_ptr(),
+                          400, n, C.data_ptr(), ws.data_ptr(), bytes_, options=opt,
+                          stream=torch.cuda.current_stream().cuda_stream)
+        assert np.all(np.abs(C.cpu().numpy() - exact) <= 36 * 2.0 ** -24 * mag)
+
+
 def test_noalloc_default_chunk():
     """The allocation-free entry point with the default chunk: the ordered merge
     of 12,000 blocks at N = 128 exceeds its scratch in chunks of 8 and fits it in
