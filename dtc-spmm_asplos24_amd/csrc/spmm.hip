@@ -20,15 +20,14 @@
 //     built by scattering the stored values at their tile ids;
 //   * C: lane l holds rows 4*(l/16) + i, i < 4, of its MFMA column, i.e. the
 //     output columns tile + q*VEC + v for the v-th MFMA.
-// What bounds it: the row gathers (a kernel of the same loads and nothing
-// else takes 2.6 ms of the 3.1 on the 2^20-node R-MAT at N = 256, 0.21 of
-// 0.36 on the 2^18-node one at N = 128), then the float32 MFMAs, which do
-// 16-row work on columns of one or two entries (0.07 ms of those 0.36, 0.28
-// of 4.3 on the 232,965-row block model at N = 128).  So the loop is built to
-// leave one exposed latency per group, the gathers' own, few vector
-// instructions around them, and five waves per SIMD to overlap one wave's
-// MFMAs with the others' gathers (a second group in flight per wave at three
-// to four waves per SIMD measured 10-35% slower).
+// What bounds it: the row gathers (the gather-only kernel of probe_gather.hip
+// takes 3.24 of 3.73 ms on the 2^20-node R-MAT at N = 256, chunk 256 and 32-column
+// tiles, 3.53 of 4.41 on the 232,965-row block model at N = 128, chunk 256 and
+// 64-column tiles), then the float32 MFMAs, which do 16-row work on columns of
+// one or two entries.  So the loop is built to leave one exposed latency per
+// group, the gathers' own, few vector instructions around them, and five waves
+// per SIMD to overlap one wave's MFMAs with the others' gathers (a second group
+// in flight per wave at three to four waves per SIMD measured 10-35% slower).
 // For FP32 the same group is fed as 8 steps of v_mfma_f32_16x16x4_f32 where
 // step j pairs A_g[:, j] with B row j of block g.  The k order inside a
 // group is a permutation shared by A and B, so every mapping sums the same

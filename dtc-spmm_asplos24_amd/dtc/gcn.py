@@ -11,7 +11,8 @@ accumulation.  A plain bf16 x bf16 product, other shapes and float32 W use a
 torch GEMM.  The backward pass:
     dXW     = A^T dH            (ME-TCF of A^T; dH gathered in bf16 for a bf16 layer)
     dX      = (dXW W^T) * [X > 0 if input_relu],  dW = act(X)^T dXW
-                                (dense GEMMs; dW split over K)
+                                (two MFMA kernels of csrc/gcn.hip; other shapes
+                                dense GEMMs, dW split over K)
     dvalues = SDDMM(dH, XW)     on A's pattern, XW rows gathered as bf16.
 The reference's GCN entry (`DTCSpMM_gcn`, DTCSpMM_kernel.cu:1033-1116) is a
 forward only and its "backward" names return A * dY (DTCSpMM.cpp:384-399).
@@ -103,10 +104,11 @@ class _GCNFunction(torch.autograd.Function):
             # A^T dH feeds GEMMs in W's precision: gather dH in it (bf16 B
             # kernel, float32 accumulation), then round the result once
             dHx = dH.to(W.dtype) if W.dtype == torch.bfloat16 else dH
-            # The chunk fixes where windows are cut, i.e. the last bit of dXW,
-            # which its rounding to bf16 in the GEMMs below turns into whole
-            # bf16 steps of dX: it is named here, not left to a default that
-            # may be tuned.
+            # The chunk fixes where windows are cut, i.e. how dXW's sums are
+            # split, and its rounding to bf16 in the GEMMs below turns a last bit
+            # into a whole bf16 step of dX: it is named here, not left to a default
+            # that may be tuned.  (Windows cut into three pieces and more still
+            # differ from run to run, by the order of the atomic adds.)
             dXW = At.spmm(dHx, schedule=ctx.schedule, values_tc=vals_t_tc,
                           chunk_blocks=default_chunk_blocks(At.block_count))
             X = X.contiguous()
