@@ -1601,15 +1601,25 @@ int long_chunk_blocks(int32_t num_blocks) {
 // Block model of 99,700 blocks of 12.5, N = 64, (32) 46 (16) 50; band of 55 a
 // block, 53,000 blocks, N = 64 (32) 37 (16) 44, 106,000, N = 256 (32) 164 (64)
 // 187, 8,750, N = 128 (8) 19.6 (16) 21.3.
-// nnz 0: not known, the shortest chunk it could be.
+// Where columns are hardly shared, windows are of one length, and a shorter chunk
+// cuts and merges every one of them: up to the average window's length the chunk
+// doubles while it leaves 27 * chunk units.  us, chunk by the rule above and this:
+// uniform 20,000 rows of 16, N = 128 (16) 34 (32) 23, bf16 B 31 and 18 (28 and 21
+// with the chunk by block count); 30,000 of 30, N = 64 (16) 57 (64) 42; 65,536 of
+// 32, N = 128 (32) 150 (64) 108; 16,384 of 60, N = 64 (16) 54 (64) 37 (128) 62;
+// 4,096 of 16, N = 64 (8) 14.4 (16) 15.1, N = 128 (8) 19.6 (16) 15.8.
+// nnz 0, windows 0: not known, the shortest chunk it could be.
 constexpr int64_t kChunkUnits = 550;
-int resolve_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n) {
+int resolve_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, int64_t windows) {
   if (opt && opt->chunk_blocks > 0) return opt->chunk_blocks;
   if (opt && opt->cut_span_blocks != 0) return long_chunk_blocks(num_blocks);
   const bool dense = nnz > 24 * (int64_t)num_blocks;
   const int64_t k = !dense && nnz > 11 * (int64_t)num_blocks ? kChunkUnits / 2 : kChunkUnits;
   int c = dense && num_blocks >= 1 << 15 ? 32 : 8;
-  while (c < 256 && (int64_t)num_blocks * ceil_div(std::max(n, 1), 64) > k * c * c) c *= 2;
+  const int64_t work = (int64_t)num_blocks * ceil_div(std::max(n, 1), 64);
+  if (windows > 0 && nnz > 0 && unshared_columns(nnz, num_blocks))
+    while (c < 256 && c * windows < num_blocks && work > 4 * 27 * c * c) c *= 2;
+  while (c < 256 && work > k * c * c) c *= 2;
   return c;
 }
 
@@ -1648,14 +1658,20 @@ size_t balanced_workspace_bytes_for(int32_t num_blocks, int32_t n, int32_t chunk
 }
 
 // The chunk for a workspace of this size: resolve_chunk's, or with the default
-// the one by the block count alone where only that one fits.
-int fit_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, size_t workspace_bytes) {
-  const int chunk = resolve_chunk(opt, num_blocks, nnz, n);
+// the one by the block count alone where only that one fits.  `need`: the least
+// workspace, which does not depend on how the windows are filled.
+int fit_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, int32_t num_nodes,
+              size_t workspace_bytes, size_t *need) {
   const bool det = opt && opt->deterministic;
-  if ((opt && (opt->chunk_blocks > 0 || opt->cut_span_blocks != 0)) ||
-      balanced_workspace_bytes_for(num_blocks, n, chunk, det) <= workspace_bytes)
+  auto bytes = [&](int chunk) { return balanced_workspace_bytes_for(num_blocks, n, chunk, det); };
+  const int chunk = resolve_chunk(opt, num_blocks, nnz, n, ceil_div(num_nodes, kBlkH));
+  const int by_count = long_chunk_blocks(num_blocks);
+  if (opt && (opt->chunk_blocks > 0 || opt->cut_span_blocks != 0)) {
+    *need = bytes(chunk);
     return chunk;
-  return std::max(chunk, long_chunk_blocks(num_blocks));
+  }
+  *need = bytes(std::max(resolve_chunk(opt, num_blocks, nnz, n, 0), by_count));
+  return bytes(chunk) <= workspace_bytes ? chunk : std::max(chunk, by_count);
 }
 
 __global__ __launch_bounds__(256) void k_zero(float *c, int64_t count) {
@@ -1915,7 +1931,7 @@ dtc_status_t dtc_spmm_balanced_workspace_size_ex(int32_t num_blocks, int32_t n,
   // For every N up to this one: a narrower N can have shorter, i.e. more chunks.
   *bytes = 0;
   for (int64_t m = n;;) {
-    const int64_t chunk = resolve_chunk(options, num_blocks, 0, (int32_t)m);
+    const int64_t chunk = resolve_chunk(options, num_blocks, 0, (int32_t)m, 0);
     *bytes = std::max(*bytes, balanced_workspace_bytes_for(num_blocks, (int32_t)m, (int32_t)chunk, det));
     if ((options && (options->chunk_blocks > 0 || options->cut_span_blocks != 0)) || chunk <= 8) break;
     m = kChunkUnits * (chunk / 2) * (chunk / 2) / num_blocks * 64;  // the widest with half the chunk
@@ -1944,7 +1960,8 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
                      mode, &var);
   if (st != DTC_SUCCESS) return st;
   const bool det = options && options->deterministic;
-  const int chunk = fit_chunk(options, num_blocks, nnz, n, workspace_bytes);
+  size_t need = 0;
+  const int chunk = fit_chunk(options, num_blocks, nnz, n, num_nodes, workspace_bytes, &need);
   int span = chunk;
   st = resolve_cut_span(options, chunk, &span);
   if (st != DTC_SUCCESS) return st;
@@ -1953,7 +1970,6 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
     return fail(DTC_ERROR_INVALID_VALUE, "deterministic must be 0 or 1");
   const int32_t W = (int32_t)ceil_div(num_nodes, kBlkH);
   if (W == 0) return DTC_SUCCESS;
-  const size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
   if (num_blocks > 0 && (!workspace || workspace_bytes < need))
     return fail(DTC_ERROR_WORKSPACE,
                 "balanced SpMM needs the workspace that dtc_spmm_balanced_workspace_size_ex reports (" +
@@ -2032,11 +2048,10 @@ dtc_status_t dtc_spmm_balanced_noalloc(const int32_t *tcblock_rowid, const uint8
   if (num_blocks < 0 || n < 0) return fail(DTC_ERROR_INVALID_VALUE, "num_blocks and N must be >= 0");
   if (options && options->chunk_blocks < 0)
     return fail(DTC_ERROR_INVALID_VALUE, "chunk_blocks must be >= 0");
-  const bool det = options && options->deterministic;
   dtc_spmm_options_t o{};
   if (options) o = *options;
-  const int chunk = fit_chunk(options, num_blocks, nnz, n, kNoAllocScratchBytes);
-  const size_t need = balanced_workspace_bytes_for(num_blocks, n, chunk, det);
+  size_t need = 0;
+  const int chunk = fit_chunk(options, num_blocks, nnz, n, num_nodes, kNoAllocScratchBytes, &need);
   o.chunk_blocks = chunk;
   if (need > kNoAllocScratchBytes)
     return fail(DTC_ERROR_UNSUPPORTED,

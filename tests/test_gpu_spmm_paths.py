@@ -151,6 +151,18 @@ def test_default_chunks(n, blocks):
     check(*random_csr(rng, rows, 400, lengths), 400, n, "balanced")
 
 
+@pytest.mark.parametrize("n", [64, 65, 192, 193])
+@pytest.mark.parametrize("blocks", [31, 32, 33])
+def test_even_windows(n, blocks):
+    """Balanced runs with the default chunk over windows of one length, a little
+    below, at and above a power of two, where the chunk keeps windows whole."""
+    rng = np.random.default_rng(blocks + n)
+    rows = 16 * 301 - 3
+    lengths = np.zeros(rows, np.int64)
+    lengths[::16] = 8 * blocks - 2
+    check(*random_csr(rng, rows, 700, lengths), 700, n, "balanced")
+
+
 @pytest.mark.parametrize("deterministic", [False, True])
 def test_balanced_workspace_by_block_count(deterministic):
     """A workspace sized by the chunk of the block count alone, or for a wider N:
