@@ -1427,8 +1427,8 @@ int operand_mode(int64_t b_rows, int64_t n, int64_t esz, int64_t nnz, int64_t nu
 // vec 0 for float32 B: 4 floats per lane (64-column tiles), less where N is
 // narrower.
 dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void *b, const float *c,
-                           bool balanced, bool dense, bool unshared, bool short_windows, int mode,
-                           Variant *out) {
+                           bool balanced, bool dense, int64_t windows, bool unshared, bool short_windows,
+                           bool few_entries, int mode, Variant *out) {
   const bool wide = mode == kPtr;
   const int prec = opt ? opt->precision : DTC_PRECISION_FP32;
   const int bdt = opt ? opt->b_dtype : DTC_B_FLOAT32;
@@ -1442,12 +1442,16 @@ dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void 
     auto fits = [&](int v) {
       return n % v == 0 && ((uintptr_t)b % (2 * v)) == 0 && ((uintptr_t)c % (4 * v)) == 0;
     };
-    // 128-column tiles where N fills more than half of one
+    // 128-column tiles where N fills more than half of one, in the unbalanced
+    // schedule not for rows of few entries, whose windows leave a wave little to
+    // overlap (us, 64 and 128 columns: band of 8 to a row, 200,000 rows, N = 256 55
+    // and 84, uniform 200,000 of 8 142 and 164; band of 12, 10^6 rows, N = 128 208 and
+    // 190, uniform 65,536 of 32 53 and 42).
     if (vec == 0) {
       if (!fits(4))
         return fail(DTC_ERROR_INVALID_VALUE,
                     "bfloat16 B needs N to be a multiple of 4 and 8-byte aligned B/C rows");
-      vec = n > 64 ? 8 : 4;
+      vec = n > 64 && !few_entries ? 8 : 4;
     } else
     if (!fits(vec))
       return fail(DTC_ERROR_INVALID_VALUE,
@@ -1482,14 +1486,20 @@ dtc_status_t resolve_shape(const dtc_spmm_options_t *opt, int32_t n, const void 
     // 627), and for dense blocks not with the limb splits, whose registers cost waves
     // in windows of a group or two (band of 5 blocks a window, N = 224, bf16x3 37 and
     // 40, bf16x6 43 and 47; of 10, N = 512 72 and 63, 77 and 75), nor where wide B
-    // leaves half of the last tile empty (N = 320 51 and 55, 384 62 and 58).
+    // leaves half of the last tile empty (N = 320 51 and 55, 384 62 and 58; the other
+    // way round where columns are unshared: 30,000 rows of 16, N = 320 85 and 77,
+    // of 8, N = 384 53 and 56).  Not where the wider tiles leave the chip short of
+    // units either (uniform 20,000 of 30, N = 96 33 and 41, band of 5,000, N = 384 11.5
+    // and 16.1).
     const bool half = n % 128 > 64 && n % 128 <= 96;
     if (nsub == 0 && balanced && half && n < 128 && !dense) vec = 2;
     if (nsub == 0 && balanced) nsub = half && dense ? 2 : 1;
     if (nsub == 0) {
       const bool limbs = prec == DTC_PRECISION_BF16X3 || prec == DTC_PRECISION_BF16X6;
-      const bool two = mode == kDense ? !(limbs && short_windows) && (half || (n > 256 && (n - 1) % 128 >= 64)) : half || n > 256;
-      nsub = two && (mode == kDense || unshared) ? 2 : 1;
+      const bool two = mode == kDense ? !(limbs && short_windows) && (half || (n > 256 && (n - 1) % 128 >= 64))
+                                      : half || (n > 256 && (n - 1) % 128 < 64);
+      const bool fills = windows * ceil_div(n, 128) >= (mode == kDense ? 1024 : 4096);
+      nsub = two && fills && (mode == kDense || unshared) ? 2 : 1;
     }
   }
   if (wide) vec = n >= 4 ? 4 : 1;
@@ -1817,7 +1827,7 @@ dtc_status_t dtc_spmm_tcgnn(const int32_t *node_pointer, const int32_t *edge_lis
   o.vec = options ? options->vec : 0;
   o.subtiles = 1;
   Variant var;
-  dtc_status_t st = resolve_shape(&o, n, b, c, false, false, false, false, kBuf, &var);
+  dtc_status_t st = resolve_shape(&o, n, b, c, false, false, 0, false, false, false, kBuf, &var);
   if (st != DTC_SUCCESS) return st;
   const int32_t W = (int32_t)ceil_div(num_nodes, kBlkH);
   if (b_rows == 0) return zero_output(c, num_nodes, n, stream);
@@ -1871,7 +1881,8 @@ dtc_status_t dtc_spmm_windows(const int32_t *row_window_offset, const uint8_t *t
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
   const bool unshared = unshared_columns(nnz, num_blocks);
-  st = resolve_shape(options, n, b, c, false, false, unshared, num_blocks <= 6 * (int64_t)num_windows, mode, &var);
+  st = resolve_shape(options, n, b, c, false, false, num_windows, unshared, num_blocks <= 6 * (int64_t)num_windows,
+                     nnz <= 160 * (int64_t)num_windows, mode, &var);
   if (st != DTC_SUCCESS) return st;
   // Only windows that hold output rows are processed.
   const int32_t W = (int32_t)std::min<int64_t>(num_windows, ceil_div(num_nodes, kBlkH));
@@ -1956,8 +1967,8 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   Variant var;
   const int esz = options && options->b_dtype == DTC_B_BFLOAT16 ? 2 : 4;
   const int mode = operand_mode(b_rows, n, esz, nnz, num_blocks, tcblocktile_id, tcblock_values);
-  st = resolve_shape(options, n, b, c, true, nnz > (num_blocks >= (1 << 19) ? 11 : 24) * (int64_t)num_blocks, false, false,
-                     mode, &var);
+  st = resolve_shape(options, n, b, c, true, nnz > (num_blocks >= (1 << 19) ? 11 : 24) * (int64_t)num_blocks, 0, false,
+                     false, false, mode, &var);
   if (st != DTC_SUCCESS) return st;
   const bool det = options && options->deterministic;
   size_t need = 0;
