@@ -33,6 +33,7 @@
 // group is a permutation shared by A and B, so every mapping sums the same
 // products.
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -1553,6 +1554,14 @@ int32_t long_window(int64_t windows, int64_t num_blocks) {
 // hubs' columns (8.3 to 13 entries a block).
 bool unshared_columns(int64_t nnz, int64_t num_blocks) { return 4 * nnz <= 33 * num_blocks; }
 
+// Whether windows hold about as many columns as random entries over all of B's
+// rows would: x entries a row of B and window fall on (1 - e^-x) / x as many columns.
+bool even_windows(int64_t nnz, int64_t num_blocks, int64_t windows, int64_t b_rows) {
+  if (nnz <= 0 || windows <= 0 || b_rows <= 0) return false;
+  const double x = (double)nnz / ((double)windows * (double)b_rows);
+  return 4.0 * (double)nnz * (-std::expm1(-x) / x) <= 33.0 * (double)num_blocks;
+}
+
 // Whether the column tiles go one after another instead of side by side.  B
 // beyond the 256 MB memory-side cache: one slice (or two) at a time, so that most
 // of its gathers hit there.  (Two tiles of 256 MB each are no faster in turn,
@@ -1611,24 +1620,26 @@ int long_chunk_blocks(int32_t num_blocks) {
 // Block model of 99,700 blocks of 12.5, N = 64, (32) 46 (16) 50; band of 55 a
 // block, 53,000 blocks, N = 64 (32) 37 (16) 44, 106,000, N = 256 (32) 164 (64)
 // 187, 8,750, N = 128 (8) 19.6 (16) 21.3.
-// Where columns are hardly shared, windows are of one length, and a shorter chunk
-// cuts and merges every one of them: up to the average window's length the chunk
-// doubles while it leaves 27 * chunk units.  us, chunk by the rule above and this:
+// Where entries are spread like random ones, windows are of one length, and a
+// shorter chunk cuts and merges every one of them: up to the average window's
+// length the chunk doubles while it leaves 27 * chunk units of 64 columns.  us, chunk by the rule above and this:
 // uniform 20,000 rows of 16, N = 128 (16) 34 (32) 23, bf16 B 31 and 18 (28 and 21
 // with the chunk by block count); 30,000 of 30, N = 64 (16) 57 (64) 42; 65,536 of
 // 32, N = 128 (32) 150 (64) 108; 16,384 of 60, N = 64 (16) 54 (64) 37 (128) 62;
 // 4,096 of 16, N = 64 (8) 14.4 (16) 15.1, N = 128 (8) 19.6 (16) 15.8.
 // nnz 0, windows 0: not known, the shortest chunk it could be.
 constexpr int64_t kChunkUnits = 550;
-int resolve_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, int64_t windows) {
+int resolve_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, int64_t windows,
+                  int64_t b_rows) {
   if (opt && opt->chunk_blocks > 0) return opt->chunk_blocks;
   if (opt && opt->cut_span_blocks != 0) return long_chunk_blocks(num_blocks);
   const bool dense = nnz > 24 * (int64_t)num_blocks;
   const int64_t k = !dense && nnz > 11 * (int64_t)num_blocks ? kChunkUnits / 2 : kChunkUnits;
   int c = dense && num_blocks >= 1 << 15 ? 32 : 8;
   const int64_t work = (int64_t)num_blocks * ceil_div(std::max(n, 1), 64);
-  if (windows > 0 && nnz > 0 && unshared_columns(nnz, num_blocks))
-    while (c < 256 && c * windows < num_blocks && work > 4 * 27 * c * c) c *= 2;
+  if (even_windows(nnz, num_blocks, windows, b_rows))
+    while (c < 256 && c * windows < num_blocks && std::min<int64_t>(work * 64, (int64_t)num_blocks * n) > 64 * 108 * c * c)
+      c *= 2;
   while (c < 256 && work > k * c * c) c *= 2;
   return c;
 }
@@ -1671,16 +1682,16 @@ size_t balanced_workspace_bytes_for(int32_t num_blocks, int32_t n, int32_t chunk
 // the one by the block count alone where only that one fits.  `need`: the least
 // workspace, which does not depend on how the windows are filled.
 int fit_chunk(const dtc_spmm_options_t *opt, int32_t num_blocks, int32_t nnz, int32_t n, int32_t num_nodes,
-              size_t workspace_bytes, size_t *need) {
+              int32_t b_rows, size_t workspace_bytes, size_t *need) {
   const bool det = opt && opt->deterministic;
   auto bytes = [&](int chunk) { return balanced_workspace_bytes_for(num_blocks, n, chunk, det); };
-  const int chunk = resolve_chunk(opt, num_blocks, nnz, n, ceil_div(num_nodes, kBlkH));
+  const int chunk = resolve_chunk(opt, num_blocks, nnz, n, ceil_div(num_nodes, kBlkH), b_rows);
   const int by_count = long_chunk_blocks(num_blocks);
   if (opt && (opt->chunk_blocks > 0 || opt->cut_span_blocks != 0)) {
     *need = bytes(chunk);
     return chunk;
   }
-  *need = bytes(std::max(resolve_chunk(opt, num_blocks, nnz, n, 0), by_count));
+  *need = bytes(std::max(resolve_chunk(opt, num_blocks, nnz, n, 0, 0), by_count));
   return bytes(chunk) <= workspace_bytes ? chunk : std::max(chunk, by_count);
 }
 
@@ -1942,7 +1953,7 @@ dtc_status_t dtc_spmm_balanced_workspace_size_ex(int32_t num_blocks, int32_t n,
   // For every N up to this one: a narrower N can have shorter, i.e. more chunks.
   *bytes = 0;
   for (int64_t m = n;;) {
-    const int64_t chunk = resolve_chunk(options, num_blocks, 0, (int32_t)m, 0);
+    const int64_t chunk = resolve_chunk(options, num_blocks, 0, (int32_t)m, 0, 0);
     *bytes = std::max(*bytes, balanced_workspace_bytes_for(num_blocks, (int32_t)m, (int32_t)chunk, det));
     if ((options && (options->chunk_blocks > 0 || options->cut_span_blocks != 0)) || chunk <= 8) break;
     m = kChunkUnits * (chunk / 2) * (chunk / 2) / num_blocks * 64;  // the widest with half the chunk
@@ -1972,7 +1983,7 @@ dtc_status_t dtc_spmm_balanced(const int32_t *tcblock_rowid, const uint8_t *tcbl
   if (st != DTC_SUCCESS) return st;
   const bool det = options && options->deterministic;
   size_t need = 0;
-  const int chunk = fit_chunk(options, num_blocks, nnz, n, num_nodes, workspace_bytes, &need);
+  const int chunk = fit_chunk(options, num_blocks, nnz, n, num_nodes, b_rows, workspace_bytes, &need);
   int span = chunk;
   st = resolve_cut_span(options, chunk, &span);
   if (st != DTC_SUCCESS) return st;
@@ -2062,7 +2073,7 @@ dtc_status_t dtc_spmm_balanced_noalloc(const int32_t *tcblock_rowid, const uint8
   dtc_spmm_options_t o{};
   if (options) o = *options;
   size_t need = 0;
-  const int chunk = fit_chunk(options, num_blocks, nnz, n, num_nodes, kNoAllocScratchBytes, &need);
+  const int chunk = fit_chunk(options, num_blocks, nnz, n, num_nodes, b_rows, kNoAllocScratchBytes, &need);
   o.chunk_blocks = chunk;
   if (need > kNoAllocScratchBytes)
     return fail(DTC_ERROR_UNSUPPORTED,
