@@ -56,11 +56,13 @@ typedef struct dtc_spmm_options {
   int32_t vec;          /* B elements per lane per gathered row: 1, 2, 4 (float32 B);
                            4, 8 (bfloat16 B); 0 = float32 B: 4, less for N <= 32 and
                            for some N <= 96 of the balanced schedule, any N and
-                           alignment; bfloat16 B: 8 for N > 64, else 4 */
-  int32_t subtiles;     /* 1 or 2 column tiles of 16*vec per wave (0 = chosen from N;
-                           float32 B) */
+                           alignment; bfloat16 B: 8 for N > 64 (unbalanced: and more than
+                           160 entries a window), else 4 */
+  int32_t subtiles;     /* 1 or 2 column tiles of 16*vec per wave (0 = chosen from N and
+                           the matrix; float32 B) */
   int32_t chunk_blocks; /* balanced schedule: TC blocks per work chunk (0 = a power of two
-                           in [8, 256] that grows with num_blocks and N; with
+                           in [8, 256] that grows with num_blocks and N, and to the
+                           average window's length where windows are even; with
                            cut_span_blocks the largest power of two in [32, 512] at most
                            num_blocks / 8192) */
   int32_t persistent;   /* balanced schedule: 1 = persistent waves pulling chunks from a queue */
